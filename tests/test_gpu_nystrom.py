@@ -143,3 +143,26 @@ def test_nystrom_argument_errors(dev):
     Z = torch.zeros((11, 100), dtype=torch.float64, device="cuda")
     with pytest.raises(dh.DHError):
         dev.nystrom(Q, Q, 11, Z)  # k > l
+
+
+# One workgroup for all pairs (n <= 64), several with 8 or 4 rounds per launch
+# (row counts at the LDS capacities of 32 pairs and at 512), odd n (a padding
+# player), and columns too long for LDS (a launch per round).
+@pytest.mark.parametrize("m,n", [(2, 2), (5, 3), (64, 64), (65, 65), (128, 66), (139, 137),
+                                 (312, 120), (313, 121), (512, 201), (513, 40)])
+def test_gesvj_round_grouping(dev, m, n):
+    import torch
+    rng = np.random.default_rng(1000 * m + n)
+    A = rng.standard_normal((m, n)) * np.logspace(0, -6, n)
+    Ad = dh.to_dev(A)
+    s = torch.zeros(n, dtype=torch.float64, device="cuda")
+    V = torch.zeros((n, n), dtype=torch.float64, device="cuda")
+    st, sweeps = dev.gesvj(Ad, s, V)
+    sg, Vg, AVg = s.cpu().numpy(), dh.from_dev(V), dh.from_dev(Ad)
+    _, so, Vo, swo = orc.gesvj(A)
+    assert st == 0 and sweeps == swo
+    assert np.abs(sg - so).max() <= 1e-12 * so[0]
+    assert np.linalg.norm(Vg.T @ Vg - np.eye(n)) < 1e-11
+    assert rel(AVg, A @ Vg) < 1e-12
+    # Same rotations in the same order: the same signs as well.
+    assert rel(Vg, Vo) < 1e-6
