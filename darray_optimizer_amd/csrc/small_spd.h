@@ -528,50 +528,76 @@ __global__ __launch_bounds__(WAVES * 64) void trsm_rows_batched_kernel(
                           16 * ((j.n + 15) / 16) + 1);
 }
 
-// Lane I of each 16-lane row, broadcast to the row (DPP row_newbcast): no
-// LDS round trip and no scalar registers.  Every lane is written (full row and
-// bank masks), so the move takes no old value: with update_dpp(0, ...) the
-// compiler zeroed the destination before each of the 240 moves per 16 x 16
-// factorisation (register Cholesky at order 272: 151 -> 144 us).
-template <int I>
-__device__ __forceinline__ double bcast16(double v) {
-    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0x150 + I, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0x150 + I, 0xF, 0xF, false);
-    return __hiloint2double(hi, lo);
+// The values of the four 16-lane rows at the lane's column: out[g] = v of lane
+// 16 g + (lane & 15).
+__device__ __forceinline__ void gather_rows(double v, double (&out)[4]) {
+    const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
+    const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);  // rows 0022, 1133
+    const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    const auto l02 = __builtin_amdgcn_permlane32_swap(l[0], l[0], false, false);
+    const auto h02 = __builtin_amdgcn_permlane32_swap(h[0], h[0], false, false);
+    const auto l13 = __builtin_amdgcn_permlane32_swap(l[1], l[1], false, false);
+    const auto h13 = __builtin_amdgcn_permlane32_swap(h[1], h[1], false, false);
+    out[0] = __hiloint2double((int)h02[0], (int)l02[0]);
+    out[1] = __hiloint2double((int)h13[0], (int)l13[0]);
+    out[2] = __hiloint2double((int)h02[1], (int)l02[1]);
+    out[3] = __hiloint2double((int)h13[1], (int)l13[1]);
 }
 
-// u[I..15] -= U(KK, I) * ukj, U(KK, I) being ukj of lane I.
-template <int I>
-__device__ __forceinline__ void chol16_update(double (&u)[NB], double ukj) {
-    if constexpr (I < NB) {
-        u[I] -= bcast16<I>(ukj) * ukj;
-        chol16_update<I + 1>(u, ukj);
-    }
+// 1/sqrt(piv): hardware estimate and two Newton steps.
+__device__ __forceinline__ double rsqrt_newton(double piv) {
+    const double hp = 0.5 * piv;
+    double y = __builtin_amdgcn_rsq(piv);
+    y = fma(y, fma(-hp * y, y, 0.5), y);
+    return fma(y, fma(-hp * y, y, 0.5), y);
 }
 
-// Column steps KK..15 of the 16 x 16 Cholesky, lane j (mod 16) holding
-// column j; bad receives the 1-based failing step.
-template <int KK>
-__device__ __forceinline__ void chol16_steps(double (&u)[NB], int li, int nreal, double tol,
-                                             int& bad) {
-    if constexpr (KK < NB) {
-        if (!bad) {
-            const double piv = readlane_d(u[KK], KK);
-            if (KK < nreal && !(piv > tol)) {
-                bad = KK + 1;
-            } else {
-                // 1/sqrt(piv): hardware estimate and two Newton steps.
-                const double hp = 0.5 * piv;
-                double y = __builtin_amdgcn_rsq(piv);
-                y = fma(y, fma(-hp * y, y, 0.5), y);
-                y = fma(y, fma(-hp * y, y, 0.5), y);
-                const double ukj = (li == KK) ? piv * y : u[KK] * y;
-                u[KK] = ukj;
-                chol16_update<KK + 1>(u, ukj);
+// Cholesky of a 16 x 16 block in MFMA accumulator layout (d[r] of lane (g, li):
+// row g + 4r, column li) by one wave, in four steps of four rows; on return d
+// holds U (entries below the diagonal are whatever the updates leave there).
+// Rows 4b .. 4b+3 are d[b] of the four lane groups.  Every lane factors the
+// 4 x 4 diagonal block for itself (uniform values) and solves the four rows at
+// its own column, so the chain of square roots crosses no lanes; then d[b] =
+// the lane's row is the operand of one MFMA that updates all later rows (rows
+// up to 4b+3 masked).  An FP64 MFMA is a chain of FMAs in ascending k, so each
+// element gets fma(-u_k, u_k', a) once per step k, as column by column.
+// Returns 0, or the 1-based step of the first pivot p with !(p > tol) among
+// the first nreal.  About 450 cycles per four rows; a step per row with
+// broadcasts of the row took 300 per row.
+__device__ __forceinline__ int chol16(dh_d4& d, int g, int li, int nreal, double tol) {
+    int bad = 0;  // no early exit: what follows a failed pivot is not used
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        double a[4];
+        gather_rows(d[b], a);
+        double m[4][4];  // the diagonal block, upper part, uniform
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int c = r; c < 4; ++c) m[r][c] = readlane_d(d[b], 16 * r + 4 * b + c);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int kk = 4 * b + r;
+            bad = bad == 0 && kk < nreal && !(m[r][r] > tol) ? kk + 1 : bad;
+            const double y = rsqrt_newton(m[r][r]);
+            a[r] *= y;
+#pragma unroll
+            for (int c = r + 1; c < 4; ++c) m[r][c] *= y;
+#pragma unroll
+            for (int i = r + 1; i < 4; ++i) {
+#pragma unroll
+                for (int c = i; c < 4; ++c) m[i][c] = fma(-m[r][i], m[r][c], m[i][c]);
+                a[i] = fma(-m[r][i], a[r], a[i]);
             }
         }
-        chol16_steps<KK + 1>(u, li, nreal, tol, bad);
+        double u = a[0];
+        u = g == 1 ? a[1] : u;
+        u = g == 2 ? a[2] : u;
+        u = g == 3 ? a[3] : u;
+        d[b] = u;
+        if (b < 3) d = Mfma<double>::op(li > 4 * b + 3 ? -u : 0.0, u, d);
     }
+    return bad;
 }
 
 // Register-resident Cholesky for orders n <= 16 * kRegBlocks (= 272), same
@@ -579,33 +605,37 @@ __device__ __forceinline__ void chol16_steps(double (&u)[NB], int li, int nreal,
 // and columns past n hold the identity, so they factor to the identity and
 // skip the pivot test) is held as 16 x 16 blocks: the off-diagonal blocks
 // (bi, bj > bi) in registers, in FP64 MFMA accumulator layout (lane: rows
-// g + 4r, column li), numbered row by row and dealt to the 8 waves round
-// robin; the diagonal blocks in LDS (sG[i][col][row]), block i updated by
-// wave i % 8.  Per 16-column panel k:
-//   A  wave k % 8 factors block (k, k) (column per lane; rows of U broadcast
-//      by DPP within 16-lane rows), inverts the factor by back substitution
-//      (rows of U from LDS), and writes
-//      U_kk to G, its inverse to Dinv and to LDS;
+// g + 4r, column li), numbered row by row and dealt to waves 1..7; the
+// diagonal blocks in LDS (sG[i][col][row]), block i updated by wave 1 + i % 7.
+// Per 16-column panel k:
+//   A  wave 0 factors block (k, k) (chol16), inverts the factor by back
+//      substitution (rows of U from LDS), and leaves both in LDS;
 //   B  the owners of blocks (k, j > k) form U_kj = U_kk^{-T} A_kj (4 MFMAs,
-//      A_kj's accumulator rows are the B operand) into the LDS panel, which
-//      the workgroup then copies to G;
+//      A_kj's accumulator rows are the B operand) into the LDS panel;
 //   C  A_ij -= U_ki^T U_kj for k < i <= j (4 MFMAs per block from the LDS
-//      panel).  Wave (k+1) % 8 updates block (k+1, k+1) first and runs step
-//      A of panel k+1 before its other updates, so that factorisation
-//      overlaps the rest of the trailing update.
+//      panel) and panel k, U_kk and its inverse to global memory, while wave 0
+//      updates block (k+1, k+1) and runs step A of panel k+1.
 // Two workgroup barriers per panel and no global loads after the first.
+// Step A is the chain that bounds the kernel from the middle panels on, so
+// its wave holds no blocks (holding 17 as the others did, it spilled, and
+// each reload waited for the global stores before it), and wave 4, which
+// shares its SIMD, holds half as many as the others: an FP64 MFMA keeps the
+// SIMD's FP64 datapath for 64 cycles.
 constexpr int kCholWaves = NT / 64;
-constexpr int kCholSlots =
-    (kRegBlocks * (kRegBlocks - 1) / 2 + kCholWaves - 1) / kCholWaves;  // 17
+// Blocks are dealt in rounds of 13: one each to waves 1 2 3 5 6 7, one to wave
+// 4, one more each to the six.
+constexpr int kCholSlots = 21;  // 136 blocks: ten rounds of 13 and one of 6
+static_assert(kRegBlocks * (kRegBlocks - 1) / 2 <= 13 * 10 + 6, "slots cover the blocks");
 
 // LDS of chol_reg_body (kernels declare it __shared__ or carve it from an arena).
 struct CholRegLds {
     double sG[kRegBlocks][NB][NB + 1];  // diagonal blocks, sG[i][col][row]
-    double sI[NB][NB + 1];              // inverse factor of panel k, sI[j][i] = U_kk^{-1}(i, j)
+    double sI[2][NB][NB + 1];  // inverse factor of panel k in sI[k & 1], [j][i] = U_kk^{-1}(i, j)
     __align__(16) double sP[NB][16 * (kRegBlocks - 1) + 4];  // U_k,k+1..nb-1
-    __align__(16) double sU[NB][NB];                         // U_kk^T for the back substitution
+    __align__(16) double sU[2][NB][NB];                      // U_kk in sU[k & 1], [row][column]
     double sRd[NB];                                          // 1 / U_kk(i, i)
     double red[2][kCholWaves];                               // diagonal max and trace
+    double s_tol;
     int s_info;
 };
 
@@ -627,18 +657,23 @@ __device__ __forceinline__ void chol_reg_body(CholRegLds& L, int n, double* __re
     const int g = lane >> 4, li = lane & 15;
 
     static_assert(NT >= 16 * kRegBlocks, "one thread per diagonal element");
-    double tol = 0.0;  // breakdown tolerance, set once the diagonal is in LDS
     const int nbk = (n + 15) / 16;
-    int bI[kCholSlots], bJ[kCholSlots];  // block of each slot; bI == nbk: unused
+    int bI[kCholSlots], bJ[kCholSlots];  // block of each slot (rising); bI == nbk: unused
+    {
+        const int q = wave < 4 ? wave - 1 : wave - 2;  // waves 1 2 3 5 6 7 -> 0..5
+        int bi = 0, first = 0;                         // first: number of block (bi, bi + 1)
 #pragma unroll
-    for (int s = 0; s < kCholSlots; ++s) {
-        int rem = s * kCholWaves + wave, bi = 0;
-        while (bi < nbk && rem >= nbk - 1 - bi) {
-            rem -= nbk - 1 - bi;
-            ++bi;
+        for (int s = 0; s < kCholSlots; ++s) {
+            const int e = wave == 0   ? nbk * nbk
+                          : wave == 4 ? 13 * s + 6
+                                      : 13 * (s >> 1) + ((s & 1) ? 7 : 0) + q;
+            while (bi < nbk && e - first >= nbk - 1 - bi) {
+                first += nbk - 1 - bi;
+                ++bi;
+            }
+            bI[s] = bi;
+            bJ[s] = bi + 1 + e - first;
         }
-        bI[s] = bi;
-        bJ[s] = bi + 1 + rem;
     }
     // Diagonal blocks to LDS: upper triangle, zero below, identity padding
     // (all loads issued first, clamped addresses).
@@ -663,96 +698,77 @@ __device__ __forceinline__ void chol_reg_body(CholRegLds& L, int n, double* __re
             }
         }
     }
-    // Off-diagonal blocks to registers in groups of four slots: the group's
-    // 16 loads are issued together (clamped addresses), then padded.
+    // Off-diagonal blocks to registers: every load of the slots in use is
+    // issued (clamped addresses) before the first is padded.
     dh_d4 a[kCholSlots];
 #pragma unroll
-    for (int s0 = 0; s0 < kCholSlots; s0 += 4) {
-        double v[4][4];
+    for (int s = 0; s < kCholSlots; ++s)
+        if (bI[s] < nbk) {  // uniform
+            const double* col = G + (size_t)min(16 * bJ[s] + li, n - 1) * ldg;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int s = min(s0 + j, kCholSlots - 1);
-            const int cc = min(16 * bJ[s] + li, n - 1);
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                v[j][r] = G[min(16 * bI[s] + g + 4 * r, n - 1) + (size_t)cc * ldg];
+            for (int r = 0; r < 4; ++r) a[s][r] = col[16 * bI[s] + g + 4 * r];
         }
+    // Rows of an off-diagonal block are never past n (bI < bJ); columns can be.
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int s = s0 + j;
-            if (s < kCholSlots) {
-                const int c = 16 * bJ[s] + li;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int row = 16 * bI[s] + g + 4 * r;
-                    a[s][r] = (row < n && c < n) ? v[j][r] : 0.0;
-                }
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);  // keep the groups apart (register pressure)
-    }
+    for (int s = 0; s < kCholSlots; ++s)
+        if (bI[s] < nbk && 16 * bJ[s] + 16 > n && 16 * bJ[s] + li >= n) a[s] = dh_d4{0, 0, 0, 0};
 
-    // Step A for panel k (wave k % 8).
-    auto factor_diag = [&](int k) {
-        // Lane j holds column j & 15 of the block (every 16-lane row a full
-        // copy, so row broadcasts serve all lanes).  Entries below the
-        // diagonal are not needed and take whatever the unmasked updates
-        // leave there.
-        double u[NB];
+    // Step A for panel k, block (k, k) in accumulator layout (stores to LDS only).
+    auto factor_diag = [&](int k, dh_d4 d) {
+        const int bad = chol16(d, g, li, n - 16 * k, L.s_tol);
+        double(*U)[NB] = sU[k & 1];
 #pragma unroll
-        for (int i = 0; i < NB; ++i) u[i] = sG[k][li][i];
-        int bad = 0;
-        chol16_steps<0>(u, li, n - 16 * k, tol, bad);
-        const int c = 16 * k + lane;
-        if (lane < NB) {
+        for (int r = 0; r < 4; ++r) U[g + 4 * r][li] = d[r];
+        {
+            double dg = d[0];
 #pragma unroll
-            for (int i = 0; i < NB; ++i) sU[i][lane] = u[i];
-            double dg = 1.0;
-#pragma unroll
-            for (int i = 0; i < NB; ++i)
-                if (i == lane) dg = u[i];
-            sRd[lane] = 1.0 / dg;
-            if (c < n)
-#pragma unroll
-                for (int i = 0; i < NB; ++i)
-                    if (i <= lane) G[(16 * k + i) + (size_t)c * ldg] = u[i];
+            for (int r = 1; r < 4; ++r) dg = (li >> 2) == r ? d[r] : dg;
+            if (g == (li & 3)) sRd[li] = 1.0 / dg;
         }
         wave_lds_sync();
-        // Column j of U_kk^{-1} by back substitution, in place: x[i] =
-        // (e_j[i] - sum_{q>i} U(i, q) x[q]) / U(i, i), two partial sums.
+        // Column li of U_kk^{-1} by back substitution: x[i] = (e_j[i] -
+        // sum_{q>i} U(i, q) x[q]) / U(i, i), two partial sums.
+        double x[NB];
 #pragma unroll
         for (int i = NB - 1; i >= 0; --i) {
-            double t0 = (i == lane) ? 1.0 : 0.0, t1 = 0.0;
+            double t0 = (i == li) ? 1.0 : 0.0, t1 = 0.0;
 #pragma unroll
             for (int q = i + 1; q < NB; ++q) {
                 if ((q - i) & 1)
-                    t0 -= sU[i][q] * u[q];
+                    t0 -= U[i][q] * x[q];
                 else
-                    t1 -= sU[i][q] * u[q];
+                    t1 -= U[i][q] * x[q];
             }
-            u[i] = (t0 + t1) * sRd[i];
+            x[i] = (t0 + t1) * sRd[i];
         }
         if (lane < NB)
 #pragma unroll
-            for (int i = 0; i < NB; ++i) {
-                sI[lane][i] = u[i];
-                Dinv[256 * k + i + 16 * lane] = (i <= lane && c < n) ? u[i] : 0.0;
-            }
+            for (int i = 0; i < NB; ++i) sI[k & 1][lane][i] = x[i];
         if (lane == 0 && bad) s_info = 16 * k + bad;
     };
-    // Diagonal block i -= U_ki^T U_ki (panel k in sP), in LDS.
-    auto update_diag = [&](int i, int k) {
-        const int pi = 16 * (i - k - 1) + li;
+    // U_kk and its inverse from LDS to G and Dinv, by 256 threads (t < 256).
+    auto store_diag = [&](int k, int t) {
+        const int i = t & 15, j = t >> 4, c = 16 * k + j;
+        if (i <= j && c < n) G[(16 * k + i) + (size_t)c * ldg] = sU[k & 1][i][j];
+        Dinv[256 * k + t] = (i <= j && c < n) ? sI[k & 1][j][i] : 0.0;
+    };
+    // Diagonal block i in accumulator layout.
+    auto load_diag = [&](int i) {
         dh_d4 d;
 #pragma unroll
         for (int r = 0; r < 4; ++r) d[r] = sG[i][li][g + 4 * r];
+        return d;
+    };
+    // Diagonal block i - U_ki^T U_ki (panel k in sP).
+    auto updated_diag = [&](int i, int k) {
+        const int pi = 16 * (i - k - 1) + li;
+        dh_d4 d = load_diag(i);
 #pragma unroll
         for (int s4 = 0; s4 < 4; ++s4) {
             const double v = sP[4 * s4 + g][pi];
             d = Mfma<double>::op(-v, v, d);
         }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sG[i][li][g + 4 * r] = d[r];
+        return d;
     };
 
     __syncthreads();  // diagonal blocks in LDS
@@ -781,7 +797,7 @@ __device__ __forceinline__ void chol_reg_body(CholRegLds& L, int n, double* __re
             m2 = fmax(m2, red[0][w]);
             t2 += red[1][w];
         }
-        tol = rel_check ? (double)n * 2.220446049250313e-16 * m2 : 0.0;
+        double tol = rel_check ? (double)n * 2.220446049250313e-16 * m2 : 0.0;
         double sh = shift ? 11.0 * ((double)m_rows * n + (double)n * (n + 1)) *
                                 1.1102230246251565e-16 * t2
                           : 0.0;
@@ -790,54 +806,65 @@ __device__ __forceinline__ void chol_reg_body(CholRegLds& L, int n, double* __re
             sh = scales[1];
         }
         if (shift && tid < n) sG[tid >> 4][tid & 15][tid & 15] += sh;
-        if (tid == 0) s_info = 0;
-    }
-    __syncthreads();  // shifted diagonal blocks and s_info in LDS
-    if (wave == 0) factor_diag(0);
-    for (int k = 0;; ++k) {
-        __syncthreads();  // U_kk, its inverse and s_info ready
-        if (s_info || k + 1 == nbk) break;
-        // ---- B: row panel U_kj = U_kk^{-T} A_kj.
-#pragma unroll
-        for (int s = 0; s < kCholSlots; ++s) {
-            if (bI[s] == k) {
-                dh_d4 acc = {0, 0, 0, 0};
-#pragma unroll
-                for (int s4 = 0; s4 < 4; ++s4)
-                    acc = Mfma<double>::op(sI[li][4 * s4 + g], a[s][s4], acc);
-                const int pc = 16 * (bJ[s] - k - 1) + li;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) sP[g + 4 * r][pc] = acc[r];
-            }
+        if (tid == 0) {
+            s_info = 0;
+            L.s_tol = tol;
         }
-        __syncthreads();  // panel k in sP
-        {  // the panel to G, 16-row runs per column
+    }
+    __syncthreads();  // shifted diagonal blocks, s_tol and s_info in LDS
+    // Wave 0 has a loop of its own (the blocks' registers are not live in it);
+    // its barriers match those of the other waves.
+    if (wave == 0) {
+        factor_diag(0, load_diag(0));
+        for (int k = 0;; ++k) {
+            __syncthreads();  // U_kk, its inverse and s_info ready
+            if (s_info || k + 1 == nbk) break;
+            __syncthreads();  // panel k in sP
+            factor_diag(k + 1, updated_diag(k + 1, k));
+        }
+    } else {
+        for (int k = 0;; ++k) {
+            __syncthreads();
+            if (s_info || k + 1 == nbk) break;
+            // ---- B: row panel U_kj = U_kk^{-T} A_kj.
+#pragma unroll
+            for (int s = 0; s < kCholSlots; ++s) {
+                if (bI[s] == k) {
+                    dh_d4 acc = {0, 0, 0, 0};
+#pragma unroll
+                    for (int s4 = 0; s4 < 4; ++s4)
+                        acc = Mfma<double>::op(sI[k & 1][li][4 * s4 + g], a[s][s4], acc);
+                    const int pc = 16 * (bJ[s] - k - 1) + li;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) sP[g + 4 * r][pc] = acc[r];
+                }
+            }
+            __syncthreads();
+            // ---- C: trailing update and panel k to global memory.
+            const int t = tid - 64;
+            if (t < 256) store_diag(k, t);
             const int cols = min(n, 16 * nbk) - 16 * (k + 1);
-            for (int e = tid; e < 16 * cols; e += NT) {
-                const int r = e & 15, cl = e >> 4;
+            for (int e = t; e < 16 * cols; e += NT - 64) {
+                const int r = e & 15, cl = e >> 4;  // 16-row runs per column
                 G[(16 * k + r) + (size_t)(16 * (k + 1) + cl) * ldg] = sP[r][cl];
             }
-        }
-        // ---- C: trailing update; block (k+1, k+1) and step A of panel k+1
-        // first on wave (k+1) % 8.
-        if (wave == (k + 1) % kCholWaves) {
-            update_diag(k + 1, k);
-            wave_lds_sync();
-            factor_diag(k + 1);
-        }
-        for (int i = k + 2 + (wave - k - 2 + 8 * kCholWaves) % kCholWaves; i < nbk;
-             i += kCholWaves)
-            update_diag(i, k);
+            for (int i = k + 2 + (wave - 1 - (k + 2) % 7 + 7) % 7; i < nbk; i += 7) {
+                const dh_d4 d = updated_diag(i, k);
 #pragma unroll
-        for (int s = 0; s < kCholSlots; ++s) {
-            if (bI[s] > k && bI[s] < nbk) {
-                const int pi = 16 * (bI[s] - k - 1) + li, pj = 16 * (bJ[s] - k - 1) + li;
+                for (int r = 0; r < 4; ++r) sG[i][li][g + 4 * r] = d[r];
+            }
 #pragma unroll
-                for (int s4 = 0; s4 < 4; ++s4)
-                    a[s] = Mfma<double>::op(-sP[4 * s4 + g][pi], sP[4 * s4 + g][pj], a[s]);
+            for (int s = 0; s < kCholSlots; ++s) {
+                if (bI[s] > k && bI[s] < nbk) {
+                    const int pi = 16 * (bI[s] - k - 1) + li, pj = 16 * (bJ[s] - k - 1) + li;
+#pragma unroll
+                    for (int s4 = 0; s4 < 4; ++s4)
+                        a[s] = Mfma<double>::op(-sP[4 * s4 + g][pi], sP[4 * s4 + g][pj], a[s]);
+                }
             }
         }
     }
+    if (!s_info && tid < 256) store_diag(nbk - 1, tid);
     if (tid == 0) *info = s_info;
 }
 

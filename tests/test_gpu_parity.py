@@ -572,3 +572,34 @@ def test_posv_mixed_nan_rhs_is_reported(dev):
     with pytest.raises(dh.DHError) as ei:
         dev.posv_mixed(dev_mat(np.triu(A)), dev_mat(B), X, 64, 1e-10, 10)
     assert ei.value.status == -1003
+
+
+@pytest.mark.parametrize("n", [2, 15, 16, 17, 31, 33, 96, 97, 112, 113, 209, 271])
+def test_cholqr2_block_edges(dev, n):
+    """The register Cholesky at the edges of its 16-column panels and of the
+    deal of its blocks to the waves: Q^T Q = I, Q R = Y, R upper with a
+    positive diagonal and equal to numpy's up to signs."""
+    import torch
+    rng = np.random.default_rng(n)
+    Y = rng.standard_normal((1500, n)) * np.logspace(0, -3, n)
+    Yd = dev_mat(Y)
+    Rd = torch.zeros((n, n), dtype=torch.float64, device="cuda")
+    assert dev.cholqr2(Yd, Rd) == 0
+    Q, R = dh.from_dev(Yd), dh.from_dev(Rd)
+    assert np.linalg.norm(Q.T @ Q - np.eye(n)) < 1e-12
+    assert rel(Q @ R, Y) < 1e-13
+    assert np.all(np.diag(R) > 0) and np.all(np.tril(R, -1) == 0)
+    assert rel(R, np.abs(np.diag(np.sign(np.diag(np.linalg.qr(Y)[1])))) @
+               (np.sign(np.diag(np.linalg.qr(Y)[1]))[:, None] * np.linalg.qr(Y)[1])) < 1e-11
+
+
+@pytest.mark.parametrize("bad", [1, 4, 5, 16, 17, 30, 47])
+def test_cholqr2_reports_the_failing_pivot(dev, bad):
+    """A zero column is the first failing pivot of its sweep, wherever it lies in
+    the four-row steps and the panels; the shifted sweep then fails at the same
+    place in its second pass or returns a completed basis status."""
+    rng = np.random.default_rng(bad)
+    Y = rng.standard_normal((400, 48))
+    Y[:, bad - 1] = 0.0
+    st = dev.cholqr2(dev_mat(Y))
+    assert st > 0 and st % 1000000 == bad
