@@ -10,6 +10,7 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <mutex>
 #include <new>
 
 #include <utility>
@@ -29,6 +30,74 @@ int dh_fail(int code, const char* fmt, ...) {
 
 extern "C" const char* dh_last_error_string(void) { return g_last_error; }
 
+namespace {
+struct Scratch {
+    std::mutex mu;
+    void* p = nullptr;
+    size_t size = 0;
+    bool busy = false;
+    int handles = 0;  // handles alive on the device
+    void drop() {     // mu held, not busy: no queued work reads the buffer
+        if (p) (void)hipFree(p);
+        p = nullptr;
+        size = 0;
+    }
+};
+constexpr int kMaxDevices = 64;
+Scratch g_scratch[kMaxDevices];
+
+// Handle count of the device; the last one to go gives the buffer back.
+void scratch_count(int device, int add) {
+    if (device >= kMaxDevices) return;
+    Scratch& s = g_scratch[device];
+    std::lock_guard<std::mutex> lock(s.mu);
+    s.handles += add;
+    if (s.handles == 0) s.drop();
+}
+
+// Gives an idle buffer back; false if there is none.
+bool scratch_trim(int device) {
+    if (device >= kMaxDevices) return false;
+    Scratch& s = g_scratch[device];
+    std::lock_guard<std::mutex> lock(s.mu);
+    if (s.busy || !s.p) return false;
+    s.drop();
+    return true;
+}
+}  // namespace
+
+void* dh_scratch_take(int device, size_t bytes) {
+    int current = -1;  // hipMalloc takes the current device's memory
+    if (device >= kMaxDevices || hipGetDevice(&current) != hipSuccess || current != device)
+        return nullptr;
+    Scratch& s = g_scratch[device];
+    std::lock_guard<std::mutex> lock(s.mu);
+    if (s.busy) return nullptr;
+    if (s.size < bytes) {
+        size_t avail = 0, total = 0;
+        if (hipMemGetInfo(&avail, &total) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        if (bytes > total / 8 || bytes > (avail + s.size) / 2) return nullptr;
+        s.drop();
+        if (hipMalloc(&s.p, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            s.p = nullptr;
+            return nullptr;
+        }
+        s.size = bytes;
+    }
+    s.busy = true;
+    return s.p;
+}
+
+void dh_scratch_release(int device) {
+    Scratch& s = g_scratch[device];
+    std::lock_guard<std::mutex> lock(s.mu);
+    s.busy = false;
+}
+
 void* dh_ws(dh_handle_t h, dh_slot slot, size_t bytes) {
     if (bytes == 0) bytes = 256;
     if (h->ws_size[slot] >= bytes) return h->ws[slot];
@@ -44,7 +113,12 @@ void* dh_ws(dh_handle_t h, dh_slot slot, size_t bytes) {
     size_t want = bytes + bytes / 8;  // headroom for slightly larger later calls
     want = (want + 4095) & ~size_t(4095);
     void* p = nullptr;
-    if (hipMalloc(&p, want) != hipSuccess) {
+    hipError_t e = hipMalloc(&p, want);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        if (scratch_trim(h->device)) e = hipMalloc(&p, want);
+    }
+    if (e != hipSuccess) {
         (void)hipGetLastError();
         dh_fail(DH_ERR_ALLOC, "hipMalloc of %zu bytes (workspace slot %d) failed", want, (int)slot);
         return nullptr;
@@ -80,6 +154,7 @@ extern "C" int dh_create(int device, void* stream, dh_handle_t* out) {
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, device) == hipSuccess) h->num_cu = prop.multiProcessorCount;
     if (h->num_cu <= 0) h->num_cu = 256;
+    scratch_count(device, 1);
     *out = h;
     return 0;
 }
@@ -101,6 +176,7 @@ extern "C" int dh_destroy(dh_handle_t h) {
     if (h->host_status) (void)hipHostFree(h->host_status);
     delete static_cast<std::map<std::pair<const void*, int>, int>*>(h->occupancy);
     if (h->own_stream) (void)hipStreamDestroy(h->stream);
+    scratch_count(h->device, -1);
     delete h;
     return 0;
 }

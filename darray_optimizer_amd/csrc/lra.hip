@@ -13,7 +13,8 @@
 int dh_project_f64_split(dh_handle_t h, int m, int n, int d, int l, const double* Xi, int ldxi,
                         const double* Xj, int ldxj, const double* ni, const double* nj,
                         const double* yi, const double* yj, double gamma, const double* O,
-                        int ldo, double beta, double* Y, int ldy);
+                        int ldo, double* Y, int ldy, void* keep, int kmode);
+size_t dh_kkeep_bytes(int m, int n, int d);
 int dh_lra_bf16_passes(dh_handle_t h, int n, int d, int l, int q, const double* X, int ldx,
                        const double* y, double gamma, const double* Omega, int ldo, double* Q,
                        int ldq, double* W, int ldw);
@@ -369,29 +370,53 @@ static int copy_panel(dh_handle_t h, int n, int l, const double* src, int lds, d
     return 0;
 }
 
+// The device's scratch buffer for the length of a call (p = nullptr: not available).
+struct ScratchHold {
+    dh_handle_t h;
+    void* p;
+    ScratchHold(dh_handle_t h_, size_t bytes) : h(h_), p(dh_scratch_take(h_->device, bytes)) {}
+    ~ScratchHold() {
+        if (!p) return;
+        (void)hipStreamSynchronize(h->stream);
+        dh_scratch_release(h->device);
+    }
+    ScratchHold(const ScratchHold&) = delete;
+    ScratchHold& operator=(const ScratchHold&) = delete;
+};
+
 // FP64 passes: Y = K*Omega -> Q; q x { K*Q -> orthonormal basis }; W = K*Q.
+//
+// All q + 2 passes multiply the same K, so the first one stores it (8 n^2
+// bytes: 34 GB at n = 65536, of 288) and the others read it back instead of
+// forming it again: at 8 bytes per 2l flops that read is a tenth of what HBM
+// gives, while the distances and exponentials it saves are almost half of a
+// pass at d = 128, l = 272 (66.0 ms with them, 36.5 ms without: 82% of the FP64
+// MFMA peak; the solve 265 -> 178 ms).  Where the device's scratch buffer
+// cannot be had every pass forms K; the bits are the same.
 static int lra_f64(dh_handle_t h, int n, int d, int l, int q, const double* X, int ldx,
                    const double* y, double gamma, const double* Omega, int ldo, double* Q,
                    int ldq, double* W, int ldw) {
     double* nrm = (double*)dh_ws(h, DH_WS_NORMS, sizeof(double) * (size_t)n);
     if (!nrm) return DH_ERR_ALLOC;
     DH_CHECK_STATUS(dh_sqnorms_f64(h, n, d, X, ldx, nrm));
+    const ScratchHold kk(h, dh_kkeep_bytes(n, n, d));
+    const int store = kk.p ? 1 : 0, use = kk.p ? 2 : 0;
     DH_CHECK_STATUS(dh_project_f64_split(h, n, n, d, l, X, ldx, X, ldx, nrm, nrm, y, y, gamma,
-                                        Omega, ldo, 0.0, Q, ldq));
+                                        Omega, ldo, Q, ldq, kk.p, store));
     DH_CHECK_STATUS(dh_range_orth(h, n, l, Q, ldq));
     // Power iterations alternate the basis between Q and W (no copy for even q).
     double *cur = Q, *nxt = W;
     int ldc = ldq, ldn = ldw;
     for (int it = 0; it < q; ++it) {
         DH_CHECK_STATUS(dh_project_f64_split(h, n, n, d, l, X, ldx, X, ldx, nrm, nrm, y, y, gamma,
-                                            cur, ldc, 0.0, nxt, ldn));
+                                            cur, ldc, nxt, ldn, kk.p, use));
         DH_CHECK_STATUS(dh_range_orth(h, n, l, nxt, ldn));
         std::swap(cur, nxt);
         std::swap(ldc, ldn);
     }
     if (cur != Q) DH_CHECK_STATUS(copy_panel(h, n, l, cur, ldc, Q, ldq));
-    return dh_project_f64_split(h, n, n, d, l, X, ldx, X, ldx, nrm, nrm, y, y, gamma, Q, ldq, 0.0,
-                               W, ldw);
+    return dh_project_f64_split(h, n, n, d, l, X, ldx, X, ldx, nrm, nrm, y, y, gamma, Q, ldq, W,
+                               ldw, kk.p, use);
 }
 
 extern "C" int dh_lra(dh_handle_t h, int prec, int n, int d, int l, int q, const double* X,

@@ -214,13 +214,19 @@ __global__ __launch_bounds__(256) void pack_omega_f64_kernel(int n, int l, int n
     Opk[idx] = v;
 }
 
-template <int DK, int NCB, bool PK>
+// KEEP: column group 0 also stores every wave's K values (labels left out) to
+// Kk as the projection MFMAs take them, for kept_project_f64_kernel: 128 pairs
+// per (16-point chunk, 16-row block), pair h 64 + L = (kv[2h], kv[2h + 1]) of
+// lane L; nrb row blocks per chunk.  Chunks are outermost because all waves
+// walk them together: the reads and writes of any moment lie side by side.
+template <int DK, int NCB, bool PK, bool KEEP>
 __global__ __launch_bounds__(256) void rbf_project_f64_kernel(
     int m, int n, int d, int l, const double* __restrict__ Xi, int ldxi,
     const double* __restrict__ Xj, int ldxj, const double* __restrict__ ni,
     const double* __restrict__ nj, const double* __restrict__ yi, const double* __restrict__ yj,
     double gamma, const double* __restrict__ O, int ldo, const d2v* __restrict__ Opk, int ncbp,
-    double beta, double* __restrict__ Y, int ldy, int jps, long ystride) {
+    double beta, double* __restrict__ Y, int ldy, int jps, long ystride, d2v* __restrict__ Kk,
+    int nrb) {
     constexpr int JB = 16;
     {  // split z of the j range: points [z jps, min((z + 1) jps, n)), partial into Y + z ystride
         const int j0 = blockIdx.z * jps;
@@ -230,6 +236,7 @@ __global__ __launch_bounds__(256) void rbf_project_f64_kernel(
         if (yj) yj += j0;
         O += j0;
         if (PK) Opk += (size_t)(j0 / JB) * ncbp * 128;
+        if (KEEP) Kk += ((size_t)(j0 / JB) * nrb + blockIdx.x * 4 + (threadIdx.x >> 6)) * 128;
         Y += blockIdx.z * ystride;
     }
     constexpr int FD = DK * 4;  // padded feature count
@@ -334,6 +341,11 @@ __global__ __launch_bounds__(256) void rbf_project_f64_kernel(
             d2 = d2 > 0.0 ? d2 : 0.0;
             kv[r] = exp_kernel_f64(-gamma * d2);
         }
+        if (KEEP && blockIdx.y == 0) {
+            d2v* kp = Kk + (size_t)(j0 / JB) * nrb * 128 + lane;
+            kp[0] = d2v{kv[0], kv[1]};
+            kp[64] = d2v{kv[2], kv[3]};
+        }
         const int sl = lane ^ ((lane >> 4) << 2);
 #pragma unroll
         for (int cb = 0; cb < NCB; ++cb) {
@@ -362,23 +374,96 @@ __global__ __launch_bounds__(256) void rbf_project_f64_kernel(
         }
 }
 
+// Y = K O from the K values that a KEEP pass stored, with that pass's packed
+// Omega image, chunk order and MFMAs, so it returns the bits that the fused
+// kernel would.  Rows, columns and splits as there; what is gone is the
+// distance product (2d of the 2(d + l) flops per entry), the exp, and the
+// staging of X, and with it the registers and LDS that held the fused kernel
+// to one workgroup per CU at l = 272: here two fit.  K comes from HBM once per
+// column group, 8 bytes per entry, a chunk ahead in registers.
+template <int NCB>
+__global__ __launch_bounds__(256, 2) void kept_project_f64_kernel(
+    int m, int n, int l, const d2v* __restrict__ Kk, int nrb, const double* __restrict__ yi,
+    const d2v* __restrict__ Opk, int ncbp, double* __restrict__ Y, int ldy, int jps,
+    long ystride) {
+    constexpr int JB = 16;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int jz = blockIdx.z * jps;
+    const int nch = (min(jps, n - jz) + JB - 1) / JB;
+    Opk += ((size_t)(jz / JB) * ncbp + blockIdx.y * NCB) * 128;
+    Kk += ((size_t)(jz / JB) * nrb + blockIdx.x * 4 + wave) * 128 + lane;
+    const size_t kstep = (size_t)nrb * 128;
+    Y += blockIdx.z * ystride;
+    __shared__ d2v sO[2][NCB][2][64];
+    const int g = lane >> 4, li = lane & 15, sl = lane ^ (g << 2);
+    dh_d4 acc[NCB];
+#pragma unroll
+    for (int cb = 0; cb < NCB; ++cb) acc[cb] = dh_d4{0, 0, 0, 0};
+    auto dma_omega = [&](int t, int b) {
+        const d2v* src = Opk + (size_t)t * ncbp * 128;
+#pragma unroll
+        for (int k = 0; k < 2 * NCB; k += 4) {
+            const int kk = k + wave;
+            if ((2 * NCB) % 4 == 0 || kk < 2 * NCB)
+                dma16(src + kk * 64, (unsigned)lane * 16u, &sO[b][kk >> 1][kk & 1][0]);
+        }
+    };
+    d2v k01 = Kk[0], k23 = Kk[64];
+    dma_omega(0, 0);
+    wait_vm();
+    __syncthreads();
+    for (int t = 0; t < nch; ++t) {
+        const int b = t & 1, tn = min(t + 1, nch - 1);
+        const d2v n01 = Kk[tn * kstep], n23 = Kk[tn * kstep + 64];
+        if (t + 1 < nch) dma_omega(t + 1, b ^ 1);
+#pragma unroll
+        for (int cb = 0; cb < NCB; ++cb) {
+            const d2v o01 = sO[b][cb][0][sl], o23 = sO[b][cb][1][sl];
+            acc[cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(k01[0], o01[0], acc[cb], 0, 0, 0);
+            acc[cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(k01[1], o01[1], acc[cb], 0, 0, 0);
+            acc[cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(k23[0], o23[0], acc[cb], 0, 0, 0);
+            acc[cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(k23[1], o23[1], acc[cb], 0, 0, 0);
+        }
+        k01 = n01;
+        k23 = n23;
+        wait_vm();
+        __syncthreads();
+    }
+#pragma unroll
+    for (int cb = 0; cb < NCB; ++cb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int i = blockIdx.x * 64 + wave * 16 + g + 4 * r;
+            const int c = (blockIdx.y * NCB + cb) * 16 + li;
+            if (i < m && c < l) {
+                double v = acc[cb][r];
+                if (yi) v *= yi[i];
+                Y[i + (size_t)c * ldy] = v;
+            }
+        }
+}
+
 template <int DK, int NCB>
 static void launch_project_f64(dh_handle_t h, dim3 grid, int m, int n, int d, int l,
                                const double* Xi, int ldxi, const double* Xj, int ldxj,
                                const double* ni, const double* nj, const double* yi,
                                const double* yj, double gamma, const double* O, int ldo,
                                const d2v* Opk, int ncbp, double beta, double* Y, int ldy, int jps,
-                               long ystride) {
+                               long ystride, d2v* Kk) {
     if constexpr (DK < 64 || NCB <= 12) {  // d > 128 with 17 blocks is never selected (spills)
         dh_timing_begin(h);
-        if (Opk)
-            rbf_project_f64_kernel<DK, NCB, true><<<grid, 256, 0, h->stream>>>(
+        if (Opk && Kk)
+            rbf_project_f64_kernel<DK, NCB, true, true><<<grid, 256, 0, h->stream>>>(
                 m, n, d, l, Xi, ldxi, Xj, ldxj, ni, nj, yi, yj, gamma, O, ldo, Opk, ncbp, beta, Y,
-                ldy, jps, ystride);
+                ldy, jps, ystride, Kk, 4 * grid.x);
+        else if (Opk)
+            rbf_project_f64_kernel<DK, NCB, true, false><<<grid, 256, 0, h->stream>>>(
+                m, n, d, l, Xi, ldxi, Xj, ldxj, ni, nj, yi, yj, gamma, O, ldo, Opk, ncbp, beta, Y,
+                ldy, jps, ystride, nullptr, 0);
         else
-            rbf_project_f64_kernel<DK, NCB, false><<<grid, 256, 0, h->stream>>>(
+            rbf_project_f64_kernel<DK, NCB, false, false><<<grid, 256, 0, h->stream>>>(
                 m, n, d, l, Xi, ldxi, Xj, ldxj, ni, nj, yi, yj, gamma, O, ldo, nullptr, 0, beta, Y,
-                ldy, jps, ystride);
+                ldy, jps, ystride, nullptr, 0);
         dh_timing_end(h);
     }
 }
@@ -388,11 +473,11 @@ static int dispatch_ncb(dh_handle_t h, int ncb, dim3 grid, int m, int n, int d, 
                         const double* Xi, int ldxi, const double* Xj, int ldxj, const double* ni,
                         const double* nj, const double* yi, const double* yj, double gamma,
                         const double* O, int ldo, const d2v* Opk, int ncbp, double beta,
-                        double* Y, int ldy, int jps, long ystride) {
+                        double* Y, int ldy, int jps, long ystride, d2v* Kk) {
 #define DH_NCB(N)                                                                              \
     case N:                                                                                    \
         launch_project_f64<DK, N>(h, grid, m, n, d, l, Xi, ldxi, Xj, ldxj, ni, nj, yi, yj, gamma, \
-                                  O, ldo, Opk, ncbp, beta, Y, ldy, jps, ystride);              \
+                                  O, ldo, Opk, ncbp, beta, Y, ldy, jps, ystride, Kk);          \
         break;
     switch (ncb) {
         DH_NCB(1)
@@ -419,23 +504,28 @@ static int dispatch_ncb(dh_handle_t h, int ncb, dim3 grid, int m, int n, int d, 
 // distance-GEMM tile kernel (FP64 MFMA, exp epilogue), and multiplied into
 // Omega by the FP64 GEMM: Y_blk = K_blk Omega + beta Y_blk.  The same split as
 // rbf_kernel's explicit tiles (dkernel.cu:144-178), with the product fused in.
+// With `keep` (m n doubles) every block has its own place there: kmode 1 forms
+// the blocks, kmode 2 takes them as an earlier pass left them.
 static int project_f64_blocked(dh_handle_t h, int m, int n, int d, int l, const double* Xi,
                                int ldxi, const double* Xj, int ldxj, const double* ni,
                                const double* nj, const double* yi, const double* yj, double gamma,
-                               const double* O, int ldo, double beta, double* Y, int ldy) {
+                               const double* O, int ldo, double beta, double* Y, int ldy,
+                               double* keep, int kmode) {
     if (n == 0)  // K has no columns: Y = beta Y
         return dh_gemm_impl<double>(h, false, false, m, l, 0, 1.0, O, 1, O, ldo, beta, Y, ldy, 0);
     const long cap = 1L << 27;
     int mb = (int)std::min<long>(m, std::max<long>(64, cap / n / 64 * 64));
-    double* Kb = (double*)dh_ws(h, DH_WS_KBLOCK, sizeof(double) * (size_t)mb * n);
+    double* Kb = keep ? keep : (double*)dh_ws(h, DH_WS_KBLOCK, sizeof(double) * (size_t)mb * n);
     if (!Kb) return DH_ERR_ALLOC;
     dh_timing_begin(h);
     for (int i0 = 0; i0 < m; i0 += mb) {
         const int ib = std::min(mb, m - i0);
+        if (keep) Kb = keep + (size_t)i0 * n;
         dim3 grid(dh_cdiv(ib, 64), dh_cdiv(n, 64));
-        rbf_tile_kernel<double, 64, 64><<<grid, 256, 0, h->stream>>>(
-            ib, n, d, Xi + (size_t)i0 * ldxi, ldxi, Xj, ldxj, ni + i0, nj, yi ? yi + i0 : nullptr,
-            yj, gamma, Kb, ib);
+        if (kmode != 2)
+            rbf_tile_kernel<double, 64, 64><<<grid, 256, 0, h->stream>>>(
+                ib, n, d, Xi + (size_t)i0 * ldxi, ldxi, Xj, ldxj, ni + i0, nj,
+                yi ? yi + i0 : nullptr, yj, gamma, Kb, ib);
         DH_CHECK_LAUNCH();
         DH_CHECK_STATUS(dh_gemm_impl<double>(h, false, false, ib, l, n, 1.0, Kb, ib, O, ldo, beta,
                                              Y + i0, ldy, 0));
@@ -452,6 +542,64 @@ static int ncb_instance(int want) {
     return 17;
 }
 
+// Omega (labels folded in) as the fused kernels' LDS images, ncbp column blocks.
+static int pack_omega_f64(dh_handle_t h, int n, int l, int ncbp, const double* O, int ldo,
+                          const double* yj, const d2v** Opk) {
+    const int nch = dh_cdiv(n, 16);
+    const long pairs = (long)nch * ncbp * 128;
+    d2v* P = (d2v*)dh_ws(h, DH_WS_PACK64, sizeof(d2v) * (size_t)pairs);
+    if (!P) return DH_ERR_ALLOC;
+    pack_omega_f64_kernel<<<dh_cdiv(pairs, 256), 256, 0, h->stream>>>(n, l, nch, ncbp, O, ldo, yj,
+                                                                     P);
+    DH_CHECK_LAUNCH();
+    *Opk = P;
+    return 0;
+}
+
+// Y (m x l) = K O from the kept K values (kept_project_f64_kernel).  Without
+// the distance operands 17 column blocks fit at every d, and how the columns
+// are grouped changes no bit.
+static int project_f64_kept(dh_handle_t h, int m, int n, int l, const double* yi,
+                            const double* yj, const double* O, int ldo, double* Y, int ldy,
+                            int jps, int splits, long ystride, const void* keep) {
+    const int ncb_total = dh_cdiv(l, 16);
+    const int ncb = ncb_instance(dh_cdiv(ncb_total, dh_cdiv(ncb_total, 17)));
+    const int groups = dh_cdiv(ncb_total, ncb);
+    const d2v* Opk = nullptr;
+    DH_CHECK_STATUS(pack_omega_f64(h, n, l, groups * ncb, O, ldo, yj, &Opk));
+    dim3 grid(dh_cdiv(m, 64), groups, splits);
+    dh_timing_begin(h);
+#define DH_NCB(N)                                                                            \
+    case N:                                                                                  \
+        kept_project_f64_kernel<N><<<grid, 256, 0, h->stream>>>(                             \
+            m, n, l, (const d2v*)keep, 4 * grid.x, yi, Opk, groups* ncb, Y, ldy, jps,        \
+            ystride);                                                                        \
+        break;
+    switch (ncb) {
+        DH_NCB(1)
+        DH_NCB(2)
+        DH_NCB(3)
+        DH_NCB(4)
+        DH_NCB(5)
+        DH_NCB(6)
+        DH_NCB(8)
+        DH_NCB(9)
+        DH_NCB(12)
+        default:
+            DH_NCB(17)
+    }
+#undef DH_NCB
+    dh_timing_end(h);
+    DH_CHECK_LAUNCH();
+    return 0;
+}
+
+// Bytes that dh_project_f64_split needs to keep K (m x n, d features).
+size_t dh_kkeep_bytes(int m, int n, int d) {
+    if (d > 256) return sizeof(double) * (size_t)m * n;
+    return sizeof(double) * ((size_t)dh_cdiv(m, 64) * 64) * ((size_t)dh_cdiv(n, 16) * 16);
+}
+
 // Y (m x l) = K(Xi, Xj) O + beta Y with the fused kernel, the j range in
 // `splits` parts (partials to P + z ystride, ld m, when splits > 1).
 // With `pack`, Omega is first packed (labels folded in) into the kernel's LDS
@@ -462,22 +610,15 @@ static int project_f64_fused(dh_handle_t h, int m, int n, int d, int l, const do
                              int ldxi, const double* Xj, int ldxj, const double* ni,
                              const double* nj, const double* yi, const double* yj, double gamma,
                              const double* O, int ldo, double beta, double* Y, int ldy, int ncb,
-                             int groups, int jps, int splits, long ystride, bool pack) {
+                             int groups, int jps, int splits, long ystride, bool pack,
+                             void* keep) {
     dim3 grid(dh_cdiv(m, 64), groups, splits);
     const d2v* Opk = nullptr;
-    const int ncbp = groups * ncb, nch = dh_cdiv(n, 16);
-    if (pack) {
-        const long pairs = (long)nch * ncbp * 128;
-        d2v* P = (d2v*)dh_ws(h, DH_WS_PACK64, sizeof(d2v) * (size_t)pairs);
-        if (!P) return DH_ERR_ALLOC;
-        pack_omega_f64_kernel<<<dh_cdiv(pairs, 256), 256, 0, h->stream>>>(n, l, nch, ncbp, O, ldo,
-                                                                         yj, P);
-        DH_CHECK_LAUNCH();
-        Opk = P;
-    }
+    const int ncbp = groups * ncb;
+    if (pack) DH_CHECK_STATUS(pack_omega_f64(h, n, l, ncbp, O, ldo, yj, &Opk));
 #define DH_DK(K)                                                                              \
     dispatch_ncb<K>(h, ncb, grid, m, n, d, l, Xi, ldxi, Xj, ldxj, ni, nj, yi, yj, gamma, O, ldo, \
-                    Opk, ncbp, beta, Y, ldy, jps, ystride)
+                    Opk, ncbp, beta, Y, ldy, jps, ystride, (d2v*)keep)
     if (d <= 32) return DH_DK(8);
     if (d <= 64) return DH_DK(16);
     if (d <= 128) return DH_DK(32);
@@ -505,11 +646,11 @@ int dh_project_f64_impl(dh_handle_t h, int m, int n, int d, int l, const double*
         return dh_gemm_impl<double>(h, false, false, m, l, 0, 1.0, O, 1, O, ldo, beta, Y, ldy, 0);
     if (d > 256)
         return project_f64_blocked(h, m, n, d, l, Xi, ldxi, Xj, ldxj, ni, nj, yi, yj, gamma, O,
-                                   ldo, beta, Y, ldy);
+                                   ldo, beta, Y, ldy, nullptr, 0);
     int ncb, groups;
     f64_columns(d, l, &ncb, &groups);
     return project_f64_fused(h, m, n, d, l, Xi, ldxi, Xj, ldxj, ni, nj, yi, yj, gamma, O, ldo,
-                             beta, Y, ldy, ncb, groups, n, 1, 0, pack);
+                             beta, Y, ldy, ncb, groups, n, 1, 0, pack, nullptr);
 }
 
 // Y = beta Y + sum over the splits z (in order) of P[z ystride + i + c m].
@@ -526,32 +667,46 @@ __global__ __launch_bounds__(256) void sum_splits_f64_kernel(int m, int l, int s
     *yp = (beta == 0.0) ? v : v + beta * (*yp);
 }
 
-// As dh_project_f64_impl; a grid of at most half a workgroup per CU splits
-// the j range over more workgroups (partials in a workspace, summed in order).
-// The range finder's passes use it; dh_rbf_project_f64 keeps the one-launch
-// form, so its allocation-free twin returns the same bits.
+// Y = K O as dh_project_f64_impl with beta = 0; a grid of at most half a
+// workgroup per CU splits the j range over more workgroups (partials in a
+// workspace, summed in order).  The range finder's passes use it;
+// dh_rbf_project_f64 keeps the one-launch form, so its allocation-free twin
+// returns the same bits.  kmode 1 also stores K to `keep` (dh_kkeep_bytes), and
+// kmode 2 takes it from there instead of forming it: same points, same bits.
 int dh_project_f64_split(dh_handle_t h, int m, int n, int d, int l, const double* Xi, int ldxi,
                          const double* Xj, int ldxj, const double* ni, const double* nj,
                          const double* yi, const double* yj, double gamma, const double* O,
-                         int ldo, double beta, double* Y, int ldy) {
-    if (m == 0 || l == 0 || n == 0 || d > 256)
+                         int ldo, double* Y, int ldy, void* keep, int kmode) {
+    if (m == 0 || l == 0) return 0;
+    if (n == 0)
         return dh_project_f64_impl(h, m, n, d, l, Xi, ldxi, Xj, ldxj, ni, nj, yi, yj, gamma, O,
-                                   ldo, beta, Y, ldy, true);
+                                   ldo, 0.0, Y, ldy, true);
+    if (d > 256)
+        return project_f64_blocked(h, m, n, d, l, Xi, ldxi, Xj, ldxj, ni, nj, yi, yj, gamma, O,
+                                   ldo, 0.0, Y, ldy, (double*)keep, kmode);
     int ncb, groups;
     f64_columns(d, l, &ncb, &groups);
     const int nch = dh_cdiv(n, 32);
     const int splits = dh_j_splits(h->num_cu, (long)dh_cdiv(m, 64) * groups, nch);
-    if (splits == 1)
-        return project_f64_fused(h, m, n, d, l, Xi, ldxi, Xj, ldxj, ni, nj, yi, yj, gamma, O,
-                                 ldo, beta, Y, ldy, ncb, groups, n, 1, 0, true);
-    const int jps = dh_cdiv(nch, splits) * 32;
-    const long ystride = (long)m * l;
-    double* P = (double*)dh_ws(h, DH_WS_SPLITN, sizeof(double) * (size_t)ystride * splits);
-    if (!P) return DH_ERR_ALLOC;
-    DH_CHECK_STATUS(project_f64_fused(h, m, n, d, l, Xi, ldxi, Xj, ldxj, ni, nj, yi, yj, gamma, O,
-                                      ldo, 0.0, P, m, ncb, groups, jps, splits, ystride, true));
+    const int jps = splits == 1 ? n : dh_cdiv(nch, splits) * 32;
+    const long ystride = splits == 1 ? 0 : (long)m * l;
+    double* P = Y;
+    int ldp = ldy;
+    if (splits > 1) {
+        P = (double*)dh_ws(h, DH_WS_SPLITN, sizeof(double) * (size_t)ystride * splits);
+        if (!P) return DH_ERR_ALLOC;
+        ldp = m;
+    }
+    if (keep && kmode == 2)
+        DH_CHECK_STATUS(project_f64_kept(h, m, n, l, yi, yj, O, ldo, P, ldp, jps, splits, ystride,
+                                         keep));
+    else
+        DH_CHECK_STATUS(project_f64_fused(h, m, n, d, l, Xi, ldxi, Xj, ldxj, ni, nj, yi, yj,
+                                          gamma, O, ldo, 0.0, P, ldp, ncb, groups, jps, splits,
+                                          ystride, true, keep));
+    if (splits == 1) return 0;
     sum_splits_f64_kernel<<<dh_cdiv(ystride, 256), 256, 0, h->stream>>>(m, l, splits, P, ystride,
-                                                                        beta, Y, ldy);
+                                                                        0.0, Y, ldy);
     DH_CHECK_LAUNCH();
     return 0;
 }

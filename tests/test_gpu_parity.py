@@ -603,3 +603,55 @@ def test_cholqr2_reports_the_failing_pivot(dev, bad):
     Y[:, bad - 1] = 0.0
     st = dev.cholqr2(dev_mat(Y))
     assert st > 0 and st % 1000000 == bad
+
+
+@pytest.mark.parametrize("n,d,l,labels", [(17, 3, 5, True), (64, 16, 16, False),
+                                          (65, 33, 1, False), (1000, 40, 96, True),
+                                          (2051, 130, 200, True), (900, 70, 280, False),
+                                          (300, 257, 20, True), (11700, 257, 3, False)])
+def test_lra_passes_on_kept_kernel_values(dev, n, d, l, labels):
+    """The FP64 range finder's later passes take K from the values its first
+    pass stored: W must be K Q for the returned Q, as the one-launch pass
+    forms it.  Both sum n products K_ij Q_jc, in different orders, so element
+    (i, c) may differ by 2 n u (K |Q|)_ic; K is in (0, 1]."""
+    import torch
+    rng = np.random.default_rng(n + d)
+    X = rng.standard_normal((n, d)) * 0.3
+    y = dev_vec(rng.choice([-1.0, 1.0], n)) if labels else None
+    Xd = dev_pts(X)
+    Om = dev_mat(rng.standard_normal((n, l)))
+    Q, W, P = (empty_mat(n, l, torch.float64) for _ in range(3))
+    assert dev.lra(Xd, Om, 1.0 / d, 2, Q, W, y=y) == 0
+    dev.rbf_project_f64(Xd, Xd, Q, 1.0 / d, P, yi=y, yj=y)
+    A = empty_mat(n, l, torch.float64)
+    dev.rbf_project_f64(Xd, Xd, Q.abs(), 1.0 / d, A)
+    assert bool(((W - P).abs() <= 2 * n * 2.0**-53 * A).all())
+
+
+def test_lra_in_two_threads_gives_the_same_bits():
+    """Two handles at once: one holds the device's scratch buffer, the other
+    forms K in every pass, and both return the bits of a call on its own."""
+    import threading
+
+    import torch
+    rng = np.random.default_rng(5)
+    X = dev_pts(rng.standard_normal((3000, 20)) * 0.3)
+    Om = dev_mat(rng.standard_normal((3000, 40)))
+    hs = [dh.Handle(0) for _ in range(2)]
+    out = [[empty_mat(3000, 40, torch.float64) for _ in range(2)] for _ in range(3)]
+    hs[0].lra(X, Om, 0.05, 1, *out[2])
+    torch.cuda.synchronize()
+
+    def work(i):
+        for _ in range(20):
+            hs[i].lra(X, Om, 0.05, 1, *out[i])
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for o in out[:2]:
+        assert torch.equal(o[0], out[2][0]) and torch.equal(o[1], out[2][1])
+    for h in hs:
+        h.close()
