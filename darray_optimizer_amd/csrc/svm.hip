@@ -9,14 +9,15 @@
 // search, t *= 20 until the gap 2n/t is below 1e-5 |f|.
 //
 // Per CG iteration Z is read twice (Z^T p by row chunks and column groups,
-// then Z v by rows): 2 n k 8 bytes, HBM-bound.  All reductions are
+// then Z v by rows), 2 n k 8 bytes, in four launches: the new direction and
+// Z^T p, the sum of its chunks, Z v and p.q, the update.  All reductions are
 // per-workgroup partial sums combined in a fixed order, so results are
 // deterministic.  Scalars of the CG recurrence stay on the device, and so
-// does the stopping test: the last kernel of an iteration clears an active
-// flag that the kernels of later iterations check first, so the host queues
-// iterations in batches and reads the flag once per batch (the iterate is the
-// one an iteration-by-iteration loop would stop at).  The line-search values
-// are read once per Newton step.
+// does the stopping test: the kernel that starts an iteration ends the one
+// before it, and every later kernel of a stopped loop returns at once, so the
+// host queues iterations in batches and reads the state once per batch (the
+// iterate is the one an iteration-by-iteration loop would stop at).  The
+// line-search values are read once per Newton step.
 //
 // Deviations from the reference (bug fixes), as the oracle states them: the
 // CG right-hand side is -grad (the reference solves with b = e_1,
@@ -54,62 +55,153 @@ __device__ __forceinline__ double block_sum(double v, double* sh) {
     return s;
 }
 
-// Sum of count values part[0..count) in a fixed order by one workgroup of
-// 256 threads; the result is returned to every thread.
-__device__ double fixed_sum(int count, const double* __restrict__ part, double* sh) {
-    double v = 0.0;
-    for (int i = threadIdx.x; i < count; i += 256) v += part[i];
-    v = wave_sum(v);
+// State of the CG loop between two iterations, in device memory.
+struct CgState {
+    double active, iters, rr, rz;
+};
+
+// Kernels of the CG iteration take the state of their iteration and do nothing
+// once the loop has stopped; NULL = always run.
+__device__ __forceinline__ bool cg_stopped(const CgState* st) { return st && st->active == 0.0; }
+
+// End of an iteration: the new r.z and r.r from the update's partial sums (in
+// a fixed order, the same in every workgroup of 256 threads), one more
+// iteration counted, and the stopping test sqrt(r.r) <= tol or max_iter.
+__device__ CgState cg_next(const CgState old, int nblk, const double* __restrict__ part2,
+                           double tol, int max_iter) {
+    __shared__ double sh0[4], sh1[4];
+    double v0 = 0.0, v1 = 0.0;
+    for (int b = threadIdx.x; b < nblk; b += 256) {
+        v0 += part2[2 * b];
+        v1 += part2[2 * b + 1];
+    }
+    v0 = wave_sum(v0);
+    v1 = wave_sum(v1);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (lane == 0) {
+        sh0[wave] = v0;
+        sh1[wave] = v1;
+    }
     __syncthreads();
-    if (lane == 0) sh[wave] = v;
-    __syncthreads();
-    const double total = (sh[0] + sh[1]) + (sh[2] + sh[3]);
-    __syncthreads();  // sh is reused by the caller
-    return total;
+    CgState st;
+    st.rz = (sh0[0] + sh0[1]) + (sh0[2] + sh0[3]);
+    st.rr = (sh1[0] + sh1[1]) + (sh1[2] + sh1[3]);
+    st.iters = old.iters + 1.0;
+    st.active = (sqrt(st.rr) > tol && st.iters < (double)max_iter) ? 1.0 : 0.0;
+    return st;
 }
 
-// part[c * nchunks + chunk] = sum over the chunk's rows of Z[r, c] * x[r].
-// Kernels of the CG iteration take `ctl` (the loop's control words, ctl[0] =
-// active flag) and do nothing once the loop has stopped; NULL = always run.
-__device__ __forceinline__ bool cg_stopped(const double* ctl) { return ctl && ctl[0] == 0.0; }
+// part[c * nchunks + chunk] = sum over the chunk's rows of Z[r, c] * xv, xv the
+// lane's values of rows chunk * kRows + lane + 64 i, for the workgroup's
+// kColGrp columns.  A wave has all its 8 columns in flight at once (one round
+// trip to memory instead of eight), and reduces them together: each exchange
+// of the butterfly hands half of the columns to the other half of the lanes, 10
+// shuffles instead of 48 with the same pairs in every sum.
+__device__ __forceinline__ void ztx_columns(int n, int k, const double* __restrict__ Z, int ldz,
+                                            const double (&xv)[4], double* __restrict__ part) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int chunk = blockIdx.x, nchunks = gridDim.x, r0 = chunk * kRows + lane;
+    constexpr int NC = kColGrp / 4;
+    static_assert(NC == 8, "the exchanges below reduce eight columns");
+    const int c0 = blockIdx.y * kColGrp + wave;  // columns c0 + 4 u
+    double s[NC], z[NC][4];
+#pragma unroll
+    for (int u = 0; u < NC; ++u) {
+        const double* zc = Z + (size_t)min(c0 + 4 * u, k - 1) * ldz;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) z[u][i] = zc[min(r0 + 64 * i, n - 1)];
+    }
+#pragma unroll
+    for (int u = 0; u < NC; ++u) {
+        s[u] = 0.0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[u] += (r0 + 64 * i < n ? z[u][i] : 0.0) * xv[i];
+    }
+    int u = 0;  // column of s[0] after the exchanges
+#pragma unroll
+    for (int o = 32, m = NC / 2; m > 0; o >>= 1, m >>= 1) {
+        const bool up = (lane & o) != 0;
+        u += up ? m : 0;
+#pragma unroll
+        for (int e = 0; e < NC / 2; ++e)
+            if (e < m) {
+                const double mine = up ? s[e + m] : s[e], other = up ? s[e] : s[e + m];
+                s[e] = mine + __shfl_xor(other, o);
+            }
+    }
+#pragma unroll
+    for (int o = 4; o > 0; o >>= 1) s[0] += __shfl_xor(s[0], o);
+    const int c = c0 + 4 * u;
+    if ((lane & 7) == 0 && c < k) part[(size_t)c * nchunks + chunk] = s[0];
+}
 
 __global__ __launch_bounds__(256) void ztx_partial_kernel(int n, int k, const double* __restrict__ Z,
                                                           int ldz, const double* __restrict__ x,
-                                                          double* __restrict__ part,
-                                                          const double* __restrict__ ctl) {
-    if (cg_stopped(ctl)) return;
-    const int chunk = blockIdx.x, nchunks = gridDim.x;
-    const int r0 = chunk * kRows;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+                                                          double* __restrict__ part) {
+    const int r0 = blockIdx.x * kRows + (threadIdx.x & 63);
+    double xv[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) xv[i] = r0 + 64 * i < n ? x[r0 + 64 * i] : 0.0;
+    ztx_columns(n, k, Z, ldz, xv, part);
+}
+
+// The start of a CG iteration: ends the one before it (state `in` -> `out`,
+// beta = (r.z)_new / (r.z), p = z + beta p_old), then Z^T p by chunks.  Every
+// workgroup of a chunk forms the chunk's p; those of column group 0 store it.
+// FIRST: the state and p are those of `in` and `p_old` (out and p_new unused).
+template <bool FIRST>
+__global__ __launch_bounds__(256) void cg_begin_kernel(
+    int n, int k, const double* __restrict__ Z, int ldz, int nblk,
+    const double* __restrict__ part2, const double* __restrict__ z,
+    const double* __restrict__ p_old, double* __restrict__ p_new, double* __restrict__ part,
+    const CgState* __restrict__ in, CgState* __restrict__ out, double tol, int max_iter) {
+    CgState old = *in, st = old;
+    const bool lead = blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0;
+    if (!FIRST) {
+        if (old.active != 0.0) st = cg_next(old, nblk, part2, tol, max_iter);
+        if (lead) *out = st;
+    }
+    if (st.active == 0.0) return;
+    const int r0 = blockIdx.x * kRows + (threadIdx.x & 63);
+    const double beta = FIRST ? 0.0 : st.rz / old.rz;
     double xv[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int r = r0 + lane + 64 * i;
-        xv[i] = r < n ? x[r] : 0.0;
-    }
-    const int c0 = blockIdx.y * kColGrp;
-    for (int cc = wave; cc < kColGrp; cc += 4) {
-        const int c = c0 + cc;
-        if (c >= k) break;
-        const double* z = Z + (size_t)c * ldz;
-        double s = 0.0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int r = r0 + lane + 64 * i;
-            if (r < n) s += z[r] * xv[i];
+        const int r = r0 + 64 * i;
+        xv[i] = 0.0;
+        if (r < n) {
+            xv[i] = FIRST ? p_old[r] : z[r] + beta * p_old[r];
+            if (!FIRST && blockIdx.y == 0 && (threadIdx.x >> 6) == i) p_new[r] = xv[i];
         }
-        s = wave_sum(s);
-        if (lane == 0) part[(size_t)c * nchunks + chunk] = s;
     }
+    ztx_columns(n, k, Z, ldz, xv, part);
+}
+
+// The end of a batch: as cg_begin_kernel without the product, so that the host
+// can read the state.
+__global__ __launch_bounds__(256) void cg_end_kernel(int n, int nblk,
+                                                     const double* __restrict__ part2,
+                                                     const double* __restrict__ z,
+                                                     const double* __restrict__ p_old,
+                                                     double* __restrict__ p_new,
+                                                     const CgState* __restrict__ in,
+                                                     CgState* __restrict__ out, double tol,
+                                                     int max_iter) {
+    CgState old = *in, st = old;
+    if (old.active != 0.0) st = cg_next(old, nblk, part2, tol, max_iter);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *out = st;
+    if (st.active == 0.0) return;
+    const double beta = st.rz / old.rz;
+    const int i = blockIdx.x * kRows + threadIdx.x;
+    if (i < n) p_new[i] = z[i] + beta * p_old[i];
 }
 
 // out[c] = sum over chunks of part[c * nchunks + chunk]; one wave per column.
 __global__ __launch_bounds__(256) void reduce_cols_kernel(int nchunks, int k,
                                                           const double* __restrict__ part,
                                                           double* __restrict__ out,
-                                                          const double* __restrict__ ctl) {
-    if (cg_stopped(ctl)) return;
+                                                          const CgState* __restrict__ st) {
+    if (cg_stopped(st)) return;
     const int c = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (c >= k) return;
     const double* p = part + (size_t)c * nchunks;
@@ -220,36 +312,56 @@ __global__ __launch_bounds__(256) void setup_reduce_kernel(int nblk, const doubl
     }
 }
 
-// q = Z v + D o p; part[b] = p.q over the workgroup's rows.
-__global__ __launch_bounds__(256) void cg_apply_kernel(int n, int k, const double* __restrict__ Z,
-                                                       int ldz, const double* __restrict__ v,
-                                                       const double* __restrict__ D,
-                                                       const double* __restrict__ p,
-                                                       double* __restrict__ q,
-                                                       double* __restrict__ part,
-                                                       const double* __restrict__ ctl) {
-    if (cg_stopped(ctl)) return;
-    __shared__ double su[kMaxK];
-    __shared__ double sh[4];
-    for (int c = threadIdx.x; c < k; c += 256) su[c] = v[c];
+// q = Z v + D o p; part[w] = p.q over the 64 rows of wave w.  One wave per
+// workgroup and row block, so that n rows spread over n / 64 CUs, with the next
+// kApplyCols columns of Z in flight while these are added up; each row's sum
+// runs over the columns in order, as one thread's chain.
+constexpr int kApplyCols = 64;
+
+__global__ __launch_bounds__(64) void cg_apply_kernel(int n, int k, const double* __restrict__ Z,
+                                                      int ldz, const double* __restrict__ v,
+                                                      const double* __restrict__ D,
+                                                      const double* __restrict__ p,
+                                                      double* __restrict__ q,
+                                                      double* __restrict__ part,
+                                                      const CgState* __restrict__ st) {
+    if (cg_stopped(st)) return;
+    __shared__ double su[kMaxK];  // v, zero-padded to a whole number of panels
+    const int i = blockIdx.x * 64 + threadIdx.x, ic = min(i, n - 1);
+    const double* zr = Z + ic;
+    double cur[kApplyCols], nxt[kApplyCols];
+#pragma unroll
+    for (int u = 0; u < kApplyCols; ++u) cur[u] = zr[(size_t)min(u, k - 1) * ldz];
+    for (int c = threadIdx.x; c < (k + kApplyCols - 1) / kApplyCols * kApplyCols; c += 64)
+        su[c] = c < k ? v[c] : 0.0;
+    const double di = D[ic], pi = p[ic];
     __syncthreads();
-    const int i = blockIdx.x * kRows + threadIdx.x;
-    const double zv = z_row_dot(i, n, k, Z, ldz, su);
+    double zv = 0.0;
+    for (int c0 = 0; c0 < k; c0 += kApplyCols) {
+        if (c0 + kApplyCols < k) {
+#pragma unroll
+            for (int u = 0; u < kApplyCols; ++u)
+                nxt[u] = zr[(size_t)min(c0 + kApplyCols + u, k - 1) * ldz];
+        }
+#pragma unroll
+        for (int u = 0; u < kApplyCols; ++u) zv += cur[u] * su[c0 + u];
+#pragma unroll
+        for (int u = 0; u < kApplyCols; ++u) cur[u] = nxt[u];
+    }
     double pq = 0.0;
     if (i < n) {
-        const double qi = zv + D[i] * p[i];
+        const double qi = zv + di * pi;
         q[i] = qi;
-        pq = p[i] * qi;
+        pq = pi * qi;
     }
-    const double s = block_sum(pq, sh);
-    if (threadIdx.x == 0) part[blockIdx.x] = s;
+    pq = wave_sum(pq);
+    if (threadIdx.x == 0) part[blockIdx.x] = pq;
 }
 
-// alpha = r.z / p.q (p.q summed from the partials in a fixed order by every
-// workgroup); s += alpha p, r -= alpha q, z = r / Pc; part2[2b..] = (r.z, r.r).
+// alpha = r.z / p.q (p.q summed from the waves' partials in a fixed order by
+// every workgroup); s += alpha p, r -= alpha q, z = r / Pc; part2[2b..] = (r.z, r.r).
 __global__ __launch_bounds__(256) void cg_update_kernel(int n, int nblk,
                                                         const double* __restrict__ part_pq,
-                                                        const double* __restrict__ sc,
                                                         const double* __restrict__ p,
                                                         const double* __restrict__ q,
                                                         const double* __restrict__ Pc,
@@ -257,17 +369,28 @@ __global__ __launch_bounds__(256) void cg_update_kernel(int n, int nblk,
                                                         double* __restrict__ r,
                                                         double* __restrict__ z,
                                                         double* __restrict__ part2,
-                                                        const double* __restrict__ ctl) {
-    if (cg_stopped(ctl)) return;
+                                                        const CgState* __restrict__ st) {
+    if (cg_stopped(st)) return;
     __shared__ double sh[4];
-    const double pq = fixed_sum(nblk, part_pq, sh);
-    const double alpha = sc[0] / pq;
-    const int i = blockIdx.x * kRows + threadIdx.x;
+    const int i = blockIdx.x * kRows + threadIdx.x, ic = min(i, n - 1);
+    const double pi = p[ic], qi = q[ic], pc = Pc[ic], si = s[ic], r0 = r[ic];
+    double v = 0.0;
+    for (int b = threadIdx.x; b < nblk; b += 256) {
+        const double* w = part_pq + 4 * (size_t)b;
+        v += (w[0] + w[1]) + (w[2] + w[3]);
+    }
+    v = wave_sum(v);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (lane == 0) sh[wave] = v;
+    __syncthreads();
+    const double pq = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+    __syncthreads();  // sh is reused below
+    const double alpha = st->rz / pq;
     double rz = 0.0, rr = 0.0;
     if (i < n) {
-        s[i] += alpha * p[i];
-        const double ri = r[i] - alpha * q[i];
-        const double zi = ri / Pc[i];
+        s[i] = si + alpha * pi;
+        const double ri = r0 - alpha * qi;
+        const double zi = ri / pc;
         r[i] = ri;
         z[i] = zi;
         rz = ri * zi;
@@ -281,64 +404,9 @@ __global__ __launch_bounds__(256) void cg_update_kernel(int n, int nblk,
     }
 }
 
-// beta = (r.z)_new / (r.z); p = z + beta p.  Every workgroup reads the old
-// r.z from sc, so the new r.z and r.r go to sc_next and a separate launch
-// (cg_commit_kernel) moves them into sc.
-__global__ __launch_bounds__(256) void cg_direction_kernel(int n, int nblk,
-                                                           const double* __restrict__ part2,
-                                                           const double* __restrict__ sc,
-                                                           const double* __restrict__ z,
-                                                           double* __restrict__ p,
-                                                           double* __restrict__ sc_next,
-                                                           const double* __restrict__ ctl) {
-    if (cg_stopped(ctl)) return;
-    __shared__ double sh[4];
-    double v0 = 0.0, v1 = 0.0;
-    for (int b = threadIdx.x; b < nblk; b += 256) {
-        v0 += part2[2 * b];
-        v1 += part2[2 * b + 1];
-    }
-    v0 = wave_sum(v0);
-    v1 = wave_sum(v1);
-    __shared__ double sh1[4];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane == 0) {
-        sh[wave] = v0;
-        sh1[wave] = v1;
-    }
-    __syncthreads();
-    const double rz_new = (sh[0] + sh[1]) + (sh[2] + sh[3]);
-    const double rr_new = (sh1[0] + sh1[1]) + (sh1[2] + sh1[3]);
-    const double beta = rz_new / sc[0];
-    const int i = blockIdx.x * kRows + threadIdx.x;
-    if (i < n) p[i] = z[i] + beta * p[i];
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        sc_next[0] = rz_new;
-        sc_next[1] = rr_new;
-    }
-}
-
-// End of an iteration: sc[0..1] = sc_next[0..1] (the next iteration's r.z and
-// the residual norm), one more iteration counted in ctl[1], and the stopping
-// test of the loop, sqrt(r.r) <= tol or max_iter iterations, into ctl[0];
-// ctl[2] = r.r for the host.
-__global__ void cg_commit_kernel(double* __restrict__ sc, const double* __restrict__ sc_next,
-                                 double* __restrict__ ctl, double tol, int max_iter) {
-    if (threadIdx.x == 0 && ctl[0] != 0.0) {
-        sc[0] = sc_next[0];
-        sc[1] = sc_next[1];
-        ctl[1] += 1.0;
-        ctl[2] = sc[1];
-        ctl[0] = (sqrt(sc[1]) > tol && ctl[1] < (double)max_iter) ? 1.0 : 0.0;
-    }
-}
-
-// Loop start: active, no iterations yet.
-__global__ void cg_start_kernel(double* __restrict__ ctl) {
-    if (threadIdx.x == 0) {
-        ctl[0] = 1.0;
-        ctl[1] = 0.0;
-    }
+// Loop start: active, no iterations yet, r.z and r.r from the setup's scalars.
+__global__ void cg_start_kernel(CgState* __restrict__ st, const double* __restrict__ sc) {
+    if (threadIdx.x == 0) *st = CgState{1.0, 0.0, sc[1], sc[0]};
 }
 
 // Line-search sums per workgroup: part[b * W + j] for j = 0: grad.s,
@@ -432,13 +500,16 @@ __global__ __launch_bounds__(256) void svm_init_kernel(int n, int k, const doubl
 
 struct Work {
     int n, k, nblk, nchunks, ngrp;
-    double *a, *M, *grad, *D, *Pc, *s, *r, *z, *p, *q;
+    double *a, *M, *grad, *D, *Pc, *s, *r, *z, *p, *p2, *q;  // p, p2: in turn
     double *u, *v;              // k-vectors
     double *part, *part2;       // per-workgroup partials
     double *ztpart;             // nchunks x k partials of Z^T x
-    double *sc, *sc_next, *ls;  // device scalars
-    double* ctl;                // CG loop control: active flag, iterations, r.r
+    double *sc, *ls;            // device scalars
+    CgState* st;                // two banks of kCgBatch + 1 states of the CG loop
 };
+
+// Iterations queued between two reads of the CG loop's state.
+constexpr int kCgBatch = 8;
 
 int grab(dh_handle_t h, int n, int k, Work& w) {
     w.n = n;
@@ -447,8 +518,9 @@ int grab(dh_handle_t h, int n, int k, Work& w) {
     w.nchunks = w.nblk;
     w.ngrp = dh_cdiv(k, kColGrp);
     const size_t nn = (size_t)std::max(n, 1);
-    const size_t doubles = 10 * nn + 2 * (size_t)k + (size_t)w.nblk * (kLsW + 4) +
-                           2 * (size_t)w.nblk + (size_t)w.nchunks * k + 80 + kLsW + 8;
+    const size_t doubles = 11 * nn + 2 * (size_t)k + (size_t)w.nblk * (kLsW + 4) +
+                           2 * (size_t)w.nblk + (size_t)w.nchunks * k + 16 + kLsW + 8 + 32 +
+                           2 * (kCgBatch + 1) * 4;
     double* base = (double*)dh_ws(h, DH_WS_SVM, sizeof(double) * doubles);
     if (!base) return DH_ERR_ALLOC;
     double* x = base;
@@ -466,6 +538,7 @@ int grab(dh_handle_t h, int n, int k, Work& w) {
     w.r = take(nn);
     w.z = take(nn);
     w.p = take(nn);
+    w.p2 = take(nn);
     w.q = take(nn);
     w.u = take(k);
     w.v = take(k);
@@ -473,21 +546,18 @@ int grab(dh_handle_t h, int n, int k, Work& w) {
     w.part2 = take(2 * (size_t)w.nblk);
     w.ztpart = take((size_t)w.nchunks * k);
     w.sc = take(16);
-    w.sc_next = take(16);
     w.ls = take(kLsW + 8 + 32);
-    w.ctl = take(16);
+    w.st = (CgState*)take(2 * (kCgBatch + 1) * 4);
     return 0;
 }
 
-// out (k) = Z^T x (skipped once the CG loop controlled by ctl has stopped;
-// ctl = NULL: always).
-int zt(dh_handle_t h, const Work& w, const double* Z, int ldz, const double* x, double* out,
-       const double* ctl = nullptr) {
+// out (k) = Z^T x.
+int zt(dh_handle_t h, const Work& w, const double* Z, int ldz, const double* x, double* out) {
     ztx_partial_kernel<<<dim3(w.nchunks, w.ngrp), 256, 0, h->stream>>>(w.n, w.k, Z, ldz, x,
-                                                                       w.ztpart, ctl);
+                                                                       w.ztpart);
     DH_CHECK_LAUNCH();
     reduce_cols_kernel<<<dh_cdiv(w.k, 4), 256, 0, h->stream>>>(w.nchunks, w.k, w.ztpart, out,
-                                                               ctl);
+                                                               nullptr);
     DH_CHECK_LAUNCH();
     return 0;
 }
@@ -501,43 +571,57 @@ int read_scalars(dh_handle_t h, const double* dev, double* host, int count) {
     return 0;
 }
 
-// Iterations queued between two reads of the CG loop's control words.
-constexpr int kCgBatch = 8;
-
 // Preconditioned CG from the state left by newton_setup_kernel (or
 // pcg_setup): iterates until sqrt(r.r) <= tol or max_iter.  The test runs on
-// the device at the end of every iteration (cg_commit_kernel); iterations
-// queued after it fails do nothing.
+// the device at the end of every iteration (cg_next); iterations queued after
+// it fails do nothing.  Iteration b of a batch has state b of the batch's
+// bank; the batch's end goes to state 0 of the other bank.
 int cg_loop(dh_handle_t h, const Work& w, const double* Z, int ldz, double tol, int max_iter,
             int* iters, double* rnorm) {
     double rr = 0.0;
     DH_CHECK_STATUS(read_scalars(h, w.sc + 1, &rr, 1));
     int it = 0;
     if (std::sqrt(rr) > tol && it < max_iter) {
-        cg_start_kernel<<<1, 64, 0, h->stream>>>(w.ctl);
+        CgState *bank = w.st, *other = w.st + kCgBatch + 1;
+        double *p = w.p, *pn = w.p2;
+        cg_start_kernel<<<1, 64, 0, h->stream>>>(bank, w.sc);
         DH_CHECK_LAUNCH();
+        const dim3 grid(w.nchunks, w.ngrp);
         for (;;) {
             const int batch = std::min(kCgBatch, max_iter - it);
             for (int b = 0; b < batch; ++b) {
-                DH_CHECK_STATUS(zt(h, w, Z, ldz, w.p, w.v, w.ctl));
-                cg_apply_kernel<<<w.nblk, 256, 0, h->stream>>>(w.n, w.k, Z, ldz, w.v, w.D, w.p,
-                                                                w.q, w.part, w.ctl);
+                CgState* st = bank + b;
+                if (b == 0) {
+                    cg_begin_kernel<true><<<grid, 256, 0, h->stream>>>(
+                        w.n, w.k, Z, ldz, w.nblk, w.part2, w.z, p, nullptr, w.ztpart, st, nullptr,
+                        tol, max_iter);
+                } else {
+                    cg_begin_kernel<false><<<grid, 256, 0, h->stream>>>(
+                        w.n, w.k, Z, ldz, w.nblk, w.part2, w.z, p, pn, w.ztpart, st - 1, st, tol,
+                        max_iter);
+                    std::swap(p, pn);
+                }
                 DH_CHECK_LAUNCH();
-                cg_update_kernel<<<w.nblk, 256, 0, h->stream>>>(w.n, w.nblk, w.part, w.sc, w.p,
-                                                                 w.q, w.Pc, w.s, w.r, w.z,
-                                                                 w.part2, w.ctl);
+                reduce_cols_kernel<<<dh_cdiv(w.k, 4), 256, 0, h->stream>>>(w.nchunks, w.k,
+                                                                           w.ztpart, w.v, st);
                 DH_CHECK_LAUNCH();
-                cg_direction_kernel<<<w.nblk, 256, 0, h->stream>>>(w.n, w.nblk, w.part2, w.sc,
-                                                                    w.z, w.p, w.sc_next, w.ctl);
+                cg_apply_kernel<<<4 * w.nblk, 64, 0, h->stream>>>(w.n, w.k, Z, ldz, w.v, w.D, p,
+                                                                  w.q, w.part, st);
                 DH_CHECK_LAUNCH();
-                cg_commit_kernel<<<1, 64, 0, h->stream>>>(w.sc, w.sc_next, w.ctl, tol, max_iter);
+                cg_update_kernel<<<w.nblk, 256, 0, h->stream>>>(w.n, w.nblk, w.part, p, w.q, w.Pc,
+                                                                w.s, w.r, w.z, w.part2, st);
                 DH_CHECK_LAUNCH();
             }
-            double c[3];
-            DH_CHECK_STATUS(read_scalars(h, w.ctl, c, 3));
-            it = (int)c[1];
-            rr = c[2];
-            if (c[0] == 0.0) break;
+            cg_end_kernel<<<w.nblk, 256, 0, h->stream>>>(w.n, w.nblk, w.part2, w.z, p, pn,
+                                                         bank + batch - 1, other, tol, max_iter);
+            DH_CHECK_LAUNCH();
+            std::swap(p, pn);
+            std::swap(bank, other);
+            CgState c;
+            DH_CHECK_STATUS(read_scalars(h, (const double*)bank, (double*)&c, 4));
+            it = (int)c.iters;
+            rr = c.rr;
+            if (c.active == 0.0) break;
         }
     }
     if (iters) *iters = it;
