@@ -8,9 +8,12 @@
 //
 // One template serves both precisions: the f64 and f32 16x16x4 MFMAs share
 // an operand layout (mfma_tile.h).
+#include <algorithm>
 #include <cstdio>
 
+#include "chol16.h"
 #include "dh_common.h"
+#include "lds_dma.h"
 #include "mfma_tile.h"
 
 // ------------------------------------------------------------------ GEMM
@@ -186,6 +189,205 @@ template int dh_gemm_impl<double>(dh_handle_t, bool, bool, int, int, int, double
 template int dh_gemm_impl<float>(dh_handle_t, bool, bool, int, int, int, float, const float*,
                                  int, const float*, int, float, float*, int, int);
 
+// ------------------------------------------------- trailing update
+//
+// C (m x n, rows i <= columns j only) -= A^T B, A (k x m) and B (k x n) with
+// contiguous k: the blocked Cholesky's rank-k update.  128 x 128 tiles by 8
+// waves of 32 x 64; both operands go to LDS by direct copies, 128 bytes of k
+// per column and stage, three stages deep, so the copies of two stages are in
+// flight while one is multiplied and one barrier per stage orders them.  The
+// stages of consecutive tiles follow each other without a gap.  The 16-byte
+// pieces of column i lie at position p ^ ((i / 2) % 8) of its 128 bytes: the copies keep
+// their lane order, and the 16 lanes of a quarter-wave read cover all 64 banks.
+// Lane group g takes pieces 2g and 2g + 1 of both operands as the k-slot g of
+// consecutive MFMAs.  The product is formed transposed (D = B^T A), so that 16
+// lanes hold 16 consecutive rows of C.
+//
+// The workgroups are persistent, one per CU (96 KB of LDS), and each XCD
+// takes a contiguous range of tiles, column by column (they share B, and A from
+// the same L2).  On the look-ahead stream eight CUs are left out, one per XCD:
+// the panel factorisation beside it is one workgroup of dependent FP64
+// operations, and an FP64 MFMA of another wave on its SIMD holds the datapath for
+// 64 cycles against the 8 of an FMA.  Its 87 KB of LDS fit only on a CU that this
+// kernel does not use (22 us per 64 x 64 block instead of 107).
+// A16: 16-byte copies (operands and leading dimensions aligned to 16 bytes);
+// otherwise 4-byte ones.
+template <typename T, bool A16>
+__global__ __launch_bounds__(512) void update_tn_kernel(int m, int n, int k, const T* A, int lda,
+                                                        const T* B, int ldb, T* C, int ldc,
+                                                        int ntiles, const int* stop) {
+    constexpr int KS = 128 / sizeof(T), VE = 16 / sizeof(T);
+    constexpr int NI = A16 ? 2 : 8;  // copies per wave, operand and stage
+    __shared__ __align__(128) char ring[3][2][128 * 128];
+    if (*stop != 0) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, li = lane & 15;
+    const int wi = wave & 3, wj = wave >> 2;
+    const int uwi = __builtin_amdgcn_readfirstlane(wi), uwj = __builtin_amdgcn_readfirstlane(wj);
+    const int rs = Mfma<T>::row(0, 1);
+    const unsigned co = (unsigned)li + (unsigned)Mfma<T>::row(g, 0) * (unsigned)ldc;
+    const int tm = (m + 127) / 128, nst = k / KS;
+    // This workgroup's tiles: XCD x has [first, last), dealt to its workgroups.
+    const int x = blockIdx.x & 7, per = ntiles / 8, rem = ntiles % 8;
+    int tile = x * per + min(x, rem);
+    const int last = tile + per + (x < rem ? 1 : 0), step = gridDim.x >> 3;
+    tile += blockIdx.x >> 3;
+    if (tile >= last) return;
+    struct Origin {
+        int m0, n0;
+    };
+    auto origin = [&](int t) {
+        int bi, bj;
+        const int tri = tm * (tm + 1) / 2;  // columns 0 .. tm-1 hold 1 .. tm tiles
+        if (t < tri) {
+            bj = (int)((sqrtf(8.0f * (float)t + 1.0f) - 1.0f) * 0.5f);
+            while ((bj + 1) * (bj + 2) / 2 <= t) ++bj;
+            while (bj * (bj + 1) / 2 > t) --bj;
+            bi = t - bj * (bj + 1) / 2;
+        } else {
+            bj = tm + (t - tri) / tm;
+            bi = (t - tri) % tm;
+        }
+        return Origin{__builtin_amdgcn_readfirstlane(bi * 128),
+                      __builtin_amdgcn_readfirstlane(bj * 128)};
+    };
+    // The copies run two stages ahead: stage fst of the tile at f, into slot fsl.
+    int ftile = tile, fst = 0, fsl = 0;
+    Origin f = origin(tile);
+    unsigned va[NI], vb[NI];  // byte offsets of this lane's pieces from column m0 / n0
+    auto offsets = [&]() {
+#pragma unroll
+        for (int u = 0; u < NI; ++u) {
+            const int q = 8 * u + wave;
+            const int row = A16 ? 8 * q + (lane >> 3) : 2 * q + (lane >> 5);
+            const int p = A16 ? lane & 7 : (lane & 31) >> 2, e = A16 ? 0 : (lane & 3) * 4;
+            const unsigned o = (unsigned)((p ^ ((row >> 1) & 7)) * 16 + e);
+            va[u] = (unsigned)(min(f.m0 + row, m - 1) - f.m0) * (unsigned)(lda * sizeof(T)) + o;
+            vb[u] = (unsigned)(min(f.n0 + row, n - 1) - f.n0) * (unsigned)(ldb * sizeof(T)) + o;
+        }
+    };
+    auto issue = [&]() {  // nothing once the last tile's stages are under way
+        if (ftile >= last) return false;
+        const T* a = A + (size_t)f.m0 * lda + fst * KS;
+        const T* b = B + (size_t)f.n0 * ldb + fst * KS;
+        char* la = ring[fsl][0];
+        char* lb = ring[fsl][1];
+#pragma unroll
+        for (int u = 0; u < NI; ++u) {
+            const int q = 8 * u + wave;
+            if constexpr (A16) {
+                dma16(a, va[u], la + 1024 * q);
+                dma16(b, vb[u], lb + 1024 * q);
+            } else {
+                dma4(a, va[u], la + 256 * q);
+                dma4(b, vb[u], lb + 256 * q);
+            }
+        }
+        fsl = fsl == 2 ? 0 : fsl + 1;
+        if (++fst == nst) {
+            fst = 0;
+            ftile += step;
+            if (ftile < last) {
+                f = origin(ftile);
+                offsets();
+            }
+        }
+        return true;
+    };
+    typedef T vec __attribute__((ext_vector_type(16 / sizeof(T))));
+    const int off0 = ((2 * g) ^ (li >> 1)) * 16, off1 = ((2 * g + 1) ^ (li >> 1)) * 16;
+    offsets();
+    issue();
+    bool ahead = issue();  // a stage after the one to be waited for is under way
+    int slot = 0;
+    for (; tile < last; tile += step) {
+        const Origin o = origin(tile);
+        const int i0 = o.m0 + wi * 32 + li, j0 = o.n0 + wj * 64;
+        // C element (cj, ci, r): uniform address + the lane's 32-bit offset.
+        T* cu = C + (o.m0 + uwi * 32) + (size_t)(o.n0 + uwj * 64) * ldc;
+        typename Mfma<T>::acc_t acc[4][2];
+        zero_acc<T, 4, 2>(acc);
+        for (int st = 0; st < nst; ++st) {
+            // The newest 2 NI copies (the stage after this one) may stay in flight.
+            if (ahead)
+                __builtin_amdgcn_s_waitcnt(A16 ? 0x0F74 : 0x4F70);  // vmcnt(4) / vmcnt(16)
+            else
+                wait_vm();
+            __syncthreads();
+            ahead = issue();
+            const char* la = ring[slot][0] + (wi * 32 + li) * 128;
+            const char* lb = ring[slot][1] + (wj * 64 + li) * 128;
+            slot = slot == 2 ? 0 : slot + 1;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int off = h ? off1 : off0;
+                vec av[2], bv[4];
+#pragma unroll
+                for (int c = 0; c < 2; ++c) av[c] = *(const vec*)(la + c * 2048 + off);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) bv[c] = *(const vec*)(lb + c * 2048 + off);
+#pragma unroll
+                for (int e = 0; e < VE; ++e)
+#pragma unroll
+                    for (int cj = 0; cj < 4; ++cj)
+#pragma unroll
+                        for (int ci = 0; ci < 2; ++ci)
+                            acc[cj][ci] = Mfma<T>::op(bv[cj][e], av[ci][e], acc[cj][ci]);
+            }
+        }
+        T cv[4][2][4];  // every load of C before the first store
+#pragma unroll
+        for (int cj = 0; cj < 4; ++cj)
+#pragma unroll
+            for (int ci = 0; ci < 2; ++ci)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int i = i0 + 16 * ci, j = j0 + 16 * cj + Mfma<T>::row(g, r);
+                    cv[cj][ci][r] = T(0);
+                    if (i < m && j < n && i <= j)
+                        cv[cj][ci][r] = (cu + 16 * ci + (size_t)(16 * cj + rs * r) * ldc)[co];
+                }
+        // One wait for all: with loads the compiler takes to be pending in some
+        // path, it would put this wait between the copies and the products.
+        wait_vm();
+#pragma unroll
+        for (int cj = 0; cj < 4; ++cj)
+#pragma unroll
+            for (int ci = 0; ci < 2; ++ci)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int i = i0 + 16 * ci, j = j0 + 16 * cj + Mfma<T>::row(g, r);
+                    if (i < m && j < n && i <= j)
+                        (cu + 16 * ci + (size_t)(16 * cj + rs * r) * ldc)[co] =
+                            cv[cj][ci][r] - acc[cj][ci][r];
+                }
+    }
+}
+
+// Upper part of C (m x n, m <= n) -= A^T B (k deep) on h->stream.  128 x 128 tiles
+// need about half a tile per CU to win over the 64 x 64 GEMM, four of which
+// share a CU; the copies need k to be whole stages and 32-bit offsets.
+template <typename T>
+static int trailing_update(dh_handle_t h, int m, int n, int k, const T* A, int lda, const T* B,
+                           int ldb, T* C, int ldc, const int* stop) {
+    const int tm = dh_cdiv(m, 128), tn = dh_cdiv(n, 128);
+    const long tiles = (long)tm * (tm + 1) / 2 + (long)(tn - tm) * tm;
+    const size_t col = sizeof(T) * (size_t)std::max(lda, ldb);
+    if (2 * tiles < h->num_cu || k % (128 / (int)sizeof(T)) != 0 || col * 128 >= (1ull << 32))
+        return gemm_stop<T>(h, true, false, m, n, k, T(-1), A, lda, B, ldb, T(1), C, ldc, 1, stop);
+    const int spare = h->stream == h->aux ? 8 : 0;
+    const int grid = (int)std::min<long>((tiles + 7) / 8 * 8, std::max(8, h->num_cu / 8 * 8 - spare));
+    const bool a16 = ((uintptr_t)A | (uintptr_t)B | (sizeof(T) * (size_t)lda) |
+                      (sizeof(T) * (size_t)ldb)) % 16 == 0;
+    if (a16)
+        update_tn_kernel<T, true><<<grid, 512, 0, h->stream>>>(m, n, k, A, lda, B, ldb, C, ldc,
+                                                               (int)tiles, stop);
+    else
+        update_tn_kernel<T, false><<<grid, 512, 0, h->stream>>>(m, n, k, A, lda, B, ldb, C, ldc,
+                                                                (int)tiles, stop);
+    DH_CHECK_LAUNCH();
+    return 0;
+}
+
 // ------------------------------------------------------ small triangles
 
 constexpr int kSmall = 64;
@@ -197,84 +399,283 @@ constexpr int kSmall = 64;
 //   U^{-T} B = Linv B,   U^{-1} B = Linv^T B,   B U^{-1} = B Linv^T.
 
 // Cholesky of the nb <= 64 diagonal block at A (upper triangle, in place)
-// together with Linv.  Symmetric Gaussian elimination on [A | I]: step k
-// subtracts m_i = A(k,i) / A(k,k) times row k from every row i > k, so the
-// left part ends as D Ut (Ut unit upper, A = Ut^T D Ut) and the right part
-// as Ut^{-T}; then U = D^{1/2} Ut and U^{-T} = D^{-1/2} Ut^{-T}.  Both parts
-// share one 64 x 64 register grid over kPotrfThreads threads (NW waves):
-// thread t holds row i = t % 64 at columns j = t / 64 + NW q (q < E = 64/NW),
-// the left part where j >= i and the strictly lower right part where j < i.
-// Row k is broadcast through LDS (double buffered: one barrier per step).
-// The step is a latency chain (write, barrier, read, divide, update), so
-// 512 threads -- 8 values each -- beat 256 with 16 (about 1300 against 1800
-// cycles per step).  A non-positive (or NaN) pivot at local step k stores
-// base + k + 1 in *info (first failure wins) and leaves A as it was.
-constexpr int kPotrfThreads = 512;
+// together with Linv, after the rows of U above it in its panel (`depth` of
+// them, a multiple of 64, straight above A) have been subtracted:
+// A -= P^T P, P the depth x nb block of U.  All arithmetic is FP64, also for
+// T = float.
+//
+// The block is factored in four 16-column steps on [A | I], both parts in LDS:
+// per step wave 0 factors the 16 x 16 diagonal block (chol16) and inverts it;
+// then the four blocks of the row -- those of A right of the diagonal and
+// those of the inverse left of it, four together in every step -- are multiplied
+// by its inverse transpose, one per wave; then wave 0 updates the next
+// diagonal block and goes on with it while the others update the rest.  It is
+// a latency chain on one CU: four chol16 and inversions bound it.
+// A non-positive (or NaN) pivot at local step k stores base + k + 1 in *info
+// (first failure wins) and leaves A as it was.
 template <typename T>
-__global__ __launch_bounds__(kPotrfThreads) void potrf_inv_small_kernel(int nb,
-                                                                         T* __restrict__ A,
-                                                                         int lda,
-                                                                         T* __restrict__ Linv,
-                                                                         int* __restrict__ info,
-                                                                         int base) {
-    constexpr int NW = kPotrfThreads / 64, E = kSmall / NW;
-    // Row k is broadcast permuted, column j at (j % NW) * E + j / NW, so the
-    // E columns a thread holds are contiguous (vector LDS reads/writes).
-    __shared__ T rows[2][kSmall];
-    __shared__ T diag[kSmall];
-    if (*info != 0) return;
-    const int t = threadIdx.x, i = t & (kSmall - 1), w = t >> 6;
-    const int pi = (i % NW) * E + i / NW;
-    T a[E];
+__global__ __launch_bounds__(256) void potrf64_kernel(int nb, int depth, T* __restrict__ A,
+                                                      int lda, T* __restrict__ Linv,
+                                                      int* __restrict__ info, int base) {
+    constexpr int P = 81;  // odd pitch: the column-wise loads and stores spread over the banks
+    __shared__ double sA[kSmall][P], sR[kSmall][P];
+    __shared__ double sU[16][16], sI[16][17], sRd[16];
+    __shared__ int s_bad;
+    const int stopped = *info;  // tested once the operands are on their way
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, li = lane & 15;
+    T av[16];
 #pragma unroll
-    for (int q = 0; q < E; ++q) {
-        const int j = w + NW * q;
-        a[q] = (i < nb && j < nb) ? (i <= j ? A[i + (size_t)j * lda] : T(0))
-                                  : (i == j ? T(1) : T(0));
+    for (int u = 0; u < 16; ++u) {
+        const int e = tid + 256 * u, i = e & 63, j = e >> 6;
+        av[u] = A[min(i, nb - 1) + (size_t)min(j, nb - 1) * lda];
     }
-    int fail = 0;
-    for (int k = 0; k < kSmall; ++k) {
-        T* rb = rows[k & 1];
-        if (i == k) {
+    // P^T P: wave w takes depth steps w, w + 4, ... of 16 rows.  Lane group g
+    // holds rows 4g .. 4g+3 of a step as the k-slot g of four MFMAs.
+    dh_d4 pp[10];
 #pragma unroll
-            for (int q = 0; q < E; ++q) rb[w * E + q] = a[q];
+    for (int b = 0; b < 10; ++b) pp[b] = dh_d4{0, 0, 0, 0};
+    const T* up = A - depth + 4 * g;
+    T nv[4][4];
+    auto load_up = [&](int r0) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                nv[c][q] = up[r0 + q + (size_t)min(16 * c + li, nb - 1) * lda];
+    };
+    if (depth > 0) load_up(16 * wave);
+    if (stopped != 0) return;
+#pragma unroll 1
+    for (int r0 = 16 * wave; r0 < depth; r0 += 64) {
+        double v[4][4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[c][q] = 16 * c + li < nb ? (double)nv[c][q] : 0.0;
+        if (r0 + 64 < depth) load_up(r0 + 64);
+        int b = 0;
+#pragma unroll
+        for (int ci = 0; ci < 4; ++ci)
+#pragma unroll
+            for (int cj = ci; cj < 4; ++cj, ++b)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) pp[b] = Mfma<double>::op(v[ci][q], v[cj][q], pp[b]);
+    }
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        const int e = tid + 256 * u, i = e & 63, j = e >> 6;
+        sA[i][j] = (i <= j && j < nb) ? (double)av[u] : (i == j ? 1.0 : 0.0);
+        sR[i][j] = i == j ? 1.0 : 0.0;
+    }
+    if (tid == 0) s_bad = 0;
+    __syncthreads();
+    for (int w = 0; w < 4 && 16 * w < depth; ++w) {  // fixed order: wave 0 first
+        if (wave == w) {
+            int b = 0;
+#pragma unroll
+            for (int ci = 0; ci < 4; ++ci)
+#pragma unroll
+                for (int cj = ci; cj < 4; ++cj, ++b)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        sA[16 * ci + g + 4 * r][16 * cj + li] -= pp[b][r];
         }
         __syncthreads();
-        // All reads of the step at once; the pivot test comes after the
-        // update (a failed factorisation writes nothing back).
-        const T piv = rb[(k % NW) * E + k / NW];
-        const T rbi = rb[pi];
-        T rj[E];
-#pragma unroll
-        for (int q = 0; q < E; ++q) rj[q] = rb[w * E + q];
-        // Branch-free update (selects keep a[] in place): rows i <= k keep
-        // their values.
-        const T mi = rbi / piv;
-#pragma unroll
-        for (int q = 0; q < E; ++q) {
-            const int j = w + NW * q;
-            const T f = (j >= i || j < k) ? rj[q] : (j == k ? T(1) : T(0));
-            const T upd = a[q] - mi * f;
-            a[q] = (i > k) ? upd : a[q];
-        }
-        if (!(piv > T(0))) {  // the same value in every thread: a uniform exit
-            fail = k + 1;
-            break;
-        }
-        if (t == 0) diag[k] = piv;
     }
-    if (fail) {
-        if (t == 0) atomicCAS(info, 0, base + fail);
-        return;
+    // U_kk and its inverse from block (k, k) in accumulator layout, by wave 0.
+    auto factor_diag = [&](int k, dh_d4 d) {
+        const int bad = chol16(d, g, li, nb - 16 * k, 0.0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            sU[g + 4 * r][li] = d[r];
+            sA[16 * k + g + 4 * r][16 * k + li] = d[r];
+        }
+        {
+            double dg = d[0];
+#pragma unroll
+            for (int r = 1; r < 4; ++r) dg = (li >> 2) == r ? d[r] : dg;
+            if (g == (li & 3)) sRd[li] = 1.0 / dg;
+        }
+        wave_lds_sync();
+        double x[16];  // column li of the inverse, by back substitution
+#pragma unroll
+        for (int i = 15; i >= 0; --i) {
+            double t0 = (i == li) ? 1.0 : 0.0, t1 = 0.0;
+#pragma unroll
+            for (int q = i + 1; q < 16; ++q) {
+                if ((q - i) & 1)
+                    t0 -= sU[i][q] * x[q];
+                else
+                    t1 -= sU[i][q] * x[q];
+            }
+            x[i] = (t0 + t1) * sRd[i];
+        }
+        if (lane < 16)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) sI[li][i] = x[i];
+        if (lane == 0 && bad && !s_bad) s_bad = 16 * k + bad;
+    };
+    // Block (i, j) of X -= (block (k, i) of A)^T (block (k, j) of X).
+    auto updated = [&](const double (*X)[P], int i, int j, int k) {
+        dh_d4 d;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) d[r] = X[16 * i + g + 4 * r][16 * j + li];
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            d = Mfma<double>::op(-sA[16 * k + 4 * s + g][16 * i + li],
+                                 X[16 * k + 4 * s + g][16 * j + li], d);
+        return d;
+    };
+    auto put = [&](double (*X)[P], int i, int j, const dh_d4& d) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) X[16 * i + g + 4 * r][16 * j + li] = d[r];
+    };
+    if (wave == 0) {
+        dh_d4 d;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) d[r] = sA[g + 4 * r][li];
+        factor_diag(0, d);
+    }
+#pragma unroll 1
+    for (int k = 0; k < 4; ++k) {
+        __syncthreads();
+        {  // row k: block k+1+wave of A, or block wave-(3-k) of the inverse
+            double(*X)[P] = wave < 3 - k ? sA : sR;
+            const int j = wave < 3 - k ? k + 1 + wave : wave - (3 - k);
+            dh_d4 acc = {0, 0, 0, 0};
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                acc = Mfma<double>::op(sI[li][4 * s + g], X[16 * k + 4 * s + g][16 * j + li], acc);
+            put(X, k, j, acc);
+        }
+        if (k == 3) break;
+        __syncthreads();
+        if (wave == 0) {
+            factor_diag(k + 1, updated(sA, k + 1, k + 1, k));
+        } else {
+            int t = 1;  // blocks in order, dealt to waves 1, 2, 3
+            for (int i = k + 1; i < 4; ++i) {
+                for (int j = i == k + 1 ? i + 1 : i; j < 4; ++j, t = t == 3 ? 1 : t + 1)
+                    if (t == wave) put(sA, i, j, updated(sA, i, j, k));
+                for (int c = 0; c <= k; ++c, t = t == 3 ? 1 : t + 1)
+                    if (t == wave) put(sR, i, c, updated(sR, i, c, k));
+            }
+        }
     }
     __syncthreads();
-    const T si = sqrt(diag[i]);
+    if (s_bad) {
+        if (tid == 0) atomicCAS(info, 0, base + s_bad);
+        return;
+    }
 #pragma unroll
-    for (int q = 0; q < E; ++q) {
-        const int j = w + NW * q;
-        if (i <= j && j < nb) A[i + (size_t)j * lda] = a[q] / si;
-        // Linv(i, j) = Ut^{-T}(i, j) / sqrt(d_i), unit diagonal of Ut^{-T}.
-        Linv[i + kSmall * j] = (j < i) ? a[q] / si : (j == i ? T(1) / si : T(0));
+    for (int u = 0; u < 16; ++u) {
+        const int e = tid + 256 * u, i = e & 63, j = e >> 6;
+        if (i <= j && j < nb) A[i + (size_t)j * lda] = (T)sA[i][j];
+        Linv[e] = j <= i ? (T)sR[i][j] : T(0);
+    }
+}
+
+// One 64-row block of a panel's row of U, left-looking: for 32 columns per
+// workgroup, C (nb x cols) := Linv (C - P^T V), P the depth x nb rows of U
+// straight above the block's diagonal block at D0, V those straight above C.
+// A wave owns 16 rows x 32 columns; both products take their operands from
+// global memory (L2) in the MFMA layout, lane group g holding depth 4g .. 4g+3
+// of a 16-deep step; the difference goes through LDS once.
+constexpr int kRowCols = 32;
+template <typename T>
+__global__ __launch_bounds__(256) void panel_row_kernel(int nb, int depth, int cols,
+                                                        const T* __restrict__ D0,
+                                                        const T* __restrict__ Linv, T* C, int lda,
+                                                        const int* __restrict__ stop) {
+    __shared__ T sT[kRowCols][kSmall + 2];
+    const int stopped = *stop;  // tested once the operands are on their way
+    __builtin_amdgcn_s_setprio(3);  // before the trailing update's waves on the same SIMDs
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, li = lane & 15;
+    const int c0 = blockIdx.x * kRowCols;
+    T cv[8];  // this thread's elements of C, rows contiguous over the lanes
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        const int e = tid + 256 * u, i = e & 63, j = c0 + (e >> 6);
+        cv[u] = C[min(i, nb - 1) + (size_t)min(j, cols - 1) * lda];
+    }
+    typename Mfma<T>::acc_t acc[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+    const T* pa = D0 - depth + (size_t)min(16 * wave + li, nb - 1) * lda + 4 * g;
+    const T* pb[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+        pb[b] = C - depth + (size_t)min(c0 + 16 * b + li, cols - 1) * lda + 4 * g;
+    // ND 16-deep steps in flight.  FP64 with three takes 144 registers, the most
+    // that fits beside two waves per SIMD of update_tn_kernel; with four, this
+    // kernel got only the CUs that the update leaves out (115 us against 28).
+    constexpr int ND = sizeof(T) == 8 ? 3 : 4;
+    T a[ND][4], v[ND][2][4];
+    auto load = [&](int s, int r0) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            a[s][q] = pa[r0 + q];
+            v[s][0][q] = pb[0][r0 + q];
+            v[s][1][q] = pb[1][r0 + q];
+        }
+    };
+#pragma unroll
+    for (int s = 0; s < ND; ++s)
+        if (16 * s < depth) load(s, 16 * s);
+    if (stopped != 0) return;
+#pragma unroll 1
+    for (int r0 = 0; r0 < depth; r0 += 16 * ND)
+#pragma unroll
+        for (int s = 0; s < ND; ++s)
+            if (r0 + 16 * s < depth) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) acc[b] = Mfma<T>::op(a[s][q], v[s][b][q], acc[b]);
+                if (r0 + 16 * (s + ND) < depth) load(s, r0 + 16 * (s + ND));
+            }
+    T lv[4][4];  // Linv's row 16 wave + li
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            lv[s][q] = Linv[16 * wave + li + (size_t)kSmall * (16 * s + 4 * g + q)];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        const int e = tid + 256 * u, i = e & 63, j = e >> 6;
+        sT[j][i] = (i < nb && c0 + j < cols) ? cv[u] : T(0);
+    }
+    __syncthreads();
+    if (depth > 0) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int i = 16 * wave + Mfma<T>::row(g, r);
+                T& t = sT[16 * b + li][i];
+                t = i < nb ? t - acc[b][r] : T(0);
+            }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int b = 0; b < 2; ++b) acc[b] = {0, 0, 0, 0};
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+        if (s <= wave) {  // Linv is lower triangular
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+                    acc[b] = Mfma<T>::op(lv[s][q], sT[16 * b + li][16 * s + 4 * g + q], acc[b]);
+        }
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sT[16 * b + li][16 * wave + Mfma<T>::row(g, r)] = acc[b][r];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        const int e = tid + 256 * u, i = e & 63, j = c0 + (e >> 6);
+        if (i < nb && j < cols) C[i + (size_t)j * lda] = sT[e >> 6][i];
     }
 }
 
@@ -630,24 +1031,24 @@ template int dh_trsm_impl<float>(dh_handle_t, char, char, bool, int, int, float,
 
 // --------------------------------------------------------- Cholesky driver
 
-// Factor one diagonal block of order b (<= any): right-looking in 64-wide
-// steps entirely on the device, leaving the Linv of each 64-block in D;
+// Rows of U of one panel: b rows from the diagonal block at A11, all `cols`
+// columns from there on, 64 rows at a time.  Left-looking inside the panel:
+// the diagonal block's kernel and the row's kernel each subtract the products
+// of the rows above, so a 64-row step is two launches for any number of
+// columns.  Linv of the 64 x 64 diagonal blocks goes to D (one block, reused);
 // failures land in *dinfo with their global index.
 template <typename T>
-static int potrf_block(dh_handle_t h, int b, T* A11, int lda, T* D, int* dinfo, int base) {
+static int potrf_panel(dh_handle_t h, int b, int cols, T* A11, int lda, T* D, int* dinfo,
+                       int base) {
     for (int ii = 0; ii < b; ii += kSmall) {
-        int bb = min(kSmall, b - ii);
+        const int bb = min(kSmall, b - ii), right = cols - ii - bb;
         T* Aii = A11 + ii + (size_t)ii * lda;
-        T* Lb = D + (size_t)4096 * (ii / kSmall);
-        potrf_inv_small_kernel<T><<<1, kPotrfThreads, 0, h->stream>>>(bb, Aii, lda, Lb, dinfo,
-                                                                     base + ii);
+        potrf64_kernel<T><<<1, 256, 0, h->stream>>>(bb, ii, Aii, lda, D, dinfo, base + ii);
         DH_CHECK_LAUNCH();
-        if (ii + bb < b) {
-            T* A12 = A11 + ii + (size_t)(ii + bb) * lda;
-            T* A22 = A11 + (ii + bb) + (size_t)(ii + bb) * lda;
-            DH_CHECK_STATUS(trsm_leaf<T>(h, 'L', 'T', bb, b - ii - bb, Lb, A12, lda, dinfo));
-            DH_CHECK_STATUS(gemm_stop<T>(h, true, false, b - ii - bb, b - ii - bb, bb, T(-1), A12,
-                                         lda, A12, lda, T(1), A22, lda, 1, dinfo));
+        if (right > 0) {
+            panel_row_kernel<T><<<dh_cdiv(right, kRowCols), 256, 0, h->stream>>>(
+                bb, ii, right, Aii, D, Aii + (size_t)bb * lda, lda, dinfo);
+            DH_CHECK_LAUNCH();
         }
     }
     return 0;
@@ -660,8 +1061,7 @@ int dh_potrf_impl(dh_handle_t h, int n, T* A, int lda, int bs, int* info_host) {
     if (bs <= 0) bs = 256;
     int* dinfo = (int*)dh_ws(h, DH_WS_INFO, 64);
     if (!dinfo) return DH_ERR_ALLOC;
-    // Linv blocks of the current panel's diagonal block.
-    T* D = (T*)dh_ws(h, DH_WS_TRSM_INV, sizeof(T) * 4096 * (size_t)dh_cdiv(min(bs, n), kSmall));
+    T* D = (T*)dh_ws(h, DH_WS_TRSM_INV, sizeof(T) * 4096);  // Linv of a diagonal block
     if (!D) return DH_ERR_ALLOC;
     set_int_kernel<<<1, 1, 0, h->stream>>>(dinfo, 0);
     DH_CHECK_LAUNCH();
@@ -671,8 +1071,10 @@ int dh_potrf_impl(dh_handle_t h, int n, T* A, int lda, int bs, int* info_host) {
     // stream, which then factors that panel (latency-bound one-workgroup
     // kernels and its panel TRSM) while the rest of the trailing matrix is
     // updated on a second stream.
-    //   stream:  ... potrf/trsm(p), record P | wait U(p-1), update rows of p+1 | potrf/trsm(p+1) ...
+    //   stream:  ... panel(p) | wait U(p-1), update rows of p+1, record P | panel(p+1) ...
     //   aux:     wait P, update the rest after p, record U(p) | ...
+    // The rest waits for the rows of p+1 as well as for panel p: both fill the GPU,
+    // and the next panel cannot start before its rows.
     // Regions: the aux update writes rows past panel p+1; panel p+1's
     // factorisation reads and writes rows of p+1 only, and U12 of panel p is
     // no longer written by anyone.
@@ -685,31 +1087,28 @@ int dh_potrf_impl(dh_handle_t h, int n, T* A, int lda, int bs, int* info_host) {
     bool pending = false;  // an aux update of an earlier panel was queued
     for (int i = 0; i < n; i += bs) {
         int b = min(bs, n - i);
-        T* A11 = A + i + (size_t)i * lda;
-        DH_CHECK_STATUS(potrf_block<T>(h, b, A11, lda, D, dinfo, i));
+        DH_CHECK_STATUS(potrf_panel<T>(h, b, n - i, A + i + (size_t)i * lda, lda, D, dinfo, i));
         if (i + b >= n) break;
         T* A12 = A + i + (size_t)(i + b) * lda;
         T* A22 = A + (i + b) + (size_t)(i + b) * lda;
         const int nt = n - i - b;
-        DH_CHECK_STATUS(trsm_rec<T>(h, 'L', 'T', b, nt, A11, lda, A12, lda, D, 0, dinfo));
         if (!lookahead) {
-            DH_CHECK_STATUS(gemm_stop<T>(h, true, false, nt, nt, b, T(-1), A12, lda, A12, lda,
-                                         T(1), A22, lda, 1, dinfo));
+            DH_CHECK_STATUS(
+                trailing_update<T>(h, nt, nt, b, A12, lda, A12, lda, A22, lda, dinfo));
             continue;
         }
         const int b2 = min(bs, nt), nr = nt - b2;
-        DH_CHECK_HIP(hipEventRecord(h->ev_panel, h->stream));
         if (pending) DH_CHECK_HIP(hipStreamWaitEvent(h->stream, h->ev_update, 0));
         // Rows of the next panel, all trailing columns (upper part only).
-        DH_CHECK_STATUS(gemm_stop<T>(h, true, false, b2, nt, b, T(-1), A12, lda, A12, lda, T(1),
-                                     A22, lda, 1, dinfo));
+        DH_CHECK_STATUS(trailing_update<T>(h, b2, nt, b, A12, lda, A12, lda, A22, lda, dinfo));
+        DH_CHECK_HIP(hipEventRecord(h->ev_panel, h->stream));
         if (nr > 0) {
             DH_CHECK_HIP(hipStreamWaitEvent(h->aux, h->ev_panel, 0));
             hipStream_t main = h->stream;
-            h->stream = h->aux;  // gemm_stop launches on h->stream
-            const int st = gemm_stop<T>(h, true, false, nr, nr, b, T(-1), A12 + (size_t)b2 * lda,
-                                        lda, A12 + (size_t)b2 * lda, lda, T(1),
-                                        A22 + b2 + (size_t)b2 * lda, lda, 1, dinfo);
+            h->stream = h->aux;  // trailing_update launches on h->stream
+            const T* A13 = A12 + (size_t)b2 * lda;
+            const int st = trailing_update<T>(h, nr, nr, b, A13, lda, A13, lda,
+                                              A22 + b2 + (size_t)b2 * lda, lda, dinfo);
             h->stream = main;
             DH_CHECK_STATUS(st);
             DH_CHECK_HIP(hipEventRecord(h->ev_update, h->aux));

@@ -655,3 +655,32 @@ def test_lra_in_two_threads_gives_the_same_bits():
         assert torch.equal(o[0], out[2][0]) and torch.equal(o[1], out[2][1])
     for h in hs:
         h.close()
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("n,ld,bs,bad", [(1, 1, 256, 0), (63, 63, 256, 40), (65, 66, 256, 65),
+                                         (130, 131, 100, 0), (257, 257, 256, 257),
+                                         (700, 704, 160, 401), (2304, 2304, 256, 0),
+                                         (2307, 2309, 256, 2200), (2501, 2504, 128, 0)])
+def test_potrf_block_edges(dev, n, ld, bs, bad, f32):
+    """The blocked Cholesky at the edges of its 64-row steps, panels and
+    128 x 128 update tiles, with aligned and odd leading dimensions.  Backward
+    error: |A - U^T U| <= (n + 1) u |U^T| |U| elementwise, whose Frobenius norm
+    is at most (n + 1) u trace(A).  The strict lower part is not touched, and a
+    pivot made negative is reported as the failing minor."""
+    import torch
+    dt, u = (torch.float32, 2.0**-24) if f32 else (torch.float64, 2.0**-53)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    M = torch.randn((n, n + 8), dtype=torch.float64, device="cuda", generator=g)
+    A = (M @ M.t() / n + torch.eye(n, dtype=torch.float64, device="cuda")).to(dt)
+    K = torch.full((n, ld), 7.0, dtype=dt, device="cuda")[:, :n]
+    K.copy_(torch.tril(A) + torch.triu(torch.full_like(A, -3.0), 1))  # row j = column j
+    if bad:
+        K[bad - 1, bad - 1] = -1.0
+        assert dev.potrf(K, bs) == bad
+        return
+    assert dev.potrf(K, bs) == 0
+    U = torch.tril(K).double()  # U^T as rows
+    err = (U @ U.t() - A.double()).norm()
+    assert float(err) <= (n + 1) * u * float(torch.trace(A.double()))
+    assert bool((torch.triu(K, 1) == torch.triu(torch.full_like(A, -3.0), 1)).all())
