@@ -111,6 +111,22 @@ void* dh_ws(dh_handle_t h, dh_slot slot, size_t bytes);
 void* dh_scratch_take(int device, size_t bytes);
 void dh_scratch_release(int device);
 
+// The device's scratch buffer for the length of a call (p = nullptr: not
+// available, or not asked for).
+struct ScratchHold {
+    dh_handle_t h;
+    void* p;
+    ScratchHold(dh_handle_t h_, size_t bytes)
+        : h(h_), p(bytes ? dh_scratch_take(h_->device, bytes) : nullptr) {}
+    ~ScratchHold() {
+        if (!p) return;
+        (void)hipStreamSynchronize(h->stream);
+        dh_scratch_release(h->device);
+    }
+    ScratchHold(const ScratchHold&) = delete;
+    ScratchHold& operator=(const ScratchHold&) = delete;
+};
+
 #define DH_CHECK_HIP(expr)                                                            \
     do {                                                                              \
         hipError_t e_ = (expr);                                                       \

@@ -370,20 +370,6 @@ static int copy_panel(dh_handle_t h, int n, int l, const double* src, int lds, d
     return 0;
 }
 
-// The device's scratch buffer for the length of a call (p = nullptr: not available).
-struct ScratchHold {
-    dh_handle_t h;
-    void* p;
-    ScratchHold(dh_handle_t h_, size_t bytes) : h(h_), p(dh_scratch_take(h_->device, bytes)) {}
-    ~ScratchHold() {
-        if (!p) return;
-        (void)hipStreamSynchronize(h->stream);
-        dh_scratch_release(h->device);
-    }
-    ScratchHold(const ScratchHold&) = delete;
-    ScratchHold& operator=(const ScratchHold&) = delete;
-};
-
 // FP64 passes: Y = K*Omega -> Q; q x { K*Q -> orthonormal basis }; W = K*Q.
 //
 // All q + 2 passes multiply the same K, so the first one stores it (8 n^2

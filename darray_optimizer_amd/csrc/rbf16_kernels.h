@@ -674,3 +674,14 @@ int dh_project_fp8(dh_handle_t h, int dpad8, int ncb, int groups, int m, int nch
                    int ncb_total, const bf16x8* Xi, const bf16x8* Xj, const float* ai,
                    const float* bj, const float* si, const float* sj, float c2,
                    const bf16x8* Op, const double* yi, double* Y, int ldy);
+
+// K (m x n, row blocks of the kept layout) for all passes of a solve, and a
+// pass that reads it (rbf16_kept.hip).
+bool dh_kept16_pays(int dpad, bool fp8, int ncb, int groups, int passes);
+size_t dh_kept16_bytes(int m, int nchunks);
+int dh_form16(dh_handle_t h, bool f16, bool fp8, int dpad, int m, int nchunks, const bf16x8* Xi,
+              const bf16x8* Xj, const float* ai, const float* bj, const float* si,
+              const float* sj, float c2, void* keep);
+int dh_project16_kept(dh_handle_t h, bool f16, int ncb, int groups, int m, int nchunks, int l,
+                      int ncb_total, const void* keep, const bf16x8* Op, const double* yi,
+                      double* Y, int ldy, int splits, long ystride);

@@ -288,7 +288,7 @@ size_t packed_omega_bytes(int n, int l) {
 template <bool F16>
 int project_16(dh_handle_t h, int m, int n, int d, int l, const LowpPoints& pi,
                  const LowpPoints& pj, float c2, const bf16x8* Op, const double* yi, double* Y,
-                 int ldy) {
+                 int ldy, const void* keep = nullptr) {
     if (m == 0 || l == 0) return 0;
     int dp = dpad_of(d);
     int nchunks = dh_cdiv(n, 32);
@@ -309,7 +309,12 @@ int project_16(dh_handle_t h, int m, int n, int d, int l, const LowpPoints& pi,
         ldp = m;
     }
     int st;
-    switch (dp) {
+    if (keep) {  // K as dh_form16 left it; same splits, same bits
+        dh_timing_begin(h);
+        st = dh_project16_kept(h, F16, cols.ncb, cols.groups, m, nchunks, l, cols.ncb_pack, keep,
+                               Op, yi, P, ldp, splits, ystride);
+        dh_timing_end(h);
+    } else switch (dp) {
         case 32:
             st = dh_project16_dk1(F16, h, cols.ncb, grid, m, nchunks, l, cols.ncb_pack, xi, xj,
                                   pi.a, pj.a, c2, Op, yi, P, ldp, splits, ystride);
@@ -485,9 +490,16 @@ int prepare_points_fp8(dh_handle_t h, int m, int n, int d, const double* Xi, int
 
 int project_fp8(dh_handle_t h, int m, int n, int d, int l, const Fp8Points& pi,
                 const Fp8Points& pj, float c2, const bf16x8* Op, const double* yi, double* Y,
-                int ldy) {
+                int ldy, const void* keep = nullptr) {
     if (m == 0 || l == 0) return 0;
     Bf16Cols cols = bf16_cols(l);
+    if (keep) {
+        dh_timing_begin(h);
+        const int st = dh_project16_kept(h, false, cols.ncb, cols.groups, m, dh_cdiv(n, 32), l,
+                                         cols.ncb_pack, keep, Op, yi, Y, ldy, 1, 0);
+        dh_timing_end(h);
+        return st;
+    }
     return dh_project_fp8(h, dpad8_of(d), cols.ncb, cols.groups, m, dh_cdiv(n, 32), l,
                           cols.ncb_pack, (const bf16x8*)pi.xb, (const bf16x8*)pj.xb, pi.a, pj.a,
                           pi.sinv, pj.sinv, c2, Op, yi, Y, ldy);
@@ -559,8 +571,16 @@ int lra_16_passes(dh_handle_t h, int n, int d, int l, int q, const double* X, in
     bf16x8* Op = (bf16x8*)dh_ws(h, DH_WS_LOWP_O, packed_omega_bytes(n, l));
     if (!Op) return DH_ERR_ALLOC;
     const float c2 = (float)(2.0 * g) * kLog2e;
+    // Where it pays, K is formed once for the q + 2 passes (rbf16_kept.hip).
+    const Bf16Cols cols = bf16_cols(l);
+    const int nch = dh_cdiv(n, 32);
+    const bool pays = dh_kept16_pays(dpad_of(d), false, cols.ncb, cols.groups, q + 2);
+    const ScratchHold kk(h, pays ? dh_kept16_bytes(n, nch) : 0);
+    if (kk.p)
+        DH_CHECK_STATUS(dh_form16(h, F16, false, dpad_of(d), n, nch, (const bf16x8*)p.xb,
+                                  (const bf16x8*)p.xb, p.a, p.a, nullptr, nullptr, c2, kk.p));
     DH_CHECK_STATUS(pack_omega<F16>(h, n, l, Omega, ldo, y, Op));
-    DH_CHECK_STATUS(project_16<F16>(h, n, n, d, l, p, p, c2, Op, y, Q, ldq));
+    DH_CHECK_STATUS(project_16<F16>(h, n, n, d, l, p, p, c2, Op, y, Q, ldq, kk.p));
     int pending = 0, redone = 0;
     DH_CHECK_STATUS(dh_range_orth_begin(h, n, l, Q, ldq, &pending));
     // Power iterations alternate the basis between Q and W (no copy for even q).
@@ -569,7 +589,7 @@ int lra_16_passes(dh_handle_t h, int n, int d, int l, int q, const double* X, in
     for (int it = 0; it < q; ++it) {
         do {
             DH_CHECK_STATUS(pack_omega<F16>(h, n, l, cur, ldc, y, Op));
-            DH_CHECK_STATUS(project_16<F16>(h, n, n, d, l, p, p, c2, Op, y, nxt, ldn));
+            DH_CHECK_STATUS(project_16<F16>(h, n, n, d, l, p, p, c2, Op, y, nxt, ldn, kk.p));
             DH_CHECK_STATUS(dh_range_orth_finish(h, n, l, cur, ldc, &pending, &redone));
         } while (redone);
         DH_CHECK_STATUS(dh_range_orth_begin(h, n, l, nxt, ldn, &pending));
@@ -585,7 +605,7 @@ int lra_16_passes(dh_handle_t h, int n, int d, int l, int q, const double* X, in
                                       hipMemcpyDeviceToDevice, h->stream));
     do {
         DH_CHECK_STATUS(pack_omega<F16>(h, n, l, Q, ldq, y, Op));
-        DH_CHECK_STATUS(project_16<F16>(h, n, n, d, l, p, p, c2, Op, y, W, ldw));
+        DH_CHECK_STATUS(project_16<F16>(h, n, n, d, l, p, p, c2, Op, y, W, ldw, kk.p));
         DH_CHECK_STATUS(dh_range_orth_finish(h, n, l, Q, ldq, &pending, &redone));
     } while (redone);
     return 0;
@@ -607,15 +627,22 @@ int dh_lra_fp8_passes(dh_handle_t h, int n, int d, int l, int q, const double* X
     bf16x8* Op = (bf16x8*)dh_ws(h, DH_WS_LOWP_O, packed_omega_bytes(n, l));
     if (!Op) return DH_ERR_ALLOC;
     const float c2 = (float)(2.0 * gamma) * kLog2e;
+    const Bf16Cols cols = bf16_cols(l);
+    const int nch = dh_cdiv(n, 32);
+    const bool pays = dh_kept16_pays(dpad8_of(d), true, cols.ncb, cols.groups, q + 2);
+    const ScratchHold kk(h, pays ? dh_kept16_bytes(n, nch) : 0);
+    if (kk.p)
+        DH_CHECK_STATUS(dh_form16(h, false, true, dpad8_of(d), n, nch, (const bf16x8*)p.xb,
+                                  (const bf16x8*)p.xb, p.a, p.a, p.sinv, p.sinv, c2, kk.p));
     DH_CHECK_STATUS(pack_omega<false>(h, n, l, Omega, ldo, y, Op));
-    DH_CHECK_STATUS(project_fp8(h, n, n, d, l, p, p, c2, Op, y, Q, ldq));
+    DH_CHECK_STATUS(project_fp8(h, n, n, d, l, p, p, c2, Op, y, Q, ldq, kk.p));
     DH_CHECK_STATUS(dh_range_orth(h, n, l, Q, ldq));
     // Power iterations alternate the basis between Q and W (no copy for even q).
     double *cur = Q, *nxt = W;
     int ldc = ldq, ldn = ldw;
     for (int it = 0; it < q; ++it) {
         DH_CHECK_STATUS(pack_omega<false>(h, n, l, cur, ldc, y, Op));
-        DH_CHECK_STATUS(project_fp8(h, n, n, d, l, p, p, c2, Op, y, nxt, ldn));
+        DH_CHECK_STATUS(project_fp8(h, n, n, d, l, p, p, c2, Op, y, nxt, ldn, kk.p));
         DH_CHECK_STATUS(dh_range_orth(h, n, l, nxt, ldn));
         std::swap(cur, nxt);
         std::swap(ldc, ldn);
@@ -625,7 +652,7 @@ int dh_lra_fp8_passes(dh_handle_t h, int n, int d, int l, int q, const double* X
                                       sizeof(double) * (size_t)ldc, sizeof(double) * (size_t)n, l,
                                       hipMemcpyDeviceToDevice, h->stream));
     DH_CHECK_STATUS(pack_omega<false>(h, n, l, Q, ldq, y, Op));
-    return project_fp8(h, n, n, d, l, p, p, c2, Op, y, W, ldw);
+    return project_fp8(h, n, n, d, l, p, p, c2, Op, y, W, ldw, kk.p);
 }
 
 int dh_lra_f16_passes(dh_handle_t h, int n, int d, int l, int q, const double* X, int ldx,

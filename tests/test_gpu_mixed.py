@@ -280,3 +280,23 @@ def test_lra_fp8_error_close_to_fp64(dev):
         errs[prec] = np.sqrt(e2 / k2)
     print(f"LRA errors: fp64 {errs[dh.DH_PREC_F64]:.4e}  fp8 {errs[dh.DH_PREC_FP8]:.4e}")
     assert errs[dh.DH_PREC_FP8] <= 1.5 * errs[dh.DH_PREC_F64] + 2e-3
+
+
+@pytest.mark.parametrize("prec", ["f16", "bf16", "fp8"])
+@pytest.mark.parametrize("n,d,l", [(200, 129, 130), (1000, 200, 144), (2051, 256, 200),
+                                   (2500, 140, 290), (33000, 256, 136)])
+def test_lra_on_kept_kernel_values_gives_the_fused_bits(dev, prec, n, d, l):
+    """At 129..256 features a solve of three passes keeps K between them where
+    that pays; its W must be bit for bit the fused pass applied to its Q."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(n + l)
+    X = 0.3 * torch.randn((n, d), dtype=torch.float64, device="cuda", generator=g)
+    y = 1.0 - 2.0 * (torch.arange(n, device="cuda") % 3 == 0).double()
+    Om = torch.randn((l, n), dtype=torch.float64, device="cuda", generator=g)
+    Q, W, P = torch.empty_like(Om), torch.empty_like(Om), torch.empty_like(Om)
+    which = {"f16": dh.DH_PREC_F16, "bf16": dh.DH_PREC_BF16, "fp8": dh.DH_PREC_FP8}[prec]
+    project = {"f16": dev.rbf_project_f16, "bf16": dev.rbf_project_bf16,
+               "fp8": dev.rbf_project_fp8}[prec]
+    assert dev.lra(X, Om, 0.5 / d, 1, Q, W, y=y, prec=which) == 0
+    project(X, X, Q, 0.5 / d, P, yi=y, yj=y)
+    assert torch.equal(W, P)
