@@ -27,6 +27,13 @@ __device__ __forceinline__ void dma16(const void* gbase, unsigned voff, void* ld
                  : "v"(voff), "s"(__builtin_amdgcn_readfirstlane(base)), "s"(uniform_ptr(gbase))
                  : "memory", "m0");
 }
+// The same with the LDS byte address `base` (uniform) instead of a pointer.
+__device__ __forceinline__ void dma16_at(const void* gbase, unsigned voff, unsigned base) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %2"
+                 :
+                 : "v"(voff), "s"(__builtin_amdgcn_readfirstlane(base)), "s"(uniform_ptr(gbase))
+                 : "memory", "m0");
+}
 __device__ __forceinline__ void dma4(const void* gbase, unsigned voff, void* lds) {
     unsigned base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)lds;
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, %2"

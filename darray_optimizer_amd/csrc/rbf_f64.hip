@@ -790,6 +790,223 @@ __global__ __launch_bounds__(256) void lra_error_f64_kernel(
     }
 }
 
+// The same sums on 128 x 128 tiles of the upper triangle: distances and
+// exponentials are symmetric, so tile (I, J) forms K once and compares it with
+// Q_I W_J^T and, off the diagonal, with the transpose of Q_J W_I^T, in the
+// same accumulator layout.  Operands are point-major copies padded to whole
+// 16-deep stages of 128 bytes (pack_points_kernel, transpose_panel_kernel),
+// staged by direct copies through a 3-deep LDS ring without a gap between the
+// phases and tiles; 8 waves of 32 x 64, one persistent workgroup per CU.  A
+// stage's 16-byte pieces of point i lie at p ^ ((i / 2) % 8) of its 128 bytes;
+// lane group g takes pieces 2g and 2g + 1 as the k-slot g of four MFMAs.  Each
+// lane adds its tiles' sums up with their rounding errors (two-sum), so how
+// many tiles a lane gets does not matter to the result's accuracy.  At n =
+// 65536, d = 128, l = 272: 50.2 ms, 57 TFLOP/s of the 2.9e12 that are left (73% of
+// the FP64 MFMA peak; the 64 x 64 tiles 63%), the exponentials between them.
+__global__ __launch_bounds__(512) void lra_error_sym_kernel(
+    int n, int sd, int sl, const double* __restrict__ Xp, const double* __restrict__ nrm,
+    const double* __restrict__ y, double gamma, int ntiles, double* __restrict__ partial) {
+    __shared__ __align__(128) char ring[3][2][128 * 128];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, li = lane & 15;
+    const int wi = wave & 3, wj = wave >> 2;
+    const int dp = 16 * sd, lp = 16 * sl;
+    const size_t qofs = (size_t)n * dp, wofs = (size_t)n * lp;  // Q after the points, W after Q
+    // Tiles in order of columns bj, rows bi <= bj; each XCD a contiguous range.
+    const int x = blockIdx.x & 7, per = ntiles / 8, rem = ntiles % 8;
+    int tile = x * per + min(x, rem);
+    const int last = tile + per + (x < rem ? 1 : 0), step = gridDim.x >> 3;
+    tile += blockIdx.x >> 3;
+    struct Tile {
+        int i0, j0, nst;
+    };
+    auto decode = [&](int t) {
+        int bj = (int)((sqrtf(8.0f * (float)t + 1.0f) - 1.0f) * 0.5f);
+        while ((bj + 1) * (bj + 2) / 2 <= t) ++bj;
+        while (bj * (bj + 1) / 2 > t) --bj;
+        const int bi = t - bj * (bj + 1) / 2;
+        return Tile{__builtin_amdgcn_readfirstlane(bi * 128),
+                    __builtin_amdgcn_readfirstlane(bj * 128),
+                    __builtin_amdgcn_readfirstlane(bi == bj ? sd + sl : sd + 2 * sl)};
+    };
+    const unsigned ring0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char*)ring;
+    int ftile = tile, fst = 0, fsl = 0;  // the next stage to copy, and its slot
+    Tile f = decode(min(tile, ntiles - 1));
+    unsigned ri[2], rj[2], off[2];  // this lane's rows from i0 / j0 and bytes within a stage
+    auto rows = [&]() {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int row = 8 * (8 * u + wave) + (lane >> 3);
+            ri[u] = (unsigned)(min(f.i0 + row, n - 1) - f.i0) * 8u;
+            rj[u] = (unsigned)(min(f.j0 + row, n - 1) - f.j0) * 8u;
+            off[u] = (unsigned)(((lane & 7) ^ ((row >> 1) & 7)) * 16);
+        }
+    };
+    auto issue = [&]() {  // false once the last tile's stages are under way
+        if (ftile >= last) return false;
+        const bool dist = fst < sd, first = fst < sd + sl;
+        // (Arithmetic instead of choices between captured values, which would be
+        // kept in memory to be chosen by address.)
+        const int pd = dist, pw = !dist && !first, pq = !dist && first;
+        const int ld = lp + pd * (dp - lp);
+        const int k0 = 16 * (fst - (1 - pd) * sd - pw * sl);
+        const double* a = Xp + (size_t)(1 - pd) * qofs + (size_t)pw * wofs + (size_t)f.i0 * ld + k0;
+        const double* b = Xp + (size_t)(1 - pd) * qofs + (size_t)pq * wofs + (size_t)f.j0 * ld + k0;
+        const unsigned to = ring0 + 32768u * fsl + 1024u * wave;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            dma16_at(a, ri[u] * (unsigned)ld + off[u], to + 8192 * u);
+            dma16_at(b, rj[u] * (unsigned)ld + off[u], to + 16384 + 8192 * u);
+        }
+        fsl = fsl == 2 ? 0 : fsl + 1;
+        if (++fst == f.nst) {
+            fst = 0;
+            ftile += step;
+            if (ftile < last) {
+                f = decode(ftile);
+                rows();
+            }
+        }
+        return true;
+    };
+    const int off0 = ((2 * g) ^ (li >> 1)) * 16, off1 = ((2 * g + 1) ^ (li >> 1)) * 16;
+    rows();
+    issue();
+    bool ahead = issue();  // a stage after the one to be waited for is under way
+    int slot = 0;
+    // acc = `count` stages of (J side) . (I side).
+    auto product = [&](dh_d4(&acc)[4][2], int count) {
+#pragma unroll
+        for (int cj = 0; cj < 4; ++cj)
+#pragma unroll
+            for (int ci = 0; ci < 2; ++ci) acc[cj][ci] = dh_d4{0, 0, 0, 0};
+        for (int st = 0; st < count; ++st) {
+            if (ahead)
+                __builtin_amdgcn_s_waitcnt(0x0F74);  // all but the newest stage's four copies
+            else
+                wait_vm();
+            __syncthreads();
+            ahead = issue();
+            const char* la = ring[slot][0] + (wi * 32 + li) * 128;
+            const char* lb = ring[slot][1] + (wj * 64 + li) * 128;
+            slot = slot == 2 ? 0 : slot + 1;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int o = h ? off1 : off0;
+                d2v av[2], bv[4];
+#pragma unroll
+                for (int c = 0; c < 2; ++c) av[c] = *(const d2v*)(la + c * 2048 + o);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) bv[c] = *(const d2v*)(lb + c * 2048 + o);
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+#pragma unroll
+                    for (int cj = 0; cj < 4; ++cj)
+#pragma unroll
+                        for (int ci = 0; ci < 2; ++ci)
+                            acc[cj][ci] = Mfma<double>::op(bv[cj][e], av[ci][e], acc[cj][ci]);
+            }
+        }
+    };
+    double se = 0.0, sk = 0.0, le = 0.0, lk = 0.0;  // sums and their rounding errors
+    auto add = [](double& s, double& c, double v) {
+        const double t = s + v, z = t - s;
+        c += (s - (t - z)) + (v - z);
+        s = t;
+    };
+    for (; tile < last; tile += step) {
+        const Tile o = decode(tile);
+        const int i1 = o.i0 + wi * 32 + li, j1 = o.j0 + wj * 64 + g;
+        dh_d4 K[4][2], P[4][2];
+        product(K, sd);
+        double ni[2], yi[2], ts = 0.0;
+#pragma unroll
+        for (int ci = 0; ci < 2; ++ci) {
+            const int i = min(i1 + 16 * ci, n - 1);
+            ni[ci] = nrm[i];
+            yi[ci] = y ? y[i] : 1.0;
+        }
+#pragma unroll
+        for (int cj = 0; cj < 4; ++cj) {
+            double nj[4], yj[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int j = min(j1 + 16 * cj + 4 * r, n - 1);
+                nj[r] = nrm[j];
+                yj[r] = y ? y[j] : 1.0;
+            }
+            wait_vm();  // here, so that no wait is left for the products' loop
+#pragma unroll
+            for (int ci = 0; ci < 2; ++ci)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    double d2 = ni[ci] + nj[r] - 2.0 * K[cj][ci][r];
+                    d2 = d2 > 0.0 ? d2 : 0.0;
+                    double kv = exp(-gamma * d2);
+                    if (y) kv *= yi[ci] * yj[r];
+                    K[cj][ci][r] = kv;
+                    ts += (i1 + 16 * ci < n && j1 + 16 * cj + 4 * r < n) ? kv * kv : 0.0;
+                }
+        }
+        const bool diag = o.i0 == o.j0;
+        add(sk, lk, diag ? ts : 2.0 * ts);
+        for (int side = 0; side < (diag ? 1 : 2); ++side) {
+            product(P, sl);
+            ts = 0.0;
+#pragma unroll
+            for (int cj = 0; cj < 4; ++cj)
+#pragma unroll
+                for (int ci = 0; ci < 2; ++ci)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const double e = K[cj][ci][r] - P[cj][ci][r];
+                        ts += (i1 + 16 * ci < n && j1 + 16 * cj + 4 * r < n) ? e * e : 0.0;
+                    }
+            add(se, le, ts);
+        }
+    }
+    se += le;
+    sk += lk;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        se += __shfl_xor(se, o);
+        sk += __shfl_xor(sk, o);
+    }
+    if (lane == 0) {
+        double* p = partial + 2 * (8 * (size_t)blockIdx.x + wave);
+        p[0] = se;
+        p[1] = sk;
+    }
+}
+
+// Points (d features each, ld ldx) as rows of dp features, zero-padded.
+__global__ __launch_bounds__(256) void pack_points_kernel(int n, int d, int dp,
+                                                          const double* __restrict__ X, int ldx,
+                                                          double* __restrict__ out) {
+    const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= (size_t)n * dp) return;
+    const int f = (int)(e % dp);
+    out[e] = f < d ? X[f + (e / dp) * ldx] : 0.0;
+}
+
+// The n x l column-major panel P as rows of lp columns, zero-padded.
+__global__ __launch_bounds__(256) void transpose_panel_kernel(int n, int l, int lp,
+                                                              const double* __restrict__ P,
+                                                              int ldp, double* __restrict__ out) {
+    __shared__ double s[32][33];
+    const int i0 = blockIdx.x * 32, c0 = blockIdx.y * 32, a = threadIdx.x & 31, b = threadIdx.x >> 5;
+#pragma unroll
+    for (int u = 0; u < 32; u += 8) {
+        const int c = c0 + b + u, i = i0 + a;
+        s[b + u][a] = (i < n && c < l) ? P[i + (size_t)c * ldp] : 0.0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 32; u += 8) {
+        const int i = i0 + b + u, c = c0 + a;
+        if (i < n && c < lp) out[(size_t)i * lp + c] = s[a][b + u];
+    }
+}
+
 // Fixed-order reduction of `count` (se, sk) pairs into out[0..1].
 __global__ __launch_bounds__(256) void reduce_pairs_kernel(size_t count,
                                                             const double* __restrict__ partial,
@@ -833,12 +1050,39 @@ extern "C" int dh_lra_error(dh_handle_t h, int n, int d, int l, const double* X,
     double* nrm = (double*)dh_ws(h, DH_WS_NORMS, sizeof(double) * (size_t)n);
     if (!nrm) return DH_ERR_ALLOC;
     DH_CHECK_STATUS(launch_sqnorms<double>(h, n, d, X, ldx, nrm));
+    // 128 x 128 tiles of one triangle from more than five per CU (n = 6401): there
+    // the last, partly filled round of tiles no longer costs more than they
+    // save (d = 20, l = 250: n = 5000 0.36 -> 0.37 ms, n = 8000 0.84 -> 0.71 ms; n = 65536,
+    // d = 128, l = 272: 71.1 -> 50.0 ms).  The 64 x 64 tiles of the whole matrix below
+    // that, and for d = 0 or l = 0.  A tile's copies have 32-bit byte offsets.
+    const int sd = dh_cdiv(d, 16), sl = dh_cdiv(l, 16), nt = dh_cdiv(n, 128);
+    const long tiles = (long)nt * (nt + 1) / 2;
+    const bool sym = tiles > 5L * h->num_cu && d > 0 && l > 0 && std::max(sd, sl) < (1 << 18) &&
+                     tiles < (1L << 30);
+    const int wgs = (int)std::min<long>((tiles + 7) / 8 * 8, std::max(8, h->num_cu / 8 * 8));
     dim3 grid(dh_cdiv(n, 64), dh_cdiv(n, 64));
-    size_t nblk = (size_t)grid.x * grid.y;
+    size_t nblk = sym ? 8 * (size_t)wgs : (size_t)grid.x * grid.y;
     double* part = (double*)dh_ws(h, DH_WS_PARTIAL, sizeof(double) * (2 * nblk + 2));
     if (!part) return DH_ERR_ALLOC;
-    lra_error_f64_kernel<<<grid, 256, 0, h->stream>>>(n, d, l, X, ldx, nrm, y, gamma, Q, ldq, W,
-                                                      ldw, part);
+    if (sym) {
+        double* Xp = (double*)dh_ws(h, DH_WS_PACK64,
+                                    sizeof(double) * 16 * (size_t)n * ((size_t)sd + 2 * sl));
+        if (!Xp) return DH_ERR_ALLOC;
+        double *Qp = Xp + 16 * (size_t)n * sd, *Wp = Qp + 16 * (size_t)n * sl;
+        pack_points_kernel<<<(unsigned)(((size_t)n * sd * 16 + 255) / 256), 256, 0, h->stream>>>(
+            n, d, 16 * sd, X, ldx, Xp);
+        DH_CHECK_LAUNCH();
+        const dim3 tg(dh_cdiv(n, 32), dh_cdiv(16 * sl, 32));
+        transpose_panel_kernel<<<tg, 256, 0, h->stream>>>(n, l, 16 * sl, Q, ldq, Qp);
+        DH_CHECK_LAUNCH();
+        transpose_panel_kernel<<<tg, 256, 0, h->stream>>>(n, l, 16 * sl, W, ldw, Wp);
+        DH_CHECK_LAUNCH();
+        lra_error_sym_kernel<<<wgs, 512, 0, h->stream>>>(n, sd, sl, Xp, nrm, y, gamma,
+                                                         (int)tiles, part);
+    } else {
+        lra_error_f64_kernel<<<grid, 256, 0, h->stream>>>(n, d, l, X, ldx, nrm, y, gamma, Q, ldq,
+                                                          W, ldw, part);
+    }
     DH_CHECK_LAUNCH();
     reduce_pairs_kernel<<<1, 256, 0, h->stream>>>(nblk, part, part + 2 * nblk);
     DH_CHECK_LAUNCH();

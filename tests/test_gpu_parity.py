@@ -684,3 +684,30 @@ def test_potrf_block_edges(dev, n, ld, bs, bad, f32):
     err = (U @ U.t() - A.double()).norm()
     assert float(err) <= (n + 1) * u * float(torch.trace(A.double()))
     assert bool((torch.triu(K, 1) == torch.triu(torch.full_like(A, -3.0), 1)).all())
+
+
+@pytest.mark.parametrize("n,d,l,labels", [(6401, 1, 1, False), (6528, 16, 16, True),
+                                          (6500, 130, 17, True), (7001, 33, 40, False),
+                                          (6690, 300, 5, True)])
+def test_lra_error_on_symmetric_tiles(dev, n, d, l, labels):
+    """||K - Q W^T||^2 and ||K||^2 from 128 x 128 tiles of one triangle against
+    plain FP64 on the whole matrix.  With e = K - Q W^T off by D, the first sum is
+    off by at most 2 |e| |D|; |D| is bounded elementwise by (l + 2) u |Q||W|^T for
+    the product and by the exponent's error for K <= 1, on either side."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(n + d)
+    X = torch.randn((n, d), dtype=torch.float64, device="cuda", generator=g) / d**0.5
+    y = (1.0 - 2.0 * (torch.arange(n, device="cuda") % 2)).double() if labels else None
+    Q, W = (torch.randn((l, n), dtype=torch.float64, device="cuda", generator=g) for _ in range(2))
+    gamma, u = 0.7, 2.0**-53
+    e2, k2 = dev.lra_error(X, gamma, Q, W, y=y)
+    s = (X * X).sum(1)
+    K = torch.exp(-gamma * (s[:, None] + s[None, :] - 2.0 * (X @ X.t())).clamp(min=0.0))
+    if y is not None:
+        K = K * y[:, None] * y[None, :]
+    E = K - Q.t().contiguous() @ W
+    kerr = (4.0 * gamma * float(s.max()) * (d + 4) + 4) * u
+    D = 2 * ((l + 2) * u * (Q.abs().t().contiguous() @ W.abs()) + kerr * K.abs())
+    ref_e, ref_k = float((E * E).sum()), float((K * K).sum())
+    assert abs(e2 - ref_e) <= 2 * float(E.norm() * D.norm()) + 1e-14 * ref_e
+    assert abs(k2 - ref_k) <= (4 * kerr + 1e-14) * ref_k
