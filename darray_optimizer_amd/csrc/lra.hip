@@ -14,7 +14,7 @@ int dh_project_f64_split(dh_handle_t h, int m, int n, int d, int l, const double
                         const double* Xj, int ldxj, const double* ni, const double* nj,
                         const double* yi, const double* yj, double gamma, const double* O,
                         int ldo, double* Y, int ldy, void* keep, int kmode);
-size_t dh_kkeep_bytes(int m, int n, int d);
+size_t dh_kkeep_bytes(int m, int n);
 int dh_lra_bf16_passes(dh_handle_t h, int n, int d, int l, int q, const double* X, int ldx,
                        const double* y, double gamma, const double* Omega, int ldo, double* Q,
                        int ldq, double* W, int ldw);
@@ -385,7 +385,7 @@ static int lra_f64(dh_handle_t h, int n, int d, int l, int q, const double* X, i
     double* nrm = (double*)dh_ws(h, DH_WS_NORMS, sizeof(double) * (size_t)n);
     if (!nrm) return DH_ERR_ALLOC;
     DH_CHECK_STATUS(dh_sqnorms_f64(h, n, d, X, ldx, nrm));
-    const ScratchHold kk(h, dh_kkeep_bytes(n, n, d));
+    const ScratchHold kk(h, dh_kkeep_bytes(n, n));
     const int store = kk.p ? 1 : 0, use = kk.p ? 2 : 0;
     DH_CHECK_STATUS(dh_project_f64_split(h, n, n, d, l, X, ldx, X, ldx, nrm, nrm, y, y, gamma,
                                         Omega, ldo, Q, ldq, kk.p, store));

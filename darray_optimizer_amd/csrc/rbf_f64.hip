@@ -374,6 +374,73 @@ __global__ __launch_bounds__(256) void rbf_project_f64_kernel(
         }
 }
 
+// K without labels in the layout of a KEEP pass, for points of any number of
+// features: 64 x 64 distance tiles (tile_mma) with the points of the columns as
+// tile rows, so that the accumulators of lane (g, li) are already its pairs.
+// SYM (Xi = Xj): one triangle of tiles, of which the strict part is stored a
+// second time with every 16 x 16 block transposed through LDS; the products
+// and norms commute, so both halves have the bits of their own tile.
+template <bool SYM>
+__global__ __launch_bounds__(256) void form_f64_kernel(int m, int n, int d,
+                                                       const double* __restrict__ Xi, int ldxi,
+                                                       const double* __restrict__ Xj, int ldxj,
+                                                       const double* __restrict__ ni,
+                                                       const double* __restrict__ nj,
+                                                       double gamma, d2v* __restrict__ Kk,
+                                                       int nrb) {
+    __shared__ double sA[kTileBK][64 + kTilePad];
+    __shared__ double sB[kTileBK][64 + kTilePad];
+    __shared__ double sT[4][16][17];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, li = lane & 15;
+    int bj = blockIdx.x, bi = blockIdx.y;  // tile rows: points of Xj; tile columns: of Xi
+    if (SYM) {
+        const int t = blockIdx.x;
+        bi = (int)((sqrtf(8.0f * (float)t + 1.0f) - 1.0f) * 0.5f);
+        while ((bi + 1) * (bi + 2) / 2 <= t) ++bi;
+        while (bi * (bi + 1) / 2 > t) --bi;
+        bj = t - bi * (bi + 1) / 2;
+    }
+    dh_d4 acc[2][2];
+    zero_acc<double, 2, 2>(acc);
+    tile_mma<double, 64, 64, true, false>(acc, sA, sB, n, m, 64 * bj, 64 * bi, 0, d, Xj, ldxj, Xi,
+                                          ldxi);
+    const int nch = (n + 15) / 16;
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const int t = 4 * bj + (wave & 1) * 2 + a, rb = 4 * bi + (wave >> 1) * 2 + b;
+            const double nrow = ni[min(16 * rb + li, m - 1)];
+            double kv[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                double d2 = nrow + nj[min(16 * t + 4 * r + g, n - 1)] - 2.0 * acc[a][b][r];
+                d2 = d2 > 0.0 ? d2 : 0.0;
+                kv[r] = exp(-gamma * d2);
+            }
+            if (t < nch) {  // row blocks are padded to whole tiles, chunks are not
+                d2v* kp = Kk + ((size_t)t * nrb + rb) * 128 + lane;
+                kp[0] = d2v{kv[0], kv[1]};
+                kp[64] = d2v{kv[2], kv[3]};
+            }
+            if (SYM && bi != bj) {  // block (rb, t) transposed: row block t, chunk rb
+#pragma unroll
+                for (int r = 0; r < 4; ++r) sT[wave][4 * r + g][li] = kv[r];
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int r = 0; r < 4; ++r) kv[r] = sT[wave][li][4 * r + g];
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                if (rb < nch) {
+                    d2v* kp = Kk + ((size_t)rb * nrb + t) * 128 + lane;
+                    kp[0] = d2v{kv[0], kv[1]};
+                    kp[64] = d2v{kv[2], kv[3]};
+                }
+            }
+        }
+}
+
 // Y = K O from the K values that a KEEP pass stored, with that pass's packed
 // Omega image, chunk order and MFMAs, so it returns the bits that the fused
 // kernel would.  Rows, columns and splits as there; what is gone is the
@@ -499,41 +566,6 @@ static int dispatch_ncb(dh_handle_t h, int ncb, dim3 grid, int m, int n, int d, 
     return 0;
 }
 
-// Above 256 features a wave's rows of Xi no longer fit in registers.  K is
-// then materialised in row blocks of at most 2^27 entries (1 GiB), each by the
-// distance-GEMM tile kernel (FP64 MFMA, exp epilogue), and multiplied into
-// Omega by the FP64 GEMM: Y_blk = K_blk Omega + beta Y_blk.  The same split as
-// rbf_kernel's explicit tiles (dkernel.cu:144-178), with the product fused in.
-// With `keep` (m n doubles) every block has its own place there: kmode 1 forms
-// the blocks, kmode 2 takes them as an earlier pass left them.
-static int project_f64_blocked(dh_handle_t h, int m, int n, int d, int l, const double* Xi,
-                               int ldxi, const double* Xj, int ldxj, const double* ni,
-                               const double* nj, const double* yi, const double* yj, double gamma,
-                               const double* O, int ldo, double beta, double* Y, int ldy,
-                               double* keep, int kmode) {
-    if (n == 0)  // K has no columns: Y = beta Y
-        return dh_gemm_impl<double>(h, false, false, m, l, 0, 1.0, O, 1, O, ldo, beta, Y, ldy, 0);
-    const long cap = 1L << 27;
-    int mb = (int)std::min<long>(m, std::max<long>(64, cap / n / 64 * 64));
-    double* Kb = keep ? keep : (double*)dh_ws(h, DH_WS_KBLOCK, sizeof(double) * (size_t)mb * n);
-    if (!Kb) return DH_ERR_ALLOC;
-    dh_timing_begin(h);
-    for (int i0 = 0; i0 < m; i0 += mb) {
-        const int ib = std::min(mb, m - i0);
-        if (keep) Kb = keep + (size_t)i0 * n;
-        dim3 grid(dh_cdiv(ib, 64), dh_cdiv(n, 64));
-        if (kmode != 2)
-            rbf_tile_kernel<double, 64, 64><<<grid, 256, 0, h->stream>>>(
-                ib, n, d, Xi + (size_t)i0 * ldxi, ldxi, Xj, ldxj, ni + i0, nj,
-                yi ? yi + i0 : nullptr, yj, gamma, Kb, ib);
-        DH_CHECK_LAUNCH();
-        DH_CHECK_STATUS(dh_gemm_impl<double>(h, false, false, ib, l, n, 1.0, Kb, ib, O, ldo, beta,
-                                             Y + i0, ldy, 0));
-    }
-    dh_timing_end(h);
-    return 0;
-}
-
 // Smallest instantiated column-block count >= want.
 static int ncb_instance(int want) {
     static const int inst[] = {1, 2, 3, 4, 5, 6, 8, 9, 12, 17};
@@ -556,24 +588,25 @@ static int pack_omega_f64(dh_handle_t h, int n, int l, int ncbp, const double* O
     return 0;
 }
 
-// Y (m x l) = K O from the kept K values (kept_project_f64_kernel).  Without
-// the distance operands 17 column blocks fit at every d, and how the columns
-// are grouped changes no bit.
-static int project_f64_kept(dh_handle_t h, int m, int n, int l, const double* yi,
-                            const double* yj, const double* O, int ldo, double* Y, int ldy,
-                            int jps, int splits, long ystride, const void* keep) {
+// Column blocking of a pass on kept K values: without the distance operands 17
+// column blocks fit at every d, and how the columns are grouped changes no bit.
+static void kept_columns(int l, int* ncb, int* groups) {
     const int ncb_total = dh_cdiv(l, 16);
-    const int ncb = ncb_instance(dh_cdiv(ncb_total, dh_cdiv(ncb_total, 17)));
-    const int groups = dh_cdiv(ncb_total, ncb);
-    const d2v* Opk = nullptr;
-    DH_CHECK_STATUS(pack_omega_f64(h, n, l, groups * ncb, O, ldo, yj, &Opk));
+    *ncb = ncb_instance(dh_cdiv(ncb_total, dh_cdiv(ncb_total, 17)));
+    *groups = dh_cdiv(ncb_total, *ncb);
+}
+
+// Y (m x l) = K O from K values in the kept layout, Omega packed in ncb x groups
+// column blocks.
+static int launch_kept_f64(dh_handle_t h, int m, int n, int l, int ncb, int groups,
+                           const double* yi, const d2v* Opk, double* Y, int ldy, int jps,
+                           int splits, long ystride, const void* keep) {
     dim3 grid(dh_cdiv(m, 64), groups, splits);
-    dh_timing_begin(h);
-#define DH_NCB(N)                                                                            \
-    case N:                                                                                  \
-        kept_project_f64_kernel<N><<<grid, 256, 0, h->stream>>>(                             \
-            m, n, l, (const d2v*)keep, 4 * grid.x, yi, Opk, groups* ncb, Y, ldy, jps,        \
-            ystride);                                                                        \
+#define DH_NCB(N)                                                                         \
+    case N:                                                                               \
+        kept_project_f64_kernel<N><<<grid, 256, 0, h->stream>>>(                          \
+            m, n, l, (const d2v*)keep, 4 * grid.x, yi, Opk, groups* ncb, Y, ldy, jps,     \
+            ystride);                                                                     \
         break;
     switch (ncb) {
         DH_NCB(1)
@@ -589,15 +622,112 @@ static int project_f64_kept(dh_handle_t h, int m, int n, int l, const double* yi
             DH_NCB(17)
     }
 #undef DH_NCB
-    dh_timing_end(h);
     DH_CHECK_LAUNCH();
     return 0;
 }
 
-// Bytes that dh_project_f64_split needs to keep K (m x n, d features).
-size_t dh_kkeep_bytes(int m, int n, int d) {
-    if (d > 256) return sizeof(double) * (size_t)m * n;
+static int project_f64_kept(dh_handle_t h, int m, int n, int l, const double* yi,
+                            const double* yj, const double* O, int ldo, double* Y, int ldy,
+                            int jps, int splits, long ystride, const void* keep) {
+    int ncb, groups;
+    kept_columns(l, &ncb, &groups);
+    const d2v* Opk = nullptr;
+    DH_CHECK_STATUS(pack_omega_f64(h, n, l, groups * ncb, O, ldo, yj, &Opk));
+    dh_timing_begin(h);
+    DH_CHECK_STATUS(launch_kept_f64(h, m, n, l, ncb, groups, yi, Opk, Y, ldy, jps, splits, ystride,
+                                    keep));
+    dh_timing_end(h);
+    return 0;
+}
+
+// Y = beta Y + sum over the splits z (in order) of P[z ystride + i + c m].
+__global__ __launch_bounds__(256) void sum_splits_f64_kernel(int m, int l, int splits,
+                                                             const double* __restrict__ P,
+                                                             long ystride, double beta,
+                                                             double* __restrict__ Y, int ldy) {
+    const long e = (long)blockIdx.x * 256 + threadIdx.x;
+    if (e >= (long)m * l) return;
+    const int i = (int)(e % m), c = (int)(e / m);
+    double v = 0.0;
+    for (int z = 0; z < splits; ++z) v += P[z * ystride + e];
+    double* yp = Y + i + (size_t)c * ldy;
+    *yp = (beta == 0.0) ? v : v + beta * (*yp);
+}
+
+// Bytes of K (m x n) in the kept layout: whole 64-row tiles, 16-point chunks.
+static size_t kept_bytes(int m, int n) {
     return sizeof(double) * ((size_t)dh_cdiv(m, 64) * 64) * ((size_t)dh_cdiv(n, 16) * 16);
+}
+
+// Above 256 features a wave's rows of Xi no longer fit in registers.  K is then
+// formed in the kept layout by distance tiles, in row blocks of at most 2^27
+// entries (1 GiB), and each block multiplied into Omega by
+// kept_project_f64_kernel.  The same split as rbf_kernel's explicit tiles
+// (dkernel.cu:144-178).  With `keep` K is one block there: kmode 1 forms it,
+// from one triangle where both point sets are the same; kmode 2 takes it as an
+// earlier pass left it.  The j range is split until there are two workgroups
+// per CU, by the whole m, so blocks and splits return the same bits.  (Column-
+// major blocks through the 64 x 64 GEMM: n = 9000, d = 600, l = 74 took 2.13 + 0.49
+// ms per pass; forming one triangle takes 1.07 and a pass 0.33.)
+static int project_f64_blocked(dh_handle_t h, int m, int n, int d, int l, const double* Xi,
+                               int ldxi, const double* Xj, int ldxj, const double* ni,
+                               const double* nj, const double* yi, const double* yj, double gamma,
+                               const double* O, int ldo, double beta, double* Y, int ldy,
+                               void* keep, int kmode) {
+    if (n == 0)  // K has no columns: Y = beta Y
+        return dh_gemm_impl<double>(h, false, false, m, l, 0, 1.0, O, 1, O, ldo, beta, Y, ldy, 0);
+    const long cap = 1L << 27;
+    const int mb = keep ? m : (int)std::min<long>(m, std::max<long>(64, cap / n / 64 * 64));
+    void* Kb = keep ? keep : dh_ws(h, DH_WS_KBLOCK, kept_bytes(mb, n));
+    if (!Kb) return DH_ERR_ALLOC;
+    int ncb, groups;
+    kept_columns(l, &ncb, &groups);
+    const int nch = dh_cdiv(n, 32);
+    int splits = 1;
+    while (splits < 8 && (long)dh_cdiv(m, 64) * groups * splits < 2L * h->num_cu &&
+           nch >= 32 * splits)
+        splits *= 2;
+    const int jps = splits == 1 ? n : dh_cdiv(nch, splits) * 32;
+    splits = dh_cdiv(n, jps);
+    const bool direct = splits == 1 && beta == 0.0;
+    double* P = nullptr;
+    if (!direct) {
+        P = (double*)dh_ws(h, DH_WS_SPLITN, sizeof(double) * (size_t)mb * l * splits);
+        if (!P) return DH_ERR_ALLOC;
+    }
+    const d2v* Opk = nullptr;
+    DH_CHECK_STATUS(pack_omega_f64(h, n, l, groups * ncb, O, ldo, yj, &Opk));
+    const bool sym = keep && Xi == Xj && ldxi == ldxj && m == n && ni == nj;
+    dh_timing_begin(h);
+    for (int i0 = 0; i0 < m; i0 += mb) {
+        const int ib = std::min(mb, m - i0), bt = dh_cdiv(ib, 64), jt = dh_cdiv(n, 64);
+        if (kmode != 2) {
+            if (sym)
+                form_f64_kernel<true><<<(unsigned)((long)bt * (bt + 1) / 2), 256, 0, h->stream>>>(
+                    ib, n, d, Xi, ldxi, Xj, ldxj, ni, nj, gamma, (d2v*)Kb, 4 * bt);
+            else
+                form_f64_kernel<false><<<dim3(jt, bt), 256, 0, h->stream>>>(
+                    ib, n, d, Xi + (size_t)i0 * ldxi, ldxi, Xj, ldxj, ni + i0, nj, gamma,
+                    (d2v*)Kb, 4 * bt);
+            DH_CHECK_LAUNCH();
+        }
+        const double* y0 = yi ? yi + i0 : nullptr;
+        const long ystride = (long)ib * l;
+        DH_CHECK_STATUS(launch_kept_f64(h, ib, n, l, ncb, groups, y0, Opk, direct ? Y + i0 : P,
+                                        direct ? ldy : ib, jps, splits, ystride, Kb));
+        if (!direct) {
+            sum_splits_f64_kernel<<<dh_cdiv(ystride, 256), 256, 0, h->stream>>>(
+                ib, l, splits, P, ystride, beta, Y + i0, ldy);
+            DH_CHECK_LAUNCH();
+        }
+    }
+    dh_timing_end(h);
+    return 0;
+}
+
+// Bytes that dh_project_f64_split needs to keep K (m x n).
+size_t dh_kkeep_bytes(int m, int n) {
+    return kept_bytes(m, n);
 }
 
 // Y (m x l) = K(Xi, Xj) O + beta Y with the fused kernel, the j range in
@@ -653,20 +783,6 @@ int dh_project_f64_impl(dh_handle_t h, int m, int n, int d, int l, const double*
                              beta, Y, ldy, ncb, groups, n, 1, 0, pack, nullptr);
 }
 
-// Y = beta Y + sum over the splits z (in order) of P[z ystride + i + c m].
-__global__ __launch_bounds__(256) void sum_splits_f64_kernel(int m, int l, int splits,
-                                                             const double* __restrict__ P,
-                                                             long ystride, double beta,
-                                                             double* __restrict__ Y, int ldy) {
-    const long e = (long)blockIdx.x * 256 + threadIdx.x;
-    if (e >= (long)m * l) return;
-    const int i = (int)(e % m), c = (int)(e / m);
-    double v = 0.0;
-    for (int z = 0; z < splits; ++z) v += P[z * ystride + e];
-    double* yp = Y + i + (size_t)c * ldy;
-    *yp = (beta == 0.0) ? v : v + beta * (*yp);
-}
-
 // Y = K O as dh_project_f64_impl with beta = 0; a grid of at most half a
 // workgroup per CU splits the j range over more workgroups (partials in a
 // workspace, summed in order).  The range finder's passes use it;
@@ -683,7 +799,7 @@ int dh_project_f64_split(dh_handle_t h, int m, int n, int d, int l, const double
                                    ldo, 0.0, Y, ldy, true);
     if (d > 256)
         return project_f64_blocked(h, m, n, d, l, Xi, ldxi, Xj, ldxj, ni, nj, yi, yj, gamma, O,
-                                   ldo, 0.0, Y, ldy, (double*)keep, kmode);
+                                   ldo, 0.0, Y, ldy, keep, kmode);
     int ncb, groups;
     f64_columns(d, l, &ncb, &groups);
     const int nch = dh_cdiv(n, 32);
