@@ -75,6 +75,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(int m, int n, int ns
     int i = (int)(idx % m), j = (int)(idx / m);
     if (uplo_upper && i > j) return;
     T s = 0;
+#pragma unroll 16
     for (int z = 0; z < nsplit; ++z) s += part[(size_t)z * mn + idx];
     T* c = C + i + (size_t)j * ldc;
     *c = (beta == T(0)) ? alpha * s : alpha * s + beta * (*c);
@@ -93,10 +94,13 @@ static int launch_gemm(dh_handle_t h, bool ta, bool tb, int m, int n, int k, T a
     }
     int nsplit = 1;
     // Tall-skinny products (CholeskyQR Gram, TRSM updates with short outputs)
-    // have few output tiles and a long k: split k for ~4 workgroups per CU.
+    // have few output tiles and a long k: split k for ~4 workgroups per CU, up
+    // to 64 parts of at least 256, or of 64 with up to four tiles, where a
+    // part's steps are one round trip to memory after the other (Gram of 2051 x
+    // 42: GRAM_US).
     if (tiles < 4L * h->num_cu && k >= 1024) {
         nsplit = (int)((4L * h->num_cu + tiles - 1) / tiles);
-        nsplit = min(nsplit, k / 256);
+        nsplit = min(nsplit, k / (tiles <= 4 ? 64 : 256));
         nsplit = max(nsplit, 1);
         nsplit = min(nsplit, 64);
     }
