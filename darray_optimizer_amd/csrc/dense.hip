@@ -97,7 +97,7 @@ static int launch_gemm(dh_handle_t h, bool ta, bool tb, int m, int n, int k, T a
     // have few output tiles and a long k: split k for ~4 workgroups per CU, up
     // to 64 parts of at least 256, or of 64 with up to four tiles, where a
     // part's steps are one round trip to memory after the other (Gram of 2051 x
-    // 42: GRAM_US).
+    // 42: 19.4 + 4.3 us for the sum with 8 parts, 8.0 + 4.8 with 32).
     if (tiles < 4L * h->num_cu && k >= 1024) {
         nsplit = (int)((4L * h->num_cu + tiles - 1) / tiles);
         nsplit = min(nsplit, k / (tiles <= 4 ? 64 : 256));

@@ -246,7 +246,10 @@ int dh_cholqr2_f64(dh_handle_t h, int m, int n, double* Y, int ldy, double* R, i
  * replaced by pseudo-random ones, so Q always has l orthonormal columns
  * spanning range(Y) and more (as the reference's Householder QR would).
  * Above 256 features every `prec` runs the FP64 passes (the low-precision
- * kernels hold d <= 256).  Synchronises. */
+ * kernels hold d <= 256).  K is kept between the passes where that pays, in a
+ * buffer of up to an eighth of the device's memory that the process's handles
+ * share and that goes back with the last of them; where it cannot be had, every
+ * pass forms K and the results are the same.  Synchronises. */
 int dh_lra(dh_handle_t h, int prec, int n, int d, int l, int q, const double* X, int ldx,
            const double* y, double gamma, const double* Omega, int ldo, double* Q, int ldq,
            double* W, int ldw);
