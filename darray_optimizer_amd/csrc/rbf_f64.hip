@@ -214,19 +214,13 @@ __global__ __launch_bounds__(256) void pack_omega_f64_kernel(int n, int l, int n
     Opk[idx] = v;
 }
 
-// KEEP: column group 0 also stores every wave's K values (labels left out) to
-// Kk as the projection MFMAs take them, for kept_project_f64_kernel: 128 pairs
-// per (16-point chunk, 16-row block), pair h 64 + L = (kv[2h], kv[2h + 1]) of
-// lane L; nrb row blocks per chunk.  Chunks are outermost because all waves
-// walk them together: the reads and writes of any moment lie side by side.
-template <int DK, int NCB, bool PK, bool KEEP>
+template <int DK, int NCB, bool PK>
 __global__ __launch_bounds__(256) void rbf_project_f64_kernel(
     int m, int n, int d, int l, const double* __restrict__ Xi, int ldxi,
     const double* __restrict__ Xj, int ldxj, const double* __restrict__ ni,
     const double* __restrict__ nj, const double* __restrict__ yi, const double* __restrict__ yj,
     double gamma, const double* __restrict__ O, int ldo, const d2v* __restrict__ Opk, int ncbp,
-    double beta, double* __restrict__ Y, int ldy, int jps, long ystride, d2v* __restrict__ Kk,
-    int nrb) {
+    double beta, double* __restrict__ Y, int ldy, int jps, long ystride) {
     constexpr int JB = 16;
     {  // split z of the j range: points [z jps, min((z + 1) jps, n)), partial into Y + z ystride
         const int j0 = blockIdx.z * jps;
@@ -236,7 +230,6 @@ __global__ __launch_bounds__(256) void rbf_project_f64_kernel(
         if (yj) yj += j0;
         O += j0;
         if (PK) Opk += (size_t)(j0 / JB) * ncbp * 128;
-        if (KEEP) Kk += ((size_t)(j0 / JB) * nrb + blockIdx.x * 4 + (threadIdx.x >> 6)) * 128;
         Y += blockIdx.z * ystride;
     }
     constexpr int FD = DK * 4;  // padded feature count
@@ -341,11 +334,6 @@ __global__ __launch_bounds__(256) void rbf_project_f64_kernel(
             d2 = d2 > 0.0 ? d2 : 0.0;
             kv[r] = exp_kernel_f64(-gamma * d2);
         }
-        if (KEEP && blockIdx.y == 0) {
-            d2v* kp = Kk + (size_t)(j0 / JB) * nrb * 128 + lane;
-            kp[0] = d2v{kv[0], kv[1]};
-            kp[64] = d2v{kv[2], kv[3]};
-        }
         const int sl = lane ^ ((lane >> 4) << 2);
 #pragma unroll
         for (int cb = 0; cb < NCB; ++cb) {
@@ -374,8 +362,115 @@ __global__ __launch_bounds__(256) void rbf_project_f64_kernel(
         }
 }
 
-// K without labels in the layout of a KEEP pass, for points of any number of
-// features: 64 x 64 distance tiles (tile_mma) with the points of the columns as
+// The kept layout: K without labels as the projection MFMAs take it, 128 pairs
+// per (16-point chunk, 16-row block), pair h 64 + L = (kv[2h], kv[2h + 1]) of
+// lane L with kv as in rbf_project_f64_kernel; nrb row blocks per chunk.  Chunks
+// are outermost because all waves walk them together: the reads and writes of
+// any moment lie side by side.
+
+// Stores block (row block rb, chunk t) of K in the kept layout and, with
+// `mirror`, the transposed block (t, rb) through the wave's 16 x 17 of LDS.
+__device__ __forceinline__ void store_kept(double (&kv)[4], int rb, int t, int nch, int nrb,
+                                           bool mirror, double (*sT)[17], d2v* __restrict__ Kk) {
+    const int lane = threadIdx.x & 63, g = lane >> 4, li = lane & 15;
+    if (t < nch) {  // row blocks are padded to whole tiles, chunks are not
+        d2v* kp = Kk + ((size_t)t * nrb + rb) * 128 + lane;
+        kp[0] = d2v{kv[0], kv[1]};
+        kp[64] = d2v{kv[2], kv[3]};
+    }
+    if (!mirror) return;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) sT[4 * r + g][li] = kv[r];
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int r = 0; r < 4; ++r) kv[r] = sT[li][4 * r + g];
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (rb < nch) {
+        d2v* kp = Kk + ((size_t)rb * nrb + t) * 128 + lane;
+        kp[0] = d2v{kv[0], kv[1]};
+        kp[64] = d2v{kv[2], kv[3]};
+    }
+}
+
+// K of one point set with up to 4 DK features, in the kept layout and with the
+// fused kernel's bits: its distance stage (products, exp) on one triangle of
+// 64 x 64 tiles, whose strict part is stored a second time transposed; products
+// and norms commute.  Workgroup (bi, z): 64 rows, the part of points [64 z seg,
+// 64 (z + 1) seg) from row tile bi on.  n = 65536, d = 128: 14.2 ms, 39 TFLOP/s beside
+// 34 GB of writes (a fused pass that stores K as it goes takes 29.5 ms more than
+// a kept one); n = 8192, d = 64: 0.166 ms against 0.31.
+template <int DK>
+__global__ __launch_bounds__(256) void form_sym_f64_kernel(int n, int d,
+                                                           const double* __restrict__ X, int ldx,
+                                                           const double* __restrict__ nrm,
+                                                           double gamma, int seg,
+                                                           d2v* __restrict__ Kk, int nrb) {
+    constexpr int JB = 16, FD = DK * 4, XP = FD + 2;
+    __shared__ double sX[2][JB * XP];
+    __shared__ double sN[2][JB];
+    __shared__ double sT[4][16][17];
+    const int bi = blockIdx.x, nt = gridDim.x;
+    const int tb = max((int)blockIdx.y * seg, bi), te = min(((int)blockIdx.y + 1) * seg, nt);
+    if (tb >= te) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, li = lane & 15;
+    const int rb = 4 * bi + wave, row = 16 * rb + li, nch = (n + JB - 1) / JB;
+    double xr[DK];
+#pragma unroll
+    for (int kk = 0; kk < DK; ++kk) {
+        const int f = g * DK + kk;
+        xr[kk] = (row < n && f < d) ? X[f + (size_t)row * ldx] : 0.0;
+    }
+    const double nrow = (row < n) ? nrm[row] : 0.0;
+    constexpr int NXL = JB * FD / 256;
+    double px[NXL], pn;
+    auto load = [&](int j0) {
+#pragma unroll
+        for (int u = 0; u < NXL; ++u) {
+            const int e = tid + 256 * u, jj = e / FD, f = e % FD;
+            px[u] = X[min(f, d - 1) + (size_t)min(j0 + jj, n - 1) * ldx];
+        }
+        pn = nrm[min(j0 + (tid % JB), n - 1)];
+    };
+    auto store = [&](int j0, int b) {
+#pragma unroll
+        for (int u = 0; u < NXL; ++u) {
+            const int e = tid + 256 * u, jj = e / FD, f = e % FD;
+            sX[b][jj * XP + f] = (j0 + jj < n && f < d) ? px[u] : 0.0;
+        }
+        if (tid < JB) sN[b][tid] = (j0 + tid < n) ? pn : 0.0;
+    };
+    load(64 * tb);
+    store(64 * tb, 0);
+    __syncthreads();
+    int b = 0;
+    for (int t = 4 * tb; t < 4 * te; ++t) {
+        const bool more = t + 1 < 4 * te;  // uniform
+        if (more) load(JB * (t + 1));
+        dh_d4 s0 = dh_d4{0, 0, 0, 0}, s1 = dh_d4{0, 0, 0, 0};
+        const double* xrow = &sX[b][li * XP + g * DK];
+#pragma unroll
+        for (int kk = 0; kk < DK; kk += 2) {
+            const d2v a2 = *(const d2v*)(xrow + kk);
+            s0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a2[0], xr[kk], s0, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a2[1], xr[kk + 1], s1, 0, 0, 0);
+        }
+        double kv[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            double d2 = nrow + sN[b][g + 4 * r] - 2.0 * (s0[r] + s1[r]);
+            d2 = d2 > 0.0 ? d2 : 0.0;
+            kv[r] = exp_kernel_f64(-gamma * d2);
+        }
+        store_kept(kv, rb, t, nch, nrb, (t >> 2) != bi, sT[wave], Kk);
+        if (more) store(JB * (t + 1), b ^ 1);
+        __syncthreads();
+        b ^= 1;
+    }
+}
+
+// K without labels in the kept layout, for points of any number of features: 64 x 64 distance tiles (tile_mma) with the points of the columns as
 // tile rows, so that the accumulators of lane (g, li) are already its pairs.
 // SYM (Xi = Xj): one triangle of tiles, of which the strict part is stored a
 // second time with every 16 x 16 block transposed through LDS; the products
@@ -418,32 +513,13 @@ __global__ __launch_bounds__(256) void form_f64_kernel(int m, int n, int d,
                 d2 = d2 > 0.0 ? d2 : 0.0;
                 kv[r] = exp(-gamma * d2);
             }
-            if (t < nch) {  // row blocks are padded to whole tiles, chunks are not
-                d2v* kp = Kk + ((size_t)t * nrb + rb) * 128 + lane;
-                kp[0] = d2v{kv[0], kv[1]};
-                kp[64] = d2v{kv[2], kv[3]};
-            }
-            if (SYM && bi != bj) {  // block (rb, t) transposed: row block t, chunk rb
-#pragma unroll
-                for (int r = 0; r < 4; ++r) sT[wave][4 * r + g][li] = kv[r];
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-#pragma unroll
-                for (int r = 0; r < 4; ++r) kv[r] = sT[wave][li][4 * r + g];
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                if (rb < nch) {
-                    d2v* kp = Kk + ((size_t)rb * nrb + t) * 128 + lane;
-                    kp[0] = d2v{kv[0], kv[1]};
-                    kp[64] = d2v{kv[2], kv[3]};
-                }
-            }
+            store_kept(kv, rb, t, nch, nrb, SYM && bi != bj, sT[wave], Kk);
         }
 }
 
-// Y = K O from the K values that a KEEP pass stored, with that pass's packed
-// Omega image, chunk order and MFMAs, so it returns the bits that the fused
-// kernel would.  Rows, columns and splits as there; what is gone is the
+// Y = K O from K values in the kept layout, with the packed Omega image, chunk
+// order and MFMAs of the fused kernel, so it returns that kernel's bits where
+// the values are its values.  Rows, columns and splits as there; what is gone is the
 // distance product (2d of the 2(d + l) flops per entry), the exp, and the
 // staging of X, and with it the registers and LDS that held the fused kernel
 // to one workgroup per CU at l = 272: here two fit.  K comes from HBM once per
@@ -516,21 +592,17 @@ static void launch_project_f64(dh_handle_t h, dim3 grid, int m, int n, int d, in
                                const double* ni, const double* nj, const double* yi,
                                const double* yj, double gamma, const double* O, int ldo,
                                const d2v* Opk, int ncbp, double beta, double* Y, int ldy, int jps,
-                               long ystride, d2v* Kk) {
+                               long ystride) {
     if constexpr (DK < 64 || NCB <= 12) {  // d > 128 with 17 blocks is never selected (spills)
         dh_timing_begin(h);
-        if (Opk && Kk)
-            rbf_project_f64_kernel<DK, NCB, true, true><<<grid, 256, 0, h->stream>>>(
+        if (Opk)
+            rbf_project_f64_kernel<DK, NCB, true><<<grid, 256, 0, h->stream>>>(
                 m, n, d, l, Xi, ldxi, Xj, ldxj, ni, nj, yi, yj, gamma, O, ldo, Opk, ncbp, beta, Y,
-                ldy, jps, ystride, Kk, 4 * grid.x);
-        else if (Opk)
-            rbf_project_f64_kernel<DK, NCB, true, false><<<grid, 256, 0, h->stream>>>(
-                m, n, d, l, Xi, ldxi, Xj, ldxj, ni, nj, yi, yj, gamma, O, ldo, Opk, ncbp, beta, Y,
-                ldy, jps, ystride, nullptr, 0);
+                ldy, jps, ystride);
         else
-            rbf_project_f64_kernel<DK, NCB, false, false><<<grid, 256, 0, h->stream>>>(
+            rbf_project_f64_kernel<DK, NCB, false><<<grid, 256, 0, h->stream>>>(
                 m, n, d, l, Xi, ldxi, Xj, ldxj, ni, nj, yi, yj, gamma, O, ldo, nullptr, 0, beta, Y,
-                ldy, jps, ystride, nullptr, 0);
+                ldy, jps, ystride);
         dh_timing_end(h);
     }
 }
@@ -540,11 +612,11 @@ static int dispatch_ncb(dh_handle_t h, int ncb, dim3 grid, int m, int n, int d, 
                         const double* Xi, int ldxi, const double* Xj, int ldxj, const double* ni,
                         const double* nj, const double* yi, const double* yj, double gamma,
                         const double* O, int ldo, const d2v* Opk, int ncbp, double beta,
-                        double* Y, int ldy, int jps, long ystride, d2v* Kk) {
+                        double* Y, int ldy, int jps, long ystride) {
 #define DH_NCB(N)                                                                              \
     case N:                                                                                    \
         launch_project_f64<DK, N>(h, grid, m, n, d, l, Xi, ldxi, Xj, ldxj, ni, nj, yi, yj, gamma, \
-                                  O, ldo, Opk, ncbp, beta, Y, ldy, jps, ystride, Kk);          \
+                                  O, ldo, Opk, ncbp, beta, Y, ldy, jps, ystride);              \
         break;
     switch (ncb) {
         DH_NCB(1)
@@ -740,15 +812,14 @@ static int project_f64_fused(dh_handle_t h, int m, int n, int d, int l, const do
                              int ldxi, const double* Xj, int ldxj, const double* ni,
                              const double* nj, const double* yi, const double* yj, double gamma,
                              const double* O, int ldo, double beta, double* Y, int ldy, int ncb,
-                             int groups, int jps, int splits, long ystride, bool pack,
-                             void* keep) {
+                             int groups, int jps, int splits, long ystride, bool pack) {
     dim3 grid(dh_cdiv(m, 64), groups, splits);
     const d2v* Opk = nullptr;
     const int ncbp = groups * ncb;
     if (pack) DH_CHECK_STATUS(pack_omega_f64(h, n, l, ncbp, O, ldo, yj, &Opk));
 #define DH_DK(K)                                                                              \
     dispatch_ncb<K>(h, ncb, grid, m, n, d, l, Xi, ldxi, Xj, ldxj, ni, nj, yi, yj, gamma, O, ldo, \
-                    Opk, ncbp, beta, Y, ldy, jps, ystride, (d2v*)keep)
+                    Opk, ncbp, beta, Y, ldy, jps, ystride)
     if (d <= 32) return DH_DK(8);
     if (d <= 64) return DH_DK(16);
     if (d <= 128) return DH_DK(32);
@@ -780,15 +851,41 @@ int dh_project_f64_impl(dh_handle_t h, int m, int n, int d, int l, const double*
     int ncb, groups;
     f64_columns(d, l, &ncb, &groups);
     return project_f64_fused(h, m, n, d, l, Xi, ldxi, Xj, ldxj, ni, nj, yi, yj, gamma, O, ldo,
-                             beta, Y, ldy, ncb, groups, n, 1, 0, pack, nullptr);
+                             beta, Y, ldy, ncb, groups, n, 1, 0, pack);
+}
+
+// K of one point set (d <= 256) in the kept layout.  Segments of up to 16 row
+// tiles, fewer while that leaves less than four workgroups per CU.
+static int form_sym_f64(dh_handle_t h, int n, int d, const double* X, int ldx, const double* nrm,
+                        double gamma, void* keep) {
+    const int nt = dh_cdiv(n, 64);
+    int seg = 16;
+    while (seg > 1 && (long)nt * nt / (2 * seg) < 4L * h->num_cu) seg /= 2;
+    const dim3 grid(nt, dh_cdiv(nt, seg));
+    dh_timing_begin(h);
+#define DH_FORM(DK)                                                                           \
+    form_sym_f64_kernel<DK><<<grid, 256, 0, h->stream>>>(n, d, X, ldx, nrm, gamma, seg,       \
+                                                         (d2v*)keep, 4 * nt)
+    if (d <= 32)
+        DH_FORM(8);
+    else if (d <= 64)
+        DH_FORM(16);
+    else if (d <= 128)
+        DH_FORM(32);
+    else
+        DH_FORM(64);
+#undef DH_FORM
+    dh_timing_end(h);
+    DH_CHECK_LAUNCH();
+    return 0;
 }
 
 // Y = K O as dh_project_f64_impl with beta = 0; a grid of at most half a
 // workgroup per CU splits the j range over more workgroups (partials in a
 // workspace, summed in order).  The range finder's passes use it;
 // dh_rbf_project_f64 keeps the one-launch form, so its allocation-free twin
-// returns the same bits.  kmode 1 also stores K to `keep` (dh_kkeep_bytes), and
-// kmode 2 takes it from there instead of forming it: same points, same bits.
+// returns the same bits.  With `keep` (dh_kkeep_bytes; one point set, Xi = Xj)
+// K is formed there first (kmode 1) or taken from there (kmode 2): same bits.
 int dh_project_f64_split(dh_handle_t h, int m, int n, int d, int l, const double* Xi, int ldxi,
                          const double* Xj, int ldxj, const double* ni, const double* nj,
                          const double* yi, const double* yj, double gamma, const double* O,
@@ -813,13 +910,14 @@ int dh_project_f64_split(dh_handle_t h, int m, int n, int d, int l, const double
         if (!P) return DH_ERR_ALLOC;
         ldp = m;
     }
-    if (keep && kmode == 2)
+    if (keep && kmode == 1) DH_CHECK_STATUS(form_sym_f64(h, n, d, Xi, ldxi, ni, gamma, keep));
+    if (keep)
         DH_CHECK_STATUS(project_f64_kept(h, m, n, l, yi, yj, O, ldo, P, ldp, jps, splits, ystride,
                                          keep));
     else
         DH_CHECK_STATUS(project_f64_fused(h, m, n, d, l, Xi, ldxi, Xj, ldxj, ni, nj, yi, yj,
                                           gamma, O, ldo, 0.0, P, ldp, ncb, groups, jps, splits,
-                                          ystride, true, keep));
+                                          ystride, true));
     if (splits == 1) return 0;
     sum_splits_f64_kernel<<<dh_cdiv(ystride, 256), 256, 0, h->stream>>>(m, l, splits, P, ystride,
                                                                         0.0, Y, ldy);
