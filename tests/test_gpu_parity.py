@@ -610,9 +610,9 @@ def test_cholqr2_reports_the_failing_pivot(dev, bad):
                                           (2051, 130, 200, True), (900, 70, 280, False),
                                           (300, 257, 20, True), (11700, 257, 3, False)])
 def test_lra_passes_on_kept_kernel_values(dev, n, d, l, labels):
-    """The FP64 range finder's later passes take K from the values its first
-    pass stored: W must be K Q for the returned Q, as the one-launch pass
-    forms it.  Both sum n products K_ij Q_jc, in different orders, so element
+    """The FP64 range finder forms K once, from one triangle, and all its passes
+    read it back: W must be K Q for the returned Q, as the one-launch pass forms
+    it.  Both sum n products K_ij Q_jc, in different orders, so element
     (i, c) may differ by 2 n u (K |Q|)_ic; K is in (0, 1]."""
     import torch
     rng = np.random.default_rng(n + d)
