@@ -1178,8 +1178,9 @@ __global__ __launch_bounds__(512) void lra_error_sym_kernel(
             add(se, le, ts);
         }
     }
-    se += le;
-    sk += lk;
+    // The error of an infinite sum is NaN: the sum stands without it.
+    se += le == le ? le : 0.0;
+    sk += lk == lk ? lk : 0.0;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
         se += __shfl_xor(se, o);

@@ -711,3 +711,33 @@ def test_lra_error_on_symmetric_tiles(dev, n, d, l, labels):
     ref_e, ref_k = float((E * E).sum()), float((K * K).sum())
     assert abs(e2 - ref_e) <= 2 * float(E.norm() * D.norm()) + 1e-14 * ref_e
     assert abs(k2 - ref_k) <= (4 * kerr + 1e-14) * ref_k
+
+
+@pytest.mark.parametrize("n", [500, 6500])
+@pytest.mark.parametrize("what,err,norm", [("inf in W", "inf", "finite"),
+                                           ("overflow in W", "inf", "finite"),
+                                           ("nan in Q", "nan", "finite"),
+                                           ("inf in y", "inf", "inf")])
+def test_lra_error_of_non_finite_input(dev, n, what, err, norm):
+    """One infinite entry, or one whose square overflows, makes the sum infinite
+    and not NaN, on the tiles of the whole matrix and on those of one triangle
+    (6500); a NaN stays a NaN, and the other sum is not touched."""
+    import math
+
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(n)
+    X = torch.randn((n, 24), dtype=torch.float64, device="cuda", generator=g) / 24**0.5
+    Q, W = (torch.randn((20, n), dtype=torch.float64, device="cuda", generator=g) for _ in range(2))
+    y = torch.ones(n, dtype=torch.float64, device="cuda")
+    _, clean = dev.lra_error(X, 0.7, Q, W, y=y)
+    if what == "inf in W":
+        W[3, n - 2] = -math.inf
+    elif what == "overflow in W":
+        W[3, n // 2] = 1e200
+    elif what == "nan in Q":
+        Q[0, 5] = math.nan
+    else:
+        y[n - 1] = math.inf
+    e2, k2 = dev.lra_error(X, 0.7, Q, W, y=y)
+    assert math.isnan(e2) if err == "nan" else e2 == math.inf
+    assert k2 == (math.inf if norm == "inf" else clean)
