@@ -731,6 +731,14 @@ static size_t kept_bytes(int m, int n) {
     return sizeof(double) * ((size_t)dh_cdiv(m, 64) * 64) * ((size_t)dh_cdiv(n, 16) * 16);
 }
 
+// Rows of a block of K (n columns): at most 2^27 entries as laid out, with the
+// columns padded to whole chunks, and at most the 65535 row tiles that the y
+// dimension of form_f64_kernel's grid holds (n <= 31).
+static int block_rows(int n) {
+    const long fit = (1L << 27) / ((n + 15L) / 16 * 16) / 64 * 64;
+    return (int)std::min(64L * 65535, std::max(64L, fit));
+}
+
 // Above 256 features a wave's rows of Xi no longer fit in registers.  K is then
 // formed in the kept layout by distance tiles, in row blocks of at most 2^27
 // entries (1 GiB), and each block multiplied into Omega by
@@ -748,8 +756,7 @@ static int project_f64_blocked(dh_handle_t h, int m, int n, int d, int l, const 
                                void* keep, int kmode) {
     if (n == 0)  // K has no columns: Y = beta Y
         return dh_gemm_impl<double>(h, false, false, m, l, 0, 1.0, O, 1, O, ldo, beta, Y, ldy, 0);
-    const long cap = 1L << 27;
-    const int mb = keep ? m : (int)std::min<long>(m, std::max<long>(64, cap / n / 64 * 64));
+    const int mb = keep ? m : std::min(m, block_rows(n));
     void* Kb = keep ? keep : dh_ws(h, DH_WS_KBLOCK, kept_bytes(mb, n));
     if (!Kb) return DH_ERR_ALLOC;
     int ncb, groups;

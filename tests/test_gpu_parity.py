@@ -741,3 +741,27 @@ def test_lra_error_of_non_finite_input(dev, n, what, err, norm):
     e2, k2 = dev.lra_error(X, 0.7, Q, W, y=y)
     assert math.isnan(e2) if err == "nan" else e2 == math.inf
     assert k2 == (math.inf if norm == "inf" else clean)
+
+
+@pytest.mark.slow
+def test_rbf_project_f64_wide_with_very_many_rows(dev):
+    """More row tiles than the y dimension of a grid holds (65535 of 64 rows) at
+    d > 256, which few column points allow.  Rows at the ends and around the
+    first block's end against plain FP64; an entry's distance product is off by
+    at most (d + 4) u 4 s, s the largest squared norm, on either side, which
+    the exponential turns into gamma times that, relative."""
+    import torch
+    m, n, d, l, gamma, u = 64 * 65535 + 100, 3, 257, 2, 0.7, 2.0**-53
+    g = torch.Generator(device="cuda").manual_seed(m)
+    X = torch.rand((m, d), dtype=torch.float64, device="cuda", generator=g).div_(d**0.5)
+    O = torch.randn((l, n), dtype=torch.float64, device="cuda", generator=g)
+    Y = torch.full((l, m), 7.0, dtype=torch.float64, device="cuda")
+    dev.rbf_project_f64(X, X[:n], O, gamma, Y)
+    b = 64 * 65535
+    rows = torch.tensor([0, 1, 63, 64, b // 2, b - 1, b, b + 1, m - 2, m - 1], device="cuda")
+    A, B = X[rows], X[:n]
+    K = torch.exp(-gamma * (A[:, None, :] - B[None, :, :]).pow(2).sum(2))
+    ref = K @ O.t().contiguous()
+    tol = 2 * (gamma * 4 * (d + 4) + n + 4) * u * float(O.abs().sum(1).max())
+    assert float((Y[:, rows].t() - ref).abs().max()) <= tol  # s <= 1
+    assert bool((Y != 7.0).all())
