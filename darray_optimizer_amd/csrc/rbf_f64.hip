@@ -668,17 +668,16 @@ static void kept_columns(int l, int* ncb, int* groups) {
     *groups = dh_cdiv(ncb_total, *ncb);
 }
 
-// Y (m x l) = K O from K values in the kept layout, Omega packed in ncb x groups
-// column blocks.
+// Y (m x l) = K O from K values in the kept layout (nrb row blocks per chunk),
+// Omega packed in ncb x groups column blocks.
 static int launch_kept_f64(dh_handle_t h, int m, int n, int l, int ncb, int groups,
                            const double* yi, const d2v* Opk, double* Y, int ldy, int jps,
-                           int splits, long ystride, const void* keep) {
+                           int splits, long ystride, const void* keep, int nrb) {
     dim3 grid(dh_cdiv(m, 64), groups, splits);
 #define DH_NCB(N)                                                                         \
     case N:                                                                               \
         kept_project_f64_kernel<N><<<grid, 256, 0, h->stream>>>(                          \
-            m, n, l, (const d2v*)keep, 4 * grid.x, yi, Opk, groups* ncb, Y, ldy, jps,     \
-            ystride);                                                                     \
+            m, n, l, (const d2v*)keep, nrb, yi, Opk, groups* ncb, Y, ldy, jps, ystride);  \
         break;
     switch (ncb) {
         DH_NCB(1)
@@ -707,7 +706,7 @@ static int project_f64_kept(dh_handle_t h, int m, int n, int l, const double* yi
     DH_CHECK_STATUS(pack_omega_f64(h, n, l, groups * ncb, O, ldo, yj, &Opk));
     dh_timing_begin(h);
     DH_CHECK_STATUS(launch_kept_f64(h, m, n, l, ncb, groups, yi, Opk, Y, ldy, jps, splits, ystride,
-                                    keep));
+                                    keep, 4 * dh_cdiv(m, 64)));
     dh_timing_end(h);
     return 0;
 }
@@ -731,12 +730,14 @@ static size_t kept_bytes(int m, int n) {
     return sizeof(double) * ((size_t)dh_cdiv(m, 64) * 64) * ((size_t)dh_cdiv(n, 16) * 16);
 }
 
-// Rows of a block of K (n columns): at most 2^27 entries as laid out, with the
-// columns padded to whole chunks, and at most the 65535 row tiles that the y
-// dimension of form_f64_kernel's grid holds (n <= 31).
-static int block_rows(int n) {
+// Rows per block of K (m x n): equal blocks of at most 2^27 entries as laid out,
+// with the columns padded to whole chunks, and of at most 65535 row tiles, which
+// lie in the y dimension of form_f64_kernel's grid (its customary limit, reached
+// with n <= 31; ROCm 7.2 launched 65538 all the same).
+static int block_rows(int m, int n) {
     const long fit = (1L << 27) / ((n + 15L) / 16 * 16) / 64 * 64;
-    return (int)std::min(64L * 65535, std::max(64L, fit));
+    const int most = (int)std::min(64L * 65535, std::max(64L, fit));
+    return dh_cdiv(dh_cdiv(m, dh_cdiv(m, most)), 64) * 64;
 }
 
 // Above 256 features a wave's rows of Xi no longer fit in registers.  K is then
@@ -745,10 +746,15 @@ static int block_rows(int n) {
 // kept_project_f64_kernel.  The same split as rbf_kernel's explicit tiles
 // (dkernel.cu:144-178).  With `keep` K is one block there: kmode 1 forms it,
 // from one triangle where both point sets are the same; kmode 2 takes it as an
-// earlier pass left it.  The j range is split until there are two workgroups
-// per CU, by the whole m, so blocks and splits return the same bits.  (Column-
-// major blocks through the 64 x 64 GEMM: n = 9000, d = 600, l = 74 took 2.13 + 0.49
-// ms per pass; forming one triangle takes 1.07 and a pass 0.33.)
+// earlier pass left it.  The j range is split until a row block has two
+// workgroups per CU, also where K is kept, so that both return the same bits.
+// (Column-major blocks through the 64 x 64 GEMM: n = 9000, d = 600, l = 74 took
+// 2.13 + 0.49 ms per pass; forming one triangle takes 1.07 and a pass 0.33.
+// One pass over row blocks, d = 300, l = 74, GEMM -> here, and with the split
+// chosen from all m rows: n = 40000 30.2 -> 26.0 and 57.8 ms, n = 65536 76.9 -> 69.8
+// and 203 ms, 300 x 500000 3.8 -> 3.4 and 11.5 ms.  With K kept the splits cost
+// 1% at n = 65536, l = 272 and gain 14% at n = 40000.)  The partial products take at
+// most 1 GiB, or 4 GiB beside a kept K, in parts of the rows.
 static int project_f64_blocked(dh_handle_t h, int m, int n, int d, int l, const double* Xi,
                                int ldxi, const double* Xj, int ldxj, const double* ni,
                                const double* nj, const double* yi, const double* yj, double gamma,
@@ -756,22 +762,24 @@ static int project_f64_blocked(dh_handle_t h, int m, int n, int d, int l, const 
                                void* keep, int kmode) {
     if (n == 0)  // K has no columns: Y = beta Y
         return dh_gemm_impl<double>(h, false, false, m, l, 0, 1.0, O, 1, O, ldo, beta, Y, ldy, 0);
-    const int mb = keep ? m : std::min(m, block_rows(n));
+    const int rows = std::min(m, block_rows(m, n)), mb = keep ? m : rows;
     void* Kb = keep ? keep : dh_ws(h, DH_WS_KBLOCK, kept_bytes(mb, n));
     if (!Kb) return DH_ERR_ALLOC;
     int ncb, groups;
     kept_columns(l, &ncb, &groups);
     const int nch = dh_cdiv(n, 32);
     int splits = 1;
-    while (splits < 8 && (long)dh_cdiv(m, 64) * groups * splits < 2L * h->num_cu &&
-           nch >= 32 * splits)
+    while ((long)dh_cdiv(rows, 64) * groups * splits < 2L * h->num_cu && nch >= 32 * splits)
         splits *= 2;
     const int jps = splits == 1 ? n : dh_cdiv(nch, splits) * 32;
     splits = dh_cdiv(n, jps);
     const bool direct = splits == 1 && beta == 0.0;
     double* P = nullptr;
+    int pr = mb;  // rows per launch
     if (!direct) {
-        P = (double*)dh_ws(h, DH_WS_SPLITN, sizeof(double) * (size_t)mb * l * splits);
+        const long fit = (keep ? 1L << 29 : 1L << 27) / ((long)l * splits) / 64 * 64;
+        pr = (int)std::min<long>(mb, std::max(64L, fit));
+        P = (double*)dh_ws(h, DH_WS_SPLITN, sizeof(double) * (size_t)pr * l * splits);
         if (!P) return DH_ERR_ALLOC;
     }
     const d2v* Opk = nullptr;
@@ -790,13 +798,17 @@ static int project_f64_blocked(dh_handle_t h, int m, int n, int d, int l, const 
                     (d2v*)Kb, 4 * bt);
             DH_CHECK_LAUNCH();
         }
-        const double* y0 = yi ? yi + i0 : nullptr;
-        const long ystride = (long)ib * l;
-        DH_CHECK_STATUS(launch_kept_f64(h, ib, n, l, ncb, groups, y0, Opk, direct ? Y + i0 : P,
-                                        direct ? ldy : ib, jps, splits, ystride, Kb));
-        if (!direct) {
+        for (int r0 = 0; r0 < ib; r0 += pr) {
+            const int rb = std::min(pr, ib - r0);
+            double* y0 = Y + i0 + r0;
+            const long ystride = (long)rb * l;
+            DH_CHECK_STATUS(launch_kept_f64(h, rb, n, l, ncb, groups, yi ? yi + i0 + r0 : nullptr,
+                                            Opk, direct ? y0 : P, direct ? ldy : rb, jps, splits,
+                                            ystride, (const d2v*)Kb + (size_t)(r0 / 16) * 128,
+                                            4 * bt));
+            if (direct) continue;
             sum_splits_f64_kernel<<<dh_cdiv(ystride, 256), 256, 0, h->stream>>>(
-                ib, l, splits, P, ystride, beta, Y + i0, ldy);
+                rb, l, splits, P, ystride, beta, y0, ldy);
             DH_CHECK_LAUNCH();
         }
     }

@@ -102,9 +102,11 @@ int dh_rbf_tile_f32(dh_handle_t h, int m, int n, int d, const float* Xi, int ldx
 /* Fused Y[m x l] = K(Xi,Xj) * O[n x l] + beta*Y in FP64 (MFMA f64 for the distance
  * and the projection, FP64 exp).  K is never stored for d <= 256 (O, with yj folded
  * in, is first packed into a workspace of 8 * ceil(n/16) * 16 * 16 * ceil(l/16)
- * bytes in the kernel's operand order); above 256 features K is materialised in
- * row blocks of at most 2^27 entries (a 1 GiB workspace), as rbf_kernel does
- * (dkernel.cu:144-178), and multiplied into O by the FP64 GEMM.  Replaces the
+ * bytes in the kernel's operand order); above 256 features K is formed in row
+ * blocks of at most 2^27 entries, the columns counted in 16s (a 1 GiB workspace;
+ * 64 rows where n is larger than 2^21), as rbf_kernel does (dkernel.cu:144-178),
+ * and multiplied into O through the same packed copy, with partial products of
+ * up to 1 GiB where the j range is split or beta != 0.  Replaces the
  * rbf_kernel + replicate + tc_gemm sequence of DArray::LRA (dkernel.h:33-42). */
 int dh_rbf_project_f64(dh_handle_t h, int m, int n, int d, int l, const double* Xi, int ldxi,
                        const double* Xj, int ldxj, const double* yi, const double* yj,

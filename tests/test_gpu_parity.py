@@ -745,7 +745,7 @@ def test_lra_error_of_non_finite_input(dev, n, what, err, norm):
 
 @pytest.mark.slow
 def test_rbf_project_f64_wide_with_very_many_rows(dev):
-    """More row tiles than the y dimension of a grid holds (65535 of 64 rows) at
+    """More than 65535 row tiles of 64 rows, a grid's customary limit in y, at
     d > 256, which few column points allow.  Rows at the ends and around the
     first block's end against plain FP64; an entry's distance product is off by
     at most (d + 4) u 4 s, s the largest squared norm, on either side, which
@@ -765,3 +765,65 @@ def test_rbf_project_f64_wide_with_very_many_rows(dev):
     tol = 2 * (gamma * 4 * (d + 4) + n + 4) * u * float(O.abs().sum(1).max())
     assert float((Y[:, rows].t() - ref).abs().max()) <= tol  # s <= 1
     assert bool((Y != 7.0).all())
+
+
+@pytest.mark.parametrize("m,n,d,l,beta", [(130, 300000, 257, 20, 0.5), (700, 300000, 260, 3, 0.0),
+                                          (1, 70000, 300, 17, 1.0), (12000, 11500, 257, 290, 0.0),
+                                          (150000, 20, 257, 1000, -0.5)])
+def test_rbf_project_f64_wide_row_blocks(dev, m, n, d, l, beta):
+    """d > 256 with few and many rows against few and many columns: several row
+    blocks, many parts of the j range, partial products in several parts of the
+    rows.  Tolerance per element: n products and beta Y in any order, and K from
+    distances that are off by at most (d + 4) u 4 s, s <= 1 the largest squared
+    norm, on either side."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    Xi, Xj = (torch.rand((c, d), dtype=torch.float64, device="cuda", generator=g).div_(d**0.5)
+              for c in (m, n))
+    yi, yj = (1.0 - 2.0 * (torch.arange(c, device="cuda") % 3 == 0).double() for c in (m, n))
+    O = torch.randn((l, n), dtype=torch.float64, device="cuda", generator=g)
+    Y = torch.randn((l, m), dtype=torch.float64, device="cuda", generator=g)
+    gamma, u = 0.7, 2.0**-53
+    Y0 = Y.clone()
+    dev.rbf_project_f64(Xi, Xj, O, gamma, Y, yi=yi, yj=yj, beta=beta)
+    Ot = O.t().contiguous()
+    step = max(1, (1 << 27) // n)
+    for i in range(0, m, step):
+        A = Xi[i:i + step]
+        K = torch.exp(-gamma * ((A * A).sum(1)[:, None] + (Xj * Xj).sum(1)[None, :]
+                                - 2.0 * (A @ Xj.t())).clamp(min=0.0))
+        K = K * yi[i:i + step, None] * yj[None, :]
+        ref = K @ Ot + beta * Y0[:, i:i + step].t()
+        size = K.abs() @ Ot.abs() + abs(beta) * Y0[:, i:i + step].t().abs()
+        tol = 2 * (gamma * 4 * (d + 4) + n + 6) * u * size
+        assert bool(((Y[:, i:i + step].t() - ref).abs() <= tol).all())
+
+
+def test_rbf_project_f64_wide_fills_the_gpu_with_few_rows():
+    """The pass over a wide K (300 x 500000) does the work of the pass over its
+    transpose; with the j range split enough it takes about as long.  Partial
+    products (4.8 GB if they were held for all 600000 x 1000) and blocks of K stay
+    within 1 GiB each, and an eighth of headroom."""
+    import torch
+    h = dh.Handle(0)
+
+    def best(m, n, l):
+        Xi, Xj = (torch.rand((c, 300), dtype=torch.float64, device="cuda") for c in (m, n))
+        O = torch.rand((l, n), dtype=torch.float64, device="cuda")
+        Y = torch.zeros((l, m), dtype=torch.float64, device="cuda")
+        ts = []
+        for _ in range(5):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            torch.cuda.synchronize()
+            a.record()
+            h.rbf_project_f64(Xi, Xj, O, 0.01, Y, beta=0.5)
+            h.synchronize()
+            b.record()
+            torch.cuda.synchronize()
+            ts.append(a.elapsed_time(b))
+        return min(ts)
+
+    assert best(300, 500000, 74) < 2.0 * best(500000, 300, 74)
+    best(600000, 20, 1000)
+    assert h.workspace_bytes() < 3 * 2**30
+    h.close()
