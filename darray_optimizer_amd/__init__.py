@@ -90,6 +90,14 @@ class Handle:
     def workspace_bytes(self) -> int:
         return lib().dh_workspace_bytes(self.h)
 
+    def scratch_bytes(self) -> int:
+        """Size of the device's shared scratch buffer (K kept between passes)."""
+        return lib().dh_scratch_bytes(self.h)
+
+    def scratch_trim(self):
+        """Give the shared scratch buffer back if no call is using it."""
+        call("dh_scratch_trim", self.h)
+
     # ---------------------------------------------------------------- RBF
     def sqnorms_f64(self, X, out):
         n, d = X.shape

@@ -55,6 +55,13 @@ void scratch_count(int device, int add) {
     if (s.handles == 0) s.drop();
 }
 
+size_t scratch_size(int device) {
+    if (device >= kMaxDevices) return 0;
+    Scratch& s = g_scratch[device];
+    std::lock_guard<std::mutex> lock(s.mu);
+    return s.size;
+}
+
 // Gives an idle buffer back; false if there is none.
 bool scratch_trim(int device) {
     if (device >= kMaxDevices) return false;
@@ -225,6 +232,15 @@ extern "C" size_t dh_workspace_bytes(dh_handle_t h) {
     size_t s = 0;
     for (int i = 0; i < DH_WS_COUNT; ++i) s += h->ws_size[i];
     return s;
+}
+
+extern "C" size_t dh_scratch_bytes(dh_handle_t h) { return h ? scratch_size(h->device) : 0; }
+
+extern "C" int dh_scratch_trim(dh_handle_t h) {
+    if (!h) return dh_fail(-1, "dh_scratch_trim: NULL handle");
+    DH_CHECK_HIP(hipSetDevice(h->device));
+    scratch_trim(h->device);
+    return 0;
 }
 
 // ------------------------------------------------------ device memory helpers

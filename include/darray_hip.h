@@ -49,8 +49,17 @@ int dh_destroy(dh_handle_t h);
 int dh_synchronize(dh_handle_t h);
 /* Message for the last non-zero status returned on this thread. */
 const char* dh_last_error_string(void);
-/* Bytes of device workspace currently held by the handle. */
+/* Bytes of device workspace currently held by the handle (the scratch buffer
+ * below, which no handle owns, is not among them). */
 size_t dh_workspace_bytes(dh_handle_t h);
+/* dh_lra keeps K between its passes in one scratch buffer per device, shared by
+ * the handles of the process: at most an eighth of the device's memory, held
+ * until the device's last handle is destroyed or a library allocation needs the
+ * memory.  dh_scratch_bytes: its present size (0 if there is none).
+ * dh_scratch_trim gives it back at once if no call is using it, for programs
+ * that need the memory elsewhere; the next dh_lra may take a new one. */
+size_t dh_scratch_bytes(dh_handle_t h);
+int dh_scratch_trim(dh_handle_t h);
 
 /* Kernel timing for measurements (no reference counterpart; DArray times
  * phases with a host millisecond clock, utils.h:436-456).  With on != 0 the
@@ -248,10 +257,9 @@ int dh_cholqr2_f64(dh_handle_t h, int m, int n, double* Y, int ldy, double* R, i
  * replaced by pseudo-random ones, so Q always has l orthonormal columns
  * spanning range(Y) and more (as the reference's Householder QR would).
  * Above 256 features every `prec` runs the FP64 passes (the low-precision
- * kernels hold d <= 256).  K is kept between the passes where that pays, in a
- * buffer of up to an eighth of the device's memory that the process's handles
- * share and that goes back with the last of them; where it cannot be had, every
- * pass forms K and the results are the same.  Synchronises. */
+ * kernels hold d <= 256).  K is kept between the passes where that pays, in the
+ * scratch buffer of dh_scratch_bytes; where it cannot be had, every pass forms K
+ * and the results are the same.  Synchronises. */
 int dh_lra(dh_handle_t h, int prec, int n, int d, int l, int q, const double* X, int ldx,
            const double* y, double gamma, const double* Omega, int ldo, double* Q, int ldq,
            double* W, int ldw);
