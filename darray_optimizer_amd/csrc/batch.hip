@@ -406,7 +406,7 @@ int build_plan(dh_handle_t h, Plan& P, int prec, int count, const dh_lra_problem
     const size_t o_counters = cv.take(sizeof(int) * (size_t)passes * classes.size() + 64);
 
     P.bytes = cv.off;
-    DH_CHECK_HIP(hipMalloc(&P.mem, P.bytes));
+    DH_CHECK_HIP(dh_device_malloc(h, &P.mem, P.bytes));
     char* base = (char*)P.mem;
     auto at = [&](size_t o) { return (void*)(base + o); };
 

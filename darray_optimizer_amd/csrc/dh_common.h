@@ -57,6 +57,7 @@ struct dh_handle_s {
     // Resident workgroups per CU of the persistent kernels, by kernel
     // (queried on the handle's device on first use; handle.hip).
     void* occupancy = nullptr;
+    size_t alloc_limit = 0;  // dh_debug_alloc_limit
 };
 
 // Creates h->aux and its events if they do not exist yet.
@@ -97,6 +98,14 @@ uint64_t dh_tune_key_bf16(int dk, int ncb, int waves, int rows);
 
 // Records a formatted message for dh_last_error_string and returns `code`.
 int dh_fail(int code, const char* fmt, ...);
+
+// hipMalloc for everything that the library allocates on the handle's device (which
+// is current): where memory is short, an idle scratch buffer is given back first.
+hipError_t dh_device_malloc(dh_handle_t h, void** p, size_t bytes);
+
+// For tests of short memory: from now on an allocation of the handle fails if it
+// and the device's scratch buffer are more than `bytes` together (0: no limit).
+extern "C" int dh_debug_alloc_limit(dh_handle_t h, size_t bytes);
 
 // Device buffer of at least `bytes` in `slot`; nullptr on failure (message set).
 void* dh_ws(dh_handle_t h, dh_slot slot, size_t bytes);

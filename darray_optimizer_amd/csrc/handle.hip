@@ -105,6 +105,26 @@ void dh_scratch_release(int device) {
     s.busy = false;
 }
 
+hipError_t dh_device_malloc(dh_handle_t h, void** p, size_t bytes) {
+    auto attempt = [&] {
+        if (h->alloc_limit && bytes + scratch_size(h->device) > h->alloc_limit)
+            return hipErrorOutOfMemory;
+        const hipError_t e = hipMalloc(p, bytes);
+        if (e != hipSuccess) (void)hipGetLastError();
+        return e;
+    };
+    hipError_t e = attempt();
+    if (e != hipSuccess && scratch_trim(h->device)) e = attempt();
+    if (e != hipSuccess) *p = nullptr;
+    return e;
+}
+
+extern "C" int dh_debug_alloc_limit(dh_handle_t h, size_t bytes) {
+    if (!h) return dh_fail(-1, "dh_debug_alloc_limit: NULL handle");
+    h->alloc_limit = bytes;
+    return 0;
+}
+
 void* dh_ws(dh_handle_t h, dh_slot slot, size_t bytes) {
     if (bytes == 0) bytes = 256;
     if (h->ws_size[slot] >= bytes) return h->ws[slot];
@@ -120,13 +140,7 @@ void* dh_ws(dh_handle_t h, dh_slot slot, size_t bytes) {
     size_t want = bytes + bytes / 8;  // headroom for slightly larger later calls
     want = (want + 4095) & ~size_t(4095);
     void* p = nullptr;
-    hipError_t e = hipMalloc(&p, want);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        if (scratch_trim(h->device)) e = hipMalloc(&p, want);
-    }
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
+    if (dh_device_malloc(h, &p, want) != hipSuccess) {
         dh_fail(DH_ERR_ALLOC, "hipMalloc of %zu bytes (workspace slot %d) failed", want, (int)slot);
         return nullptr;
     }
@@ -253,11 +267,8 @@ extern "C" int dh_malloc(dh_handle_t h, size_t bytes, void** ptr) {
     *ptr = nullptr;
     if (bytes == 0) return 0;
     DH_CHECK_HIP(hipSetDevice(h->device));
-    if (hipMalloc(ptr, bytes) != hipSuccess) {
-        *ptr = nullptr;
-        (void)hipGetLastError();
+    if (dh_device_malloc(h, ptr, bytes) != hipSuccess)
         return dh_fail(DH_ERR_ALLOC, "dh_malloc: %zu bytes", bytes);
-    }
     return 0;
 }
 

@@ -23,6 +23,8 @@ namespace {
 
 dh_handle_t g_handle = nullptr;
 
+dh_handle_t handle();
+
 struct DevBuf {
     void* p = nullptr;
     size_t bytes = 0;
@@ -31,7 +33,7 @@ struct DevBuf {
         if (p) (void)hipFree(p);
         p = nullptr;
         bytes = 0;
-        if (hipMalloc(&p, want) != hipSuccess) {
+        if (dh_malloc(handle(), want, &p) != 0) {
             fprintf(stderr, "GPUassert: hipMalloc of %zu bytes failed\n", want);
             exit(1);
         }

@@ -37,3 +37,50 @@ def test_scratch_is_reported_and_given_back(dev):
     assert dev.scratch_bytes() == 0 and dev.workspace_bytes() == held
     b = solve(dev, X, Om)
     assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
+@pytest.fixture
+def limit(dev):
+    """Allocations of `dev` beyond the given bytes, the scratch buffer included, fail."""
+    import ctypes as C
+    fn = dh._capi.lib().dh_debug_alloc_limit
+    fn.argtypes, fn.restype = [C.c_void_p, C.c_size_t], C.c_int
+    yield lambda h, b: fn(h.h, int(b))
+    fn(dev.h, 0)
+
+
+def test_allocations_take_the_idle_scratch_back(limit):
+    """A workspace, dh_malloc and the batch's plan in memory that the idle scratch
+    buffer fills: each gives it back and succeeds; what is larger still fails."""
+    import ctypes as C
+
+    import torch
+    h = dh.Handle(0)
+    X, Om, _ = problem(3000, 40, 24)
+    solve(h, X, Om)
+    size = h.scratch_bytes()
+    assert size >= 8 * 3000 * 3000
+    limit(h, size)
+    p = C.c_void_p()
+    dh._capi.call("dh_malloc", h.h, size // 2, C.byref(p))
+    assert p.value and h.scratch_bytes() == 0
+    dh._capi.call("dh_free", h.h, p)
+    with pytest.raises(dh.DHError):
+        dh._capi.call("dh_malloc", h.h, 2 * size, C.byref(p))
+    assert not p.value
+    limit(h, 0)
+    solve(h, X, Om)
+    assert h.scratch_bytes() == size
+    limit(h, size)
+    K = torch.empty((3000, 3000), dtype=torch.float64, device="cuda")
+    torch.nn.init.eye_(K)
+    assert h.potrf(K) == 0  # new workspaces
+    assert h.scratch_bytes() == 0
+    limit(h, 0)
+    solve(h, X, Om)
+    limit(h, size)
+    probs = [{"X": X, "y": None, "Omega": Om, "gamma": 0.01, "q": 0, "Q": torch.empty_like(Om),
+              "W": torch.empty_like(Om)}]
+    info, _ = h.lra_batched(probs, prec=dh.DH_PREC_BF16)
+    assert info == 0 and h.scratch_bytes() == 0
+    h.close()
