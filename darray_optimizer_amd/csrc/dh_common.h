@@ -58,6 +58,7 @@ struct dh_handle_s {
     // (queried on the handle's device on first use; handle.hip).
     void* occupancy = nullptr;
     size_t alloc_limit = 0;  // dh_debug_alloc_limit
+    bool no_scratch = false, scratch_used = false;  // ScratchHold
 };
 
 // Creates h->aux and its events if they do not exist yet.
@@ -121,12 +122,14 @@ void* dh_scratch_take(int device, size_t bytes);
 void dh_scratch_release(int device);
 
 // The device's scratch buffer for the length of a call (p = nullptr: not
-// available, or not asked for).
+// available, not asked for, or the handle does without it).
 struct ScratchHold {
     dh_handle_t h;
     void* p;
     ScratchHold(dh_handle_t h_, size_t bytes)
-        : h(h_), p(bytes ? dh_scratch_take(h_->device, bytes) : nullptr) {}
+        : h(h_), p(bytes && !h_->no_scratch ? dh_scratch_take(h_->device, bytes) : nullptr) {
+        if (p) h->scratch_used = true;
+    }
     ~ScratchHold() {
         if (!p) return;
         (void)hipStreamSynchronize(h->stream);

@@ -423,15 +423,24 @@ extern "C" int dh_lra(dh_handle_t h, int prec, int n, int d, int l, int q, const
     // The low-precision kernels hold at most 256 features: above that every
     // precision runs the FP64 passes (materialised K row blocks).
     if (d > 256) prec = DH_PREC_F64;
-    int st;
-    if (prec == DH_PREC_F64)
-        st = lra_f64(h, n, d, l, q, X, ldx, y, gamma, Omega, ldo, Q, ldq, W, ldw);
-    else if (prec == DH_PREC_BF16)
-        st = dh_lra_bf16_passes(h, n, d, l, q, X, ldx, y, gamma, Omega, ldo, Q, ldq, W, ldw);
-    else if (prec == DH_PREC_F16)
-        st = dh_lra_f16_passes(h, n, d, l, q, X, ldx, y, gamma, Omega, ldo, Q, ldq, W, ldw);
-    else
-        st = dh_lra_fp8_passes(h, n, d, l, q, X, ldx, y, gamma, Omega, ldo, Q, ldq, W, ldw);
+    auto passes = [&] {
+        if (prec == DH_PREC_F64)
+            return lra_f64(h, n, d, l, q, X, ldx, y, gamma, Omega, ldo, Q, ldq, W, ldw);
+        if (prec == DH_PREC_BF16)
+            return dh_lra_bf16_passes(h, n, d, l, q, X, ldx, y, gamma, Omega, ldo, Q, ldq, W, ldw);
+        if (prec == DH_PREC_F16)
+            return dh_lra_f16_passes(h, n, d, l, q, X, ldx, y, gamma, Omega, ldo, Q, ldq, W, ldw);
+        return dh_lra_fp8_passes(h, n, d, l, q, X, ldx, y, gamma, Omega, ldo, Q, ldq, W, ldw);
+    };
+    h->scratch_used = false;
+    int st = passes();
+    // K kept in the scratch buffer can be what a workspace lacked: again without
+    // it (Q and W are outputs; an Omega in their place may be overwritten by now).
+    if (st == DH_ERR_ALLOC && h->scratch_used && Omega != Q && Omega != W) {
+        h->no_scratch = true;
+        st = passes();
+        h->no_scratch = false;
+    }
     if (st) return st;
     DH_CHECK_HIP(hipStreamSynchronize(h->stream));
     return 0;

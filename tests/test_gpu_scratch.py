@@ -84,3 +84,27 @@ def test_allocations_take_the_idle_scratch_back(limit):
     info, _ = h.lra_batched(probs, prec=dh.DH_PREC_BF16)
     assert info == 0 and h.scratch_bytes() == 0
     h.close()
+
+
+@pytest.mark.parametrize("prec,d", [("f64", 40), ("f64", 300), ("f16", 200), ("fp8", 256)])
+def test_lra_without_the_memory_for_kept_k(limit, prec, d):
+    """Memory for every workspace or for K, not for both: the solve gives K up and
+    returns the bits of a solve that kept it."""
+    import torch
+    which = {"f64": dh.DH_PREC_F64, "f16": dh.DH_PREC_F16, "fp8": dh.DH_PREC_FP8}[prec]
+    X, Om, y = problem(13000, d, 140, labels=True)
+    dev = dh.Handle(0)
+    dev.scratch_trim()
+    a = solve(dev, X, Om, 2, y, which)
+    kept = dev.scratch_bytes()
+    assert kept >= (8 if prec == "f64" else 2) * 13000 * 13000
+    h = dh.Handle(0)
+    limit(h, kept)
+    b = solve(h, X, Om, 2, y, which)
+    assert h.scratch_bytes() == 0  # given up
+    limit(h, 0)
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+    c = solve(h, X, Om, 2, y, which)
+    assert h.scratch_bytes() == kept and torch.equal(a[1], c[1])
+    h.close()
+    dev.close()
