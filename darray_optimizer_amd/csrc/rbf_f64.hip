@@ -1288,20 +1288,21 @@ extern "C" int dh_lra_error(dh_handle_t h, int n, int d, int l, const double* X,
     // the last, partly filled round of tiles no longer costs more than they
     // save (d = 20, l = 250: n = 5000 0.36 -> 0.37 ms, n = 8000 0.84 -> 0.71 ms; n = 65536,
     // d = 128, l = 272: 71.1 -> 50.0 ms).  The 64 x 64 tiles of the whole matrix below
-    // that, and for d = 0 or l = 0.  A tile's copies have 32-bit byte offsets.
+    // that, for d = 0 or l = 0, and where the point-major copies cannot be had.  A
+    // tile's copies have 32-bit byte offsets, a launch fewer than 2^32 threads.
     const int sd = dh_cdiv(d, 16), sl = dh_cdiv(l, 16), nt = dh_cdiv(n, 128);
     const long tiles = (long)nt * (nt + 1) / 2;
-    const bool sym = tiles > 5L * h->num_cu && d > 0 && l > 0 && std::max(sd, sl) < (1 << 18) &&
-                     tiles < (1L << 30);
+    double* Xp = nullptr;
+    if (tiles > 5L * h->num_cu && d > 0 && l > 0 && std::max(sd, sl) < (1 << 18) &&
+        tiles < (1L << 30) && (long)n * sd < (1L << 28) - 16)
+        Xp = (double*)dh_ws(h, DH_WS_PACK64,
+                            sizeof(double) * 16 * (size_t)n * ((size_t)sd + 2 * sl));
     const int wgs = (int)std::min<long>((tiles + 7) / 8 * 8, std::max(8, h->num_cu / 8 * 8));
     dim3 grid(dh_cdiv(n, 64), dh_cdiv(n, 64));
-    size_t nblk = sym ? 8 * (size_t)wgs : (size_t)grid.x * grid.y;
+    size_t nblk = Xp ? 8 * (size_t)wgs : (size_t)grid.x * grid.y;
     double* part = (double*)dh_ws(h, DH_WS_PARTIAL, sizeof(double) * (2 * nblk + 2));
     if (!part) return DH_ERR_ALLOC;
-    if (sym) {
-        double* Xp = (double*)dh_ws(h, DH_WS_PACK64,
-                                    sizeof(double) * 16 * (size_t)n * ((size_t)sd + 2 * sl));
-        if (!Xp) return DH_ERR_ALLOC;
+    if (Xp) {
         double *Qp = Xp + 16 * (size_t)n * sd, *Wp = Qp + 16 * (size_t)n * sl;
         pack_points_kernel<<<(unsigned)(((size_t)n * sd * 16 + 255) / 256), 256, 0, h->stream>>>(
             n, d, 16 * sd, X, ldx, Xp);

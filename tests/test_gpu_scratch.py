@@ -108,3 +108,22 @@ def test_lra_without_the_memory_for_kept_k(limit, prec, d):
     assert h.scratch_bytes() == kept and torch.equal(a[1], c[1])
     h.close()
     dev.close()
+
+
+def test_lra_error_without_the_memory_for_its_copies(limit):
+    """n > 6400 with no room for the point-major copies of X, Q and W: the 64 x 64
+    tiles, which need none.  Both sum n^2 squares that agree to the rounding of
+    K - Q W^T, whose entries are of the order of one (l = 20 products)."""
+    h = dh.Handle(0)
+    h.scratch_trim()
+    X, Q, y = problem(6500, 24, 20, labels=True)
+    W = problem(6500, 24, 20, seed=1)[1]
+    a = h.lra_error(X, 0.3, Q, W, y=y)
+    h.close()
+    h = dh.Handle(0)
+    copies = 8 * 16 * 6500 * (2 + 2 * 2)
+    limit(h, copies)  # and an eighth of headroom
+    b = h.lra_error(X, 0.3, Q, W, y=y)
+    assert h.workspace_bytes() < copies
+    assert abs(a[0] - b[0]) <= 1e-13 * a[0] and abs(a[1] - b[1]) <= 1e-13 * a[1]
+    h.close()
