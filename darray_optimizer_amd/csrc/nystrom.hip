@@ -486,10 +486,12 @@ JacobiPlan jacobi_plan(int m, int n) {
 }
 
 // Doubles of work space that jacobi_sweeps wants beside A and V: a second
-// buffer for A's columns and the rotations of two sweeps.
+// buffer for A's columns and the rotations of two sweeps, or nothing where a
+// round is a launch.
 size_t jacobi_work_doubles(int m, int n) {
+    if (jacobi_plan(m, n).own == 0) return 0;
     const size_t N = n + (n & 1);
-    return (size_t)m * n + (N > 0 ? 2 * (N - 1) * N : 0) + 2;
+    return (size_t)m * n + 2 * (N - 1) * N + 2;
 }
 
 int launch_rounds(dh_handle_t h, int m, int n, int N, int r0, int T, int own, const double* Ain,

@@ -166,3 +166,18 @@ def test_gesvj_round_grouping(dev, m, n):
     assert rel(AVg, A @ Vg) < 1e-12
     # Same rotations in the same order: the same signs as well.
     assert rel(Vg, Vo) < 1e-6
+
+
+def test_gesvj_workspace_of_long_columns():
+    """Columns too long for LDS keep no rotation log: a copy of A and of V, and an
+    eighth of headroom."""
+    import torch
+    m, n = 600, 400
+    h = dh.Handle(0)
+    Ad = dh.to_dev(np.random.default_rng(3).standard_normal((m, n)))
+    s = torch.zeros(n, dtype=torch.float64, device="cuda")
+    V = torch.zeros((n, n), dtype=torch.float64, device="cuda")
+    st, _ = h.gesvj(Ad, s, V)
+    assert st == 0
+    assert h.workspace_bytes() <= 1.125 * (8 * (m * n + n * n + 2 * n) + 1024) + 8192
+    h.close()
