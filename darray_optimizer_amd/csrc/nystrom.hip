@@ -453,16 +453,15 @@ __global__ __launch_bounds__(256) void copy_cols_kernel(int m, int n, const doub
 int grid_for(size_t total) { return (int)std::min<size_t>((total + 255) / 256, 4096); }
 
 // How the rounds of a sweep are grouped: `own` cells per workgroup, at most T
-// rounds per launch, `launches` per sweep.  own = 0: one launch per round.  A
-// round costs about 0.8 us + 0.25 us per four cells of a workgroup, a launch
-// with its loads and stores 5 us.  So up to 20 cells are one workgroup and one
-// launch per sweep, and larger orders are cut into many small workgroups that
-// share cells: 4 own cells and 12 rounds (28 cells at the first) measured best
-// at order 272: 11.2 ms per factor against 11.6 (8 own, 8 rounds), 11.5 (4, 10)
-// and 12.6 (4, 6) with V's update on the same stream, and 26.6 with one launch
-// per round (n = 65536, 14 sweeps; 11.2 again with V's update beside and the
-// correctly rounded angle).  Long columns lower T until the cells fit in LDS.  `launches` is even there, so that a sweep
-// ends in the buffer that it began in.
+// rounds per launch, `launches` per sweep.  own = 0: one launch per round, for
+// columns or orders that LDS does not hold and for a single pair.  A round
+// costs about 0.8 us + 0.25 us per four cells of a workgroup, a launch with its
+// loads and stores 5 us.  So up to 20 cells are one workgroup and one launch per
+// sweep (order 16 0.47 -> 0.23 ms, 4 0.14 ms either way, 2 0.09 ms and 0.14 in one
+// workgroup), and larger orders are cut into many small workgroups that share
+// cells: 4 own cells and 12 rounds, 28 cells at the first (order 272, n = 65536: 26.6
+// -> 11.2 ms per factor).  Long columns lower T until the cells fit in LDS.
+// `launches` is even there, so that a sweep ends in the buffer that it began in.
 struct JacobiPlan {
     int own = 0, T = 0, launches = 0;
 };
@@ -470,7 +469,7 @@ struct JacobiPlan {
 JacobiPlan jacobi_plan(int m, int n) {
     JacobiPlan p;
     const int N = n + (n & 1), half = N / 2;
-    if (m > 512 || N > kJacApplyMaxN) return p;
+    if (m > 512 || N > kJacApplyMaxN || N == 2) return p;
     const int cap = kJacDoubles / (128 * dh_cdiv(m, 64));  // cells that fit in LDS (>= 19)
     if (half <= std::min(cap, 20)) {
         p.own = half;
@@ -521,9 +520,10 @@ int launch_rounds(dh_handle_t h, int m, int n, int N, int r0, int T, int own, co
 // Jacobi sweeps on A (m x n) accumulating V (n x n, set to I here); flags and
 // the sweep counter live in `words` (8 ints of device memory), `work` holds
 // jacobi_work_doubles(m, n).  *sweeps_out receives the sweeps run, or -1 if
-// kMaxSweeps did not converge.  V's update of a sweep runs on the handle's
-// second stream beside the next sweep (1 ms of 11 at order 272); the handle's
-// stream waits for it before the call goes on.
+// kMaxSweeps did not converge.  Where a sweep is several launches V's update
+// runs on the handle's second stream beside the next sweep (1 ms of 11 at order
+// 272), and the handle's stream waits for it before the call goes on; where it
+// is one launch the events would cost more (orders up to 16: 0.25 ms against 0.14).
 int jacobi_sweeps(dh_handle_t h, int m, int n, double* A, int lda, double* V, int ldv,
                   double* work, int* words, int* sweeps_out) {
     hipStream_t s = h->stream;
@@ -537,7 +537,8 @@ int jacobi_sweeps(dh_handle_t h, int m, int n, double* A, int lda, double* V, in
     if (!host) return dh_fail(DH_ERR_ALLOC, "dh_gesvj: pinned status words unavailable");
     const int N = n + (n & 1);
     const JacobiPlan plan = jacobi_plan(m, n);
-    if (plan.own) DH_CHECK_STATUS(dh_aux_stream(h));
+    const bool beside = plan.launches > 1;  // V's update on the second stream
+    if (beside) DH_CHECK_STATUS(dh_aux_stream(h));
     double* A2 = work;
     double2* log = (double2*)(((uintptr_t)(work + (size_t)m * n) + 15) & ~(uintptr_t)15);
     bool pending = false;  // an update of V was queued
@@ -573,15 +574,17 @@ int jacobi_sweeps(dh_handle_t h, int m, int n, double* A, int lda, double* V, in
             // The next sweep reuses the log of the sweep before this one: wait
             // for that one's update of V, then queue this one's.
             if (pending) DH_CHECK_HIP(hipStreamWaitEvent(s, h->ev_update, 0));
-            DH_CHECK_HIP(hipEventRecord(h->ev_panel, s));
-            DH_CHECK_HIP(hipStreamWaitEvent(h->aux, h->ev_panel, 0));
+            if (beside) {
+                DH_CHECK_HIP(hipEventRecord(h->ev_panel, s));
+                DH_CHECK_HIP(hipStreamWaitEvent(h->aux, h->ev_panel, 0));
+            }
             jacobi_apply_kernel<<<dh_cdiv(n, kJacRows),
-                                  std::min(1024, 64 * dh_cdiv(N / 2 * kJacRows, 64)), 0, h->aux>>>(
+                                  std::min(1024, 64 * dh_cdiv(N / 2 * kJacRows, 64)), 0, beside ? h->aux : s>>>(
                 n, N, log + (sweep & 1) * (size_t)(N - 1) * (N / 2), V, ldv,
                 words + 4 + sweep % 4);
             DH_CHECK_LAUNCH();
-            DH_CHECK_HIP(hipEventRecord(h->ev_update, h->aux));
-            pending = true;
+            if (beside) DH_CHECK_HIP(hipEventRecord(h->ev_update, h->aux));
+            pending = beside;
         }
         if (sweep >= 5 || sweep == kMaxSweeps - 1) {
             DH_CHECK_HIP(hipMemcpyAsync(host, words, 3 * sizeof(int), hipMemcpyDeviceToHost, s));

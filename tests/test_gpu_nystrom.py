@@ -145,9 +145,9 @@ def test_nystrom_argument_errors(dev):
         dev.nystrom(Q, Q, 11, Z)  # k > l
 
 
-# One workgroup for all pairs (n <= 64), several with 8 or 4 rounds per launch
-# (row counts at the LDS capacities of 32 pairs and at 512), odd n (a padding
-# player), and columns too long for LDS (a launch per round).
+# One workgroup for all pairs (n <= 40), several with up to 12 rounds per launch,
+# fewer for long columns (up to 512 rows), odd n (a padding player), a single
+# pair, and columns too long for LDS (a launch per round).
 @pytest.mark.parametrize("m,n", [(2, 2), (5, 3), (64, 64), (65, 65), (128, 66), (139, 137),
                                  (312, 120), (313, 121), (512, 201), (513, 40)])
 def test_gesvj_round_grouping(dev, m, n):
@@ -180,4 +180,31 @@ def test_gesvj_workspace_of_long_columns():
     st, _ = h.gesvj(Ad, s, V)
     assert st == 0
     assert h.workspace_bytes() <= 1.125 * (8 * (m * n + n * n + 2 * n) + 1024) + 8192
+    h.close()
+
+
+@pytest.mark.parametrize("n", [2, 4])
+def test_gesvj_of_few_columns_is_no_slower_than_round_by_round(n):
+    """Orders of a few columns, where launches and events are the whole time,
+    against columns of 520 entries, which take a launch per round."""
+    import time
+
+    import torch
+    h = dh.Handle(0)
+
+    def median(m):
+        A0 = dh.to_dev(np.random.default_rng(n).standard_normal((m, n)))
+        A, V = A0.clone(), torch.zeros((n, n), dtype=torch.float64, device="cuda")
+        s = torch.zeros(n, dtype=torch.float64, device="cuda")
+        ts = []
+        for _ in range(31):
+            A.copy_(A0)
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            h.gesvj(A, s, V)
+            torch.cuda.synchronize()
+            ts.append(time.perf_counter() - t0)
+        return sorted(ts)[15]
+
+    assert median(n) < 1.5 * median(520)
     h.close()
