@@ -114,10 +114,11 @@ void* dh_ws(dh_handle_t h, dh_slot slot, size_t bytes);
 // One large scratch buffer per device for the length of a call, shared by all
 // handles of the process.  dh_scratch_take returns nullptr, with no message,
 // when another call holds it, when `bytes` would be more than an eighth of the
-// device's memory or more than half of what is free, or when it cannot be
+// device's memory or more than half of what is free, when buffers given back
+// just before still wait to be wiped (handle.hip), or when it cannot be
 // allocated: its callers can do without it.  The buffer stays allocated until
-// the device's last handle is destroyed or another workspace needs the memory.
-// The taker waits for its stream before dh_scratch_release.
+// the device's last handle is destroyed, another allocation needs the memory, or
+// dh_scratch_trim.  The taker waits for its stream before dh_scratch_release.
 void* dh_scratch_take(int device, size_t bytes);
 void dh_scratch_release(int device);
 

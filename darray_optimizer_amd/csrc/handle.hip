@@ -6,6 +6,8 @@
 // the handle's one stream, and device workspaces are allocated once and
 // grown on demand instead of the per-call cudaMallocManaged / cudaFree of
 // rbf_kernel and tc_gemm (dkernel.cu:135-147, 196-198).
+#include <algorithm>
+#include <chrono>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -31,14 +33,33 @@ int dh_fail(int code, const char* fmt, ...) {
 extern "C" const char* dh_last_error_string(void) { return g_last_error; }
 
 namespace {
+// Freed device memory is wiped in the background at about 36 GB/s, and from some
+// point on an allocation waits for it.  With a handle for every FP64 solve, and a
+// new buffer each time, n = 65536, l = 272, q = 1 took 128 ms for up to seven calls
+// and 972 ms for each one after them, n = 32768 250 ms; without keeping K 200 and
+// 51 ms.  So buffers that were given back count as unwiped for a while, and no new
+// one is taken beside more than an eighth of the device's memory of them (185 and
+// 50 ms: every sixth or so of the solves keeps K).
+constexpr double kWipeRate = 25e9;  // bytes per second
+
 struct Scratch {
     std::mutex mu;
     void* p = nullptr;
     size_t size = 0;
     bool busy = false;
     int handles = 0;  // handles alive on the device
-    void drop() {     // mu held, not busy: no queued work reads the buffer
-        if (p) (void)hipFree(p);
+    double freed = 0.0;  // bytes given back and not wiped yet at `then`
+    std::chrono::steady_clock::time_point then;
+    double unwiped(std::chrono::steady_clock::time_point now) const {
+        return std::max(0.0, freed - kWipeRate * std::chrono::duration<double>(now - then).count());
+    }
+    void drop() {  // mu held, not busy: no queued work reads the buffer
+        if (p) {
+            (void)hipFree(p);
+            const auto now = std::chrono::steady_clock::now();
+            freed = unwiped(now) + (double)size;
+            then = now;
+        }
         p = nullptr;
         size = 0;
     }
@@ -87,6 +108,7 @@ void* dh_scratch_take(int device, size_t bytes) {
             return nullptr;
         }
         if (bytes > total / 8 || bytes > (avail + s.size) / 2) return nullptr;
+        if (s.unwiped(std::chrono::steady_clock::now()) > (double)(total / 8)) return nullptr;
         s.drop();
         if (hipMalloc(&s.p, bytes) != hipSuccess) {
             (void)hipGetLastError();

@@ -127,3 +127,28 @@ def test_lra_error_without_the_memory_for_its_copies(limit):
     assert h.workspace_bytes() < copies
     assert abs(a[0] - b[0]) <= 1e-13 * a[0] and abs(a[1] - b[1]) <= 1e-13 * a[1]
     h.close()
+
+
+def test_handles_made_for_every_solve_do_not_wait_for_the_wipe(limit):
+    """A handle per solve gives K's buffer back each time, and the driver wipes freed
+    memory at a limited rate: buffers are taken no faster than that (25 GB/s, after
+    the first eighth of the device's memory), the other solves form K in every
+    pass and return the same bits."""
+    import time
+
+    import torch
+    X, Om, _ = problem(20000, 16, 16)
+    total = torch.cuda.get_device_properties(0).total_memory
+    size, kept, t0, first = 8 * 20032 * 20000, 0, time.perf_counter(), None
+    for _ in range(40):
+        h = dh.Handle(0)
+        h.scratch_trim()  # as the last handle's end does
+        out = solve(h, X, Om, 2)
+        kept += h.scratch_bytes() >= size
+        h.scratch_trim()
+        h.close()
+        first = first or out
+        assert torch.equal(out[0], first[0]) and torch.equal(out[1], first[1])
+    allowed = total / 8 + 25e9 * (time.perf_counter() - t0) + 2 * size
+    assert 1 <= kept and kept * size <= allowed
+    time.sleep(total / 8 / 25e9)  # for the tests after this one
