@@ -14,7 +14,7 @@ int dh_project_f64_split(dh_handle_t h, int m, int n, int d, int l, const double
                         const double* Xj, int ldxj, const double* ni, const double* nj,
                         const double* yi, const double* yj, double gamma, const double* O,
                         int ldo, double* Y, int ldy, void* keep, int kmode);
-size_t dh_kkeep_bytes(int m, int n);
+size_t dh_kkeep_bytes(dh_handle_t h, int n, int d, int l, int q);
 int dh_lra_bf16_passes(dh_handle_t h, int n, int d, int l, int q, const double* X, int ldx,
                        const double* y, double gamma, const double* Omega, int ldo, double* Q,
                        int ldq, double* W, int ldw);
@@ -372,20 +372,19 @@ static int copy_panel(dh_handle_t h, int n, int l, const double* src, int lds, d
 
 // FP64 passes: Y = K*Omega -> Q; q x { K*Q -> orthonormal basis }; W = K*Q.
 //
-// All q + 2 passes multiply the same K, so it is formed once, from one triangle,
-// and kept (8 n^2 bytes: 34 GB at n = 65536, of 288): at 8 bytes per 2l flops
-// reading it back is a tenth of what HBM gives, while the distances and
-// exponentials are almost half of a fused pass at d = 128, l = 272 (66.0 ms with
-// them, 36.5 ms without: 82% of the FP64 MFMA peak; forming K 14.2 ms; the solve
-// 265 -> 163 ms).  Where the device's scratch buffer cannot be had every pass
-// forms K; the bits are the same.
+// All q + 2 passes multiply the same K, so where it pays (dh_kkeep_bytes) it is
+// formed once, from one triangle, and kept (8 n^2 bytes: 34 GB at n = 65536, of
+// 288).  At d = 128, l = 272 the distances and exponentials are almost half of a
+// fused pass (66.0 ms with them, 36.5 ms without: 82% of the FP64 MFMA peak, at a
+// tenth of what HBM gives; forming K 14.2 ms; the solve 265 -> 163 ms).  Where the
+// device's scratch buffer cannot be had every pass forms K; the bits are the same.
 static int lra_f64(dh_handle_t h, int n, int d, int l, int q, const double* X, int ldx,
                    const double* y, double gamma, const double* Omega, int ldo, double* Q,
                    int ldq, double* W, int ldw) {
     double* nrm = (double*)dh_ws(h, DH_WS_NORMS, sizeof(double) * (size_t)n);
     if (!nrm) return DH_ERR_ALLOC;
     DH_CHECK_STATUS(dh_sqnorms_f64(h, n, d, X, ldx, nrm));
-    const ScratchHold kk(h, dh_kkeep_bytes(n, n));
+    const ScratchHold kk(h, dh_kkeep_bytes(h, n, d, l, q));
     const int form = kk.p ? 1 : 0, use = kk.p ? 2 : 0;
     DH_CHECK_STATUS(dh_project_f64_split(h, n, n, d, l, X, ldx, X, ldx, nrm, nrm, y, y, gamma,
                                         Omega, ldo, Q, ldq, kk.p, form));

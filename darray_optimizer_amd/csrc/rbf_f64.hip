@@ -816,9 +816,22 @@ static int project_f64_blocked(dh_handle_t h, int m, int n, int d, int l, const 
     return 0;
 }
 
-// Bytes that dh_project_f64_split needs to keep K (m x n).
-size_t dh_kkeep_bytes(int m, int n) {
-    return kept_bytes(m, n);
+// Bytes that dh_project_f64_split needs to keep K (n x n) over the q + 2 passes of a
+// solve, 0 where that does not pay.  A kept pass is bound by its workgroups' chunk
+// by chunk reads where K is larger than the 256 MB cache and there is about one
+// workgroup per CU; with two column blocks and up to 32 features a fused pass is as
+// fast there, and forming K has to come back over the passes.  d = l = 16, fused ->
+// kept: n = 8192 0.56 -> 0.63 ms (q = 0), 0.86 -> 0.90 (q = 1), 1.15 -> 1.14 (q = 2);
+// n = 16384 1.94 -> 2.03 (q = 0), 2.98 -> 2.85 (q = 1).  On the other side: n = 5000 1.3x,
+// 6000 and 10000 1.03x, 20000 1.2x, 65536 1.17x (q = 0); n = 8192 with l = 33 1.06x or d =
+// 33 1.1x; up to 3.1x at d = 256; d > 256, where a pass forms K anyway, 1.1x to 3x.
+size_t dh_kkeep_bytes(dh_handle_t h, int n, int d, int l, int q) {
+    const size_t bytes = kept_bytes(n, n);
+    if (d > 32 || l > 32 || bytes <= (256u << 20)) return bytes;
+    const long tiles = dh_cdiv(n, 64);
+    const int splits = dh_j_splits(h->num_cu, tiles, dh_cdiv(n, 32));
+    const bool once = 4 * tiles * splits > 3L * h->num_cu && tiles * splits <= h->num_cu;
+    return once && (q == 0 || (q == 1 && splits > 1)) ? 0 : bytes;
 }
 
 // Y (m x l) = K(Xi, Xj) O + beta Y with the fused kernel, the j range in

@@ -129,6 +129,21 @@ def test_lra_error_without_the_memory_for_its_copies(limit):
     h.close()
 
 
+@pytest.mark.parametrize("n,d,l,q,kept", [(8192, 16, 16, 0, False), (8000, 32, 32, 1, False),
+                                          (16384, 8, 20, 0, False), (8192, 16, 16, 2, True),
+                                          (8192, 33, 16, 0, True), (8192, 16, 33, 0, True),
+                                          (4096, 16, 16, 0, True), (10000, 16, 16, 0, True),
+                                          (16384, 8, 20, 1, True), (20000, 16, 16, 0, True),
+                                          (8192, 300, 16, 0, True)])
+def test_f64_keeps_k_where_that_pays(dev, n, d, l, q, kept):
+    """With two column blocks and up to 32 features a kept pass is no faster than a
+    fused one where the grid has about one workgroup per CU (256 of them)."""
+    X, Om, _ = problem(n, d, l)
+    dev.scratch_trim()
+    solve(dev, X, Om, q)
+    assert (dev.scratch_bytes() > 0) == kept
+
+
 def test_handles_made_for_every_solve_do_not_wait_for_the_wipe(limit):
     """A handle per solve gives K's buffer back each time, and the driver wipes freed
     memory at a limited rate: buffers are taken no faster than that (25 GB/s, after
