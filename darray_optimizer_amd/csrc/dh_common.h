@@ -107,6 +107,8 @@ hipError_t dh_device_malloc(dh_handle_t h, void** p, size_t bytes);
 // For tests of short memory: from now on an allocation of the handle fails if it
 // and the device's scratch buffer are more than `bytes` together (0: no limit).
 extern "C" int dh_debug_alloc_limit(dh_handle_t h, size_t bytes);
+// For tests of kept K: the handle's calls do without the scratch buffer.
+extern "C" int dh_debug_no_scratch(dh_handle_t h, int on);
 
 // Device buffer of at least `bytes` in `slot`; nullptr on failure (message set).
 void* dh_ws(dh_handle_t h, dh_slot slot, size_t bytes);

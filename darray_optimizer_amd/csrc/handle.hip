@@ -147,6 +147,12 @@ extern "C" int dh_debug_alloc_limit(dh_handle_t h, size_t bytes) {
     return 0;
 }
 
+extern "C" int dh_debug_no_scratch(dh_handle_t h, int on) {
+    if (!h) return dh_fail(-1, "dh_debug_no_scratch: NULL handle");
+    h->no_scratch = on != 0;
+    return 0;
+}
+
 void* dh_ws(dh_handle_t h, dh_slot slot, size_t bytes) {
     if (bytes == 0) bytes = 256;
     if (h->ws_size[slot] >= bytes) return h->ws[slot];

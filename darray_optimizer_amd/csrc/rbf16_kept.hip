@@ -239,14 +239,19 @@ size_t dh_kept16_bytes(int m, int nchunks) {
 // keeping K pays where the fused pass is slow: at 256 features, whose Xi
 // fragments leave 16-bit distances 32 rows for each of four waves, and whose FP8
 // distances pair up or carry few columns, and over at least three passes, for
-// the forming of K.  Solves with q = 1, fused -> kept: FP16 n = 65536, l = 138: 9.8
-// -> 7.6 ms, l = 272: 14.8 -> 10.8 ms; FP8 n = 131072, l = 544: 71.2 -> 68.7 ms; n =
-// 32768, l = 138, q = 2: 5.2 -> 3.7 ms.  On the other side: FP8 at l = 272 9.7 ->
-// 10.0 ms, two passes of BF16 2.8 -> 2.7 ms, FP16 at 128 features 9.8 -> 10.1 ms (q
-// = 2: 13.2 -> 13.0 ms).
-bool dh_kept16_pays(int dpad, bool fp8, int ncb, int groups, int passes) {
+// the forming of K.  Solves with q = 1, fused -> kept: FP16 n = 65536, l = 138: 10.1
+// -> 7.8 ms, l = 272: 15.6 -> 10.8 ms, l = 544: 33.3 -> 22.1 ms; FP8 n = 16384, l = 138: 2.11
+// -> 1.56 ms, l = 544: 4.76 -> 4.46 ms, n = 65536, l = 544: 21.9 -> 21.0 ms (n = 131072 73.1
+// -> 72.1, within the runs' range; q = 2 98.9 -> 94.8).  16-bit distances at few points
+// do not pay for the forming and its launch: l = 138 from n = 8192 on (1.04x; n = 2048 to
+// 4096 0.98x, 6000 1.00x), 17 column blocks above it (l = 272, n = 8500 to 11500 1.02x to
+// 1.05x; n = 2048 to 6000 0.96x to 0.98x, 8192 0.99x).  Also not: FP8 at l = 272 9.7 ->
+// 10.0 ms, two passes of BF16 2.8 -> 2.7 ms, FP16 at 128 features 9.8 -> 10.1 ms (q = 2:
+// 13.2 -> 13.0 ms).
+bool dh_kept16_pays(int n, int dpad, bool fp8, int ncb, int groups, int passes) {
     if (dpad != 256 || passes < 3) return false;
-    return ncb == 9 || (ncb == 17 && (!fp8 || groups % 2 == 0));
+    if (fp8) return ncb == 9 || (ncb == 17 && groups % 2 == 0);
+    return (ncb == 9 && n >= 8192) || (ncb == 17 && n > 8192);
 }
 
 int dh_form16(dh_handle_t h, bool f16, bool fp8, int dpad, int m, int nchunks, const bf16x8* Xi,

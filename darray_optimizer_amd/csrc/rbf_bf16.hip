@@ -574,7 +574,7 @@ int lra_16_passes(dh_handle_t h, int n, int d, int l, int q, const double* X, in
     // Where it pays, K is formed once for the q + 2 passes (rbf16_kept.hip).
     const Bf16Cols cols = bf16_cols(l);
     const int nch = dh_cdiv(n, 32);
-    const bool pays = dh_kept16_pays(dpad_of(d), false, cols.ncb, cols.groups, q + 2);
+    const bool pays = dh_kept16_pays(n, dpad_of(d), false, cols.ncb, cols.groups, q + 2);
     const ScratchHold kk(h, pays ? dh_kept16_bytes(n, nch) : 0);
     if (kk.p)
         DH_CHECK_STATUS(dh_form16(h, F16, false, dpad_of(d), n, nch, (const bf16x8*)p.xb,
@@ -629,7 +629,7 @@ int dh_lra_fp8_passes(dh_handle_t h, int n, int d, int l, int q, const double* X
     const float c2 = (float)(2.0 * gamma) * kLog2e;
     const Bf16Cols cols = bf16_cols(l);
     const int nch = dh_cdiv(n, 32);
-    const bool pays = dh_kept16_pays(dpad8_of(d), true, cols.ncb, cols.groups, q + 2);
+    const bool pays = dh_kept16_pays(n, dpad8_of(d), true, cols.ncb, cols.groups, q + 2);
     const ScratchHold kk(h, pays ? dh_kept16_bytes(n, nch) : 0);
     if (kk.p)
         DH_CHECK_STATUS(dh_form16(h, false, true, dpad8_of(d), n, nch, (const bf16x8*)p.xb,

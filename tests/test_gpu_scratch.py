@@ -129,6 +129,47 @@ def test_lra_error_without_the_memory_for_its_copies(limit):
     h.close()
 
 
+def kept_and_not(h, X, Om, q, y, prec):
+    """The solve on kept K (it must have been kept) and with K formed in every pass."""
+    import ctypes as C
+    fn = dh._capi.lib().dh_debug_no_scratch
+    fn.argtypes, fn.restype = [C.c_void_p, C.c_int], C.c_int
+    h.scratch_trim()
+    a = solve(h, X, Om, q, y, prec)
+    size = h.scratch_bytes()
+    assert size >= (8 if prec == dh.DH_PREC_F64 or X.shape[1] > 256 else 2) * X.shape[0] ** 2
+    h.scratch_trim()
+    fn(h.h, 1)
+    try:
+        b = solve(h, X, Om, q, y, prec)
+        assert h.scratch_bytes() == 0
+    finally:
+        fn(h.h, 0)
+    return a, b
+
+
+@pytest.mark.parametrize("prec", ["f16", "bf16"])
+@pytest.mark.parametrize("n,d,l,q", [(8192, 129, 130, 1), (8201, 200, 144, 2), (8300, 256, 280, 1),
+                                     (8193, 256, 272, 1), (12037, 140, 260, 2),
+                                     (8500, 256, 544, 1)])
+def test_16_bit_solves_on_kept_k_return_the_fused_bits(dev, prec, n, d, l, q):
+    """9 and 17 column blocks, single and paired, whole and ragged row tiles, chunks
+    and columns, with labels that are not +-1."""
+    import torch
+    X, Om, y = problem(n, d, l, labels=True)
+    a, b = kept_and_not(dev, X, Om, q, y, {"f16": dh.DH_PREC_F16, "bf16": dh.DH_PREC_BF16}[prec])
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
+@pytest.mark.parametrize("n,l,kept", [(4096, 138, False), (8192, 138, True), (8192, 272, False),
+                                      (8192, 544, False), (8500, 272, True)])
+def test_16_bit_solves_keep_k_where_that_pays(dev, n, l, kept):
+    X, Om, _ = problem(n, 256, l)
+    dev.scratch_trim()
+    solve(dev, X, Om, 1, prec=dh.DH_PREC_F16)
+    assert (dev.scratch_bytes() > 0) == kept
+
+
 @pytest.mark.parametrize("n,d,l,q,kept", [(8192, 16, 16, 0, False), (8000, 32, 32, 1, False),
                                           (16384, 8, 20, 0, False), (8192, 16, 16, 2, True),
                                           (8192, 33, 16, 0, True), (8192, 16, 33, 0, True),
