@@ -161,6 +161,23 @@ def test_16_bit_solves_on_kept_k_return_the_fused_bits(dev, prec, n, d, l, q):
     assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
 
 
+@pytest.mark.parametrize("prec,n,d,l,q", [("f64", 65, 8, 17, 1), ("f64", 3001, 20, 40, 1),
+                                          ("f64", 2050, 64, 272, 0), ("f64", 2999, 130, 300, 1),
+                                          ("f64", 301, 250, 290, 2), ("f64", 5001, 257, 33, 1),
+                                          ("f64", 1501, 300, 560, 0), ("f64", 11800, 260, 5, 0),
+                                          ("f16", 2000, 300, 50, 1), ("fp8", 300, 130, 140, 1),
+                                          ("fp8", 2051, 256, 544, 1), ("fp8", 4099, 200, 288, 2)])
+def test_solves_on_kept_k_return_the_same_bits(dev, prec, n, d, l, q):
+    """Every feature width of the forming kernel, one and two column groups, odd
+    sizes, triangle against row blocks above 256 features (FP64 for every
+    precision there), FP8; labels that are not +-1."""
+    import torch
+    X, Om, y = problem(n, d, l, labels=True)
+    which = {"f64": dh.DH_PREC_F64, "f16": dh.DH_PREC_F16, "fp8": dh.DH_PREC_FP8}[prec]
+    a, b = kept_and_not(dev, X, Om, q, y, which)
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
 @pytest.mark.parametrize("n,l,kept", [(4096, 138, False), (8192, 138, True), (8192, 272, False),
                                       (8192, 544, False), (8500, 272, True)])
 def test_16_bit_solves_keep_k_where_that_pays(dev, n, l, kept):
