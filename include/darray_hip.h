@@ -196,7 +196,8 @@ int dh_trsm_f32(dh_handle_t h, char side, char uplo, char transa, char diag, int
                 float alpha, const float* A, int lda, float* B, int ldb);
 
 /* Right-looking blocked Cholesky A = U^T U of the n x n upper triangle, block bs
- * (cholesky_factorize, lapack_like.h:9-56: potrf(A11) -> trsm(L,U,T) -> syrk).
+ * (cholesky_factorize, lapack_like.h:9-56: potrf(A11) -> trsm(L,U,T) -> syrk);
+ * bs <= 0 means 256, more than 512 means 512.
  * The strict lower triangle is never written.  Returns 0 or info > 0, the
  * global 1-based order of the first non-positive pivot; A is then partially
  * factored (lapack_like.h:25-28).  Synchronises.  uplo must be 'U'.

@@ -827,3 +827,50 @@ def test_rbf_project_f64_wide_fills_the_gpu_with_few_rows():
     best(600000, 20, 1000)
     assert h.workspace_bytes() < 3 * 2**30
     h.close()
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("n,bs,bad", [(600, 600, 0), (1100, 1024, 0), (1100, 5000, 1090),
+                                      (2501, 2501, 0), (2501, 100, 0), (2503, 100, 2301),
+                                      (2501, 40, 0)])
+def test_potrf_wide_and_odd_panels(dev, n, bs, bad, f32):
+    """Panels wider than the kernels take at once, and panel widths that are not
+    whole stages of the trailing update's copies at sizes that otherwise use it.
+    Backward error as in test_potrf_block_edges."""
+    import torch
+    dt, u = (torch.float32, 2.0**-24) if f32 else (torch.float64, 2.0**-53)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    M = torch.randn((n, n + 8), dtype=torch.float64, device="cuda", generator=g)
+    A = (M @ M.t() / n + torch.eye(n, dtype=torch.float64, device="cuda")).to(dt)
+    K = A.clone()
+    if bad:
+        K[bad - 1, bad - 1] = -1.0
+        assert dev.potrf(K, bs) == bad
+        return
+    assert dev.potrf(K, bs) == 0
+    U = torch.tril(K).double()
+    err = (U @ U.t() - A.double()).norm()
+    assert float(err) <= (n + 1) * u * float(torch.trace(A.double()))
+
+
+def test_potrf_with_one_panel_is_as_fast_as_with_several(dev):
+    import time
+
+    import torch
+    n = 4096
+    g = torch.Generator(device="cuda").manual_seed(1)
+    M = torch.randn((n, 64), dtype=torch.float64, device="cuda", generator=g)
+    A = M @ M.t() + n * torch.eye(n, dtype=torch.float64, device="cuda")
+    K = A.clone()
+
+    def best(bs):
+        ts = []
+        for _ in range(6):
+            K.copy_(A)
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            assert dev.potrf(K, bs) == 0
+            ts.append(time.perf_counter() - t0)
+        return min(ts)
+
+    assert best(n) < 1.5 * best(256)
