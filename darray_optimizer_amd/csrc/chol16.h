@@ -39,9 +39,9 @@ __device__ __forceinline__ void gather_rows(double v, double (&out)[4]) {
     out[3] = __hiloint2double((int)h13[1], (int)l13[1]);
 }
 
-// 1/sqrt(piv): hardware estimate and two Newton steps.
+// 1/sqrt(piv): hardware estimate and two Newton steps; 0 for infinity.
 __device__ __forceinline__ double rsqrt_newton(double piv) {
-    const double hp = 0.5 * piv;
+    const double hp = 0.5 * fmin(piv, 0x1.fffffffffffffp+1023);  // finite beside an estimate of 0
     double y = __builtin_amdgcn_rsq(piv);
     y = fma(y, fma(-hp * y, y, 0.5), y);
     return fma(y, fma(-hp * y, y, 0.5), y);
@@ -54,7 +54,7 @@ __device__ __forceinline__ double rsqrt_newton(double piv) {
 // 4 x 4 diagonal block for itself (uniform values) and solves the four rows at
 // its own column, so the chain of square roots crosses no lanes; then d[b] =
 // the lane's row is the operand of one MFMA that updates all later rows (rows
-// up to 4b+3 masked).  An FP64 MFMA is a chain of FMAs in ascending k, so each
+// and columns up to 4b+3 masked).  An FP64 MFMA is a chain of FMAs in ascending k, so each
 // element gets fma(-u_k, u_k', a) once per step k, as column by column.
 // Returns 0, or the 1-based step of the first pivot p with !(p > tol) among
 // the first nreal.  About 450 cycles per four rows; a step per row with
@@ -90,7 +90,10 @@ __device__ __forceinline__ int chol16(dh_d4& d, int g, int li, int nreal, double
         u = g == 2 ? a[2] : u;
         u = g == 3 ? a[3] : u;
         d[b] = u;
-        if (b < 3) d = Mfma<double>::op(li > 4 * b + 3 ? -u : 0.0, u, d);
+        // Columns up to 4b+3 of both operands masked: an infinite pivot's inf / inf
+        // stays where it is.
+        const double v = li > 4 * b + 3 ? u : 0.0;
+        if (b < 3) d = Mfma<double>::op(-v, v, d);
     }
     return bad;
 }

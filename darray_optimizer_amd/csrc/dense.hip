@@ -498,7 +498,8 @@ __global__ __launch_bounds__(256) void potrf64_kernel(int nb, int depth, T* __re
             double dg = d[0];
 #pragma unroll
             for (int r = 1; r < 4; ++r) dg = (li >> 2) == r ? d[r] : dg;
-            if (g == (li & 3)) sRd[li] = 1.0 / dg;
+            // NaN stands for an infinite pivot (inf / inf), whose row is zero.
+            if (g == (li & 3)) sRd[li] = dg == dg ? 1.0 / dg : 0.0;
         }
         wave_lds_sync();
         double x[16];  // column li of the inverse, by back substitution

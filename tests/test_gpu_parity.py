@@ -874,3 +874,23 @@ def test_potrf_with_one_panel_is_as_fast_as_with_several(dev):
         return min(ts)
 
     assert best(n) < 1.5 * best(256)
+
+
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("n,at", [(50, 20), (200, 0), (700, 150), (700, 600)])
+def test_potrf_with_an_infinite_diagonal_entry(dev, n, at, f32):
+    """An infinite pivot is positive: its row of U is zero beside the diagonal (inf /
+    inf there) and the other rows are the Cholesky factor of the rest."""
+    import torch
+    dt, u = (torch.float32, 2.0**-24) if f32 else (torch.float64, 2.0**-53)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    M = torch.randn((n, n + 8), dtype=torch.float64, device="cuda", generator=g)
+    A = (M @ M.t() / n + torch.eye(n, dtype=torch.float64, device="cuda")).to(dt)
+    K = A.clone()
+    K[at, at] = float("inf")
+    assert dev.potrf(K) == 0
+    L = torch.tril(K).double()  # U^T
+    assert bool(torch.isnan(L[at, at])) and bool((L[at + 1:, at] == 0).all())
+    keep = [i for i in range(n) if i != at]
+    L, B = L[keep][:, keep], A.double()[keep][:, keep]
+    assert float((L @ L.t() - B).norm()) <= (n + 1) * u * float(torch.trace(B))
