@@ -509,8 +509,10 @@ __global__ __launch_bounds__(256) void form_f64_kernel(int m, int n, int d,
             double kv[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                double d2 = nrow + nj[min(16 * t + 4 * r + g, n - 1)] - 2.0 * acc[a][b][r];
-                d2 = d2 > 0.0 ? d2 : 0.0;
+                const int i = 16 * rb + li, j = 16 * t + 4 * r + g;
+                double d2 = nrow + nj[min(j, n - 1)] - 2.0 * acc[a][b][r];
+                // Past the last point 1, which a negative gamma cannot take to infinity.
+                d2 = d2 > 0.0 && i < m && j < n ? d2 : 0.0;
                 kv[r] = exp(-gamma * d2);
             }
             store_kept(kv, rb, t, nch, nrb, SYM && bi != bj, sT[wave], Kk);

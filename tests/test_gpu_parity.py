@@ -894,3 +894,21 @@ def test_potrf_with_an_infinite_diagonal_entry(dev, n, at, f32):
     keep = [i for i in range(n) if i != at]
     L, B = L[keep][:, keep], A.double()[keep][:, keep]
     assert float((L @ L.t() - B).norm()) <= (n + 1) * u * float(torch.trace(B))
+
+
+def test_rbf_project_f64_wide_with_negative_gamma(dev):
+    """d > 256 with far but close-lying points: K = exp(+|xi - xj|^2) is finite, and
+    the padding of the columns (17 -> 32) must not bring an infinity in.
+    Tolerance: distances off by (d + 4) u 4 s on either side, s the largest norm."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(3)
+    d, n, l, u = 300, 17, 5, 2.0**-53
+    X = 1.5 + 0.01 * torch.randn((n, d), dtype=torch.float64, device="cuda", generator=g)
+    O = torch.randn((l, n), dtype=torch.float64, device="cuda", generator=g)
+    Y, Q, W = (torch.empty_like(O) for _ in range(3))
+    dev.rbf_project_f64(X, X, O, -1.0, Y)
+    K = torch.exp((X[:, None, :] - X[None, :, :]).pow(2).sum(2))
+    s = float((X * X).sum(1).max())  # about 700
+    tol = 2 * (4 * (d + 4) * s + n + 4) * u * float(K.max() * O.abs().sum(1).max())
+    assert float((Y.t() - K @ O.t().contiguous()).abs().max()) <= tol
+    assert dev.lra(X, O, -1.0, 0, Q, W) == 0 and bool(torch.isfinite(W).all())
