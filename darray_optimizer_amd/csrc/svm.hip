@@ -10,9 +10,9 @@
 //
 // Per CG iteration Z is read twice (Z^T p by row chunks and column groups,
 // then Z v by rows), 2 n k 8 bytes, in four launches: the new direction and
-// Z^T p, the sum of its chunks, Z v and p.q, the update.  All reductions are
-// per-workgroup partial sums combined in a fixed order, so results are
-// deterministic.  Scalars of the CG recurrence stay on the device, and so
+// Z^T p, the sum of its chunks, Z v and p.q, the update (six from 1024 row blocks
+// on, see cg_loop).  All reductions are per-workgroup partial sums combined in a
+// fixed order, so results are deterministic.  Scalars of the CG recurrence stay on the device, and so
 // does the stopping test: the kernel that starts an iteration ends the one
 // before it, and every later kernel of a stopped loop returns at once, so the
 // host queues iterations in batches and reads the state once per batch (the
@@ -93,48 +93,52 @@ __device__ CgState cg_next(const CgState old, int nblk, const double* __restrict
 
 // part[c * nchunks + chunk] = sum over the chunk's rows of Z[r, c] * xv, xv the
 // lane's values of rows chunk * kRows + lane + 64 i, for the workgroup's
-// kColGrp columns.  A wave has all its 8 columns in flight at once (one round
-// trip to memory instead of eight), and reduces them together: each exchange
-// of the butterfly hands half of the columns to the other half of the lanes, 10
-// shuffles instead of 48 with the same pairs in every sum.
+// kColGrp columns, 8 per wave, NC of them in flight at once (one round trip to
+// memory instead of NC) and reduced together: each exchange of the butterfly hands
+// half of the columns to the other half of the lanes, 10 shuffles instead of 48
+// for NC = 8, with the same pairs in every sum.
+template <int NC>
 __device__ __forceinline__ void ztx_columns(int n, int k, const double* __restrict__ Z, int ldz,
                                             const double (&xv)[4], double* __restrict__ part) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int chunk = blockIdx.x, nchunks = gridDim.x, r0 = chunk * kRows + lane;
-    constexpr int NC = kColGrp / 4;
-    static_assert(NC == 8, "the exchanges below reduce eight columns");
-    const int c0 = blockIdx.y * kColGrp + wave;  // columns c0 + 4 u
-    double s[NC], z[NC][4];
+    static_assert(kColGrp / 4 % NC == 0 && (NC & (NC - 1)) == 0, "columns of a wave");
+    for (int u0 = 0; u0 < kColGrp / 4; u0 += NC) {
+        const int c0 = blockIdx.y * kColGrp + wave + 4 * u0;  // columns c0 + 4 u
+        if (c0 >= k) break;
+        double s[NC], z[NC][4];
 #pragma unroll
-    for (int u = 0; u < NC; ++u) {
-        const double* zc = Z + (size_t)min(c0 + 4 * u, k - 1) * ldz;
+        for (int u = 0; u < NC; ++u) {
+            const double* zc = Z + (size_t)min(c0 + 4 * u, k - 1) * ldz;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) z[u][i] = zc[min(r0 + 64 * i, n - 1)];
+            for (int i = 0; i < 4; ++i) z[u][i] = zc[min(r0 + 64 * i, n - 1)];
+        }
+#pragma unroll
+        for (int u = 0; u < NC; ++u) {
+            s[u] = 0.0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[u] += (r0 + 64 * i < n ? z[u][i] : 0.0) * xv[i];
+        }
+        int u = 0;  // column of s[0] after the exchanges
+#pragma unroll
+        for (int o = 32, m = NC / 2; m > 0; o >>= 1, m >>= 1) {
+            const bool up = (lane & o) != 0;
+            u += up ? m : 0;
+#pragma unroll
+            for (int e = 0; e < NC / 2; ++e)
+                if (e < m) {
+                    const double mine = up ? s[e + m] : s[e], other = up ? s[e] : s[e + m];
+                    s[e] = mine + __shfl_xor(other, o);
+                }
+        }
+#pragma unroll
+        for (int o = 32 / NC; o > 0; o >>= 1) s[0] += __shfl_xor(s[0], o);
+        const int c = c0 + 4 * u;
+        if ((lane & (64 / NC - 1)) == 0 && c < k) part[(size_t)c * nchunks + chunk] = s[0];
     }
-#pragma unroll
-    for (int u = 0; u < NC; ++u) {
-        s[u] = 0.0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) s[u] += (r0 + 64 * i < n ? z[u][i] : 0.0) * xv[i];
-    }
-    int u = 0;  // column of s[0] after the exchanges
-#pragma unroll
-    for (int o = 32, m = NC / 2; m > 0; o >>= 1, m >>= 1) {
-        const bool up = (lane & o) != 0;
-        u += up ? m : 0;
-#pragma unroll
-        for (int e = 0; e < NC / 2; ++e)
-            if (e < m) {
-                const double mine = up ? s[e + m] : s[e], other = up ? s[e] : s[e + m];
-                s[e] = mine + __shfl_xor(other, o);
-            }
-    }
-#pragma unroll
-    for (int o = 4; o > 0; o >>= 1) s[0] += __shfl_xor(s[0], o);
-    const int c = c0 + 4 * u;
-    if ((lane & 7) == 0 && c < k) part[(size_t)c * nchunks + chunk] = s[0];
 }
 
+template <int NC>
 __global__ __launch_bounds__(256) void ztx_partial_kernel(int n, int k, const double* __restrict__ Z,
                                                           int ldz, const double* __restrict__ x,
                                                           double* __restrict__ part) {
@@ -142,43 +146,57 @@ __global__ __launch_bounds__(256) void ztx_partial_kernel(int n, int k, const do
     double xv[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) xv[i] = r0 + 64 * i < n ? x[r0 + 64 * i] : 0.0;
-    ztx_columns(n, k, Z, ldz, xv, part);
+    ztx_columns<NC>(n, k, Z, ldz, xv, part);
 }
 
 // The start of a CG iteration: ends the one before it (state `in` -> `out`,
 // beta = (r.z)_new / (r.z), p = z + beta p_old), then Z^T p by chunks.  Every
 // workgroup of a chunk forms the chunk's p; those of column group 0 store it.
-// FIRST: the state and p are those of `in` and `p_old` (out and p_new unused).
-template <bool FIRST>
+// kFirst: the state and p are those of `in` and `p_old` (out and p_new unused);
+// kEnded: cg_state_kernel has ended the iteration before already.
+enum CgStart { kFirst, kEnds, kEnded };
+
+template <CgStart START, int NC>
 __global__ __launch_bounds__(256) void cg_begin_kernel(
     int n, int k, const double* __restrict__ Z, int ldz, int nblk,
     const double* __restrict__ part2, const double* __restrict__ z,
     const double* __restrict__ p_old, double* __restrict__ p_new, double* __restrict__ part,
     const CgState* __restrict__ in, CgState* __restrict__ out, double tol, int max_iter) {
-    CgState old = *in, st = old;
+    CgState old = *in, st = START == kEnded ? *out : old;
     const bool lead = blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0;
-    if (!FIRST) {
+    if (START == kEnds) {
         if (old.active != 0.0) st = cg_next(old, nblk, part2, tol, max_iter);
         if (lead) *out = st;
     }
     if (st.active == 0.0) return;
     const int r0 = blockIdx.x * kRows + (threadIdx.x & 63);
-    const double beta = FIRST ? 0.0 : st.rz / old.rz;
+    const double beta = START == kFirst ? 0.0 : st.rz / old.rz;
     double xv[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int r = r0 + 64 * i;
         xv[i] = 0.0;
         if (r < n) {
-            xv[i] = FIRST ? p_old[r] : z[r] + beta * p_old[r];
-            if (!FIRST && blockIdx.y == 0 && (threadIdx.x >> 6) == i) p_new[r] = xv[i];
+            xv[i] = START == kFirst ? p_old[r] : z[r] + beta * p_old[r];
+            if (START != kFirst && blockIdx.y == 0 && (threadIdx.x >> 6) == i) p_new[r] = xv[i];
         }
     }
-    ztx_columns(n, k, Z, ldz, xv, part);
+    ztx_columns<NC>(n, k, Z, ldz, xv, part);
+}
+
+// Ends an iteration by one workgroup, for many of them to read the state.
+__global__ __launch_bounds__(256) void cg_state_kernel(int nblk, const double* __restrict__ part2,
+                                                       const CgState* __restrict__ in,
+                                                       CgState* __restrict__ out, double tol,
+                                                       int max_iter) {
+    CgState st = *in;
+    if (st.active != 0.0) st = cg_next(st, nblk, part2, tol, max_iter);
+    if (threadIdx.x == 0) *out = st;
 }
 
 // The end of a batch: as cg_begin_kernel without the product, so that the host
 // can read the state.
+template <CgStart START>
 __global__ __launch_bounds__(256) void cg_end_kernel(int n, int nblk,
                                                      const double* __restrict__ part2,
                                                      const double* __restrict__ z,
@@ -187,9 +205,11 @@ __global__ __launch_bounds__(256) void cg_end_kernel(int n, int nblk,
                                                      const CgState* __restrict__ in,
                                                      CgState* __restrict__ out, double tol,
                                                      int max_iter) {
-    CgState old = *in, st = old;
-    if (old.active != 0.0) st = cg_next(old, nblk, part2, tol, max_iter);
-    if (blockIdx.x == 0 && threadIdx.x == 0) *out = st;
+    CgState old = *in, st = START == kEnded ? *out : old;
+    if (START == kEnds) {
+        if (old.active != 0.0) st = cg_next(old, nblk, part2, tol, max_iter);
+        if (blockIdx.x == 0 && threadIdx.x == 0) *out = st;
+    }
     if (st.active == 0.0) return;
     const double beta = st.rz / old.rz;
     const int i = blockIdx.x * kRows + threadIdx.x;
@@ -314,10 +334,9 @@ __global__ __launch_bounds__(256) void setup_reduce_kernel(int nblk, const doubl
 
 // q = Z v + D o p; part[w] = p.q over the 64 rows of wave w.  One wave per
 // workgroup and row block, so that n rows spread over n / 64 CUs, with the next
-// kApplyCols columns of Z in flight while these are added up; each row's sum
-// runs over the columns in order, as one thread's chain.
-constexpr int kApplyCols = 64;
-
+// COLS columns of Z in flight while these are added up; each row's sum runs over
+// the columns in order, as one thread's chain.
+template <int COLS>
 __global__ __launch_bounds__(64) void cg_apply_kernel(int n, int k, const double* __restrict__ Z,
                                                       int ldz, const double* __restrict__ v,
                                                       const double* __restrict__ D,
@@ -329,24 +348,22 @@ __global__ __launch_bounds__(64) void cg_apply_kernel(int n, int k, const double
     __shared__ double su[kMaxK];  // v, zero-padded to a whole number of panels
     const int i = blockIdx.x * 64 + threadIdx.x, ic = min(i, n - 1);
     const double* zr = Z + ic;
-    double cur[kApplyCols], nxt[kApplyCols];
+    double cur[COLS], nxt[COLS];
 #pragma unroll
-    for (int u = 0; u < kApplyCols; ++u) cur[u] = zr[(size_t)min(u, k - 1) * ldz];
-    for (int c = threadIdx.x; c < (k + kApplyCols - 1) / kApplyCols * kApplyCols; c += 64)
-        su[c] = c < k ? v[c] : 0.0;
+    for (int u = 0; u < COLS; ++u) cur[u] = zr[(size_t)min(u, k - 1) * ldz];
+    for (int c = threadIdx.x; c < (k + COLS - 1) / COLS * COLS; c += 64) su[c] = c < k ? v[c] : 0.0;
     const double di = D[ic], pi = p[ic];
     __syncthreads();
     double zv = 0.0;
-    for (int c0 = 0; c0 < k; c0 += kApplyCols) {
-        if (c0 + kApplyCols < k) {
+    for (int c0 = 0; c0 < k; c0 += COLS) {
+        if (c0 + COLS < k) {
 #pragma unroll
-            for (int u = 0; u < kApplyCols; ++u)
-                nxt[u] = zr[(size_t)min(c0 + kApplyCols + u, k - 1) * ldz];
+            for (int u = 0; u < COLS; ++u) nxt[u] = zr[(size_t)min(c0 + COLS + u, k - 1) * ldz];
         }
 #pragma unroll
-        for (int u = 0; u < kApplyCols; ++u) zv += cur[u] * su[c0 + u];
+        for (int u = 0; u < COLS; ++u) zv += cur[u] * su[c0 + u];
 #pragma unroll
-        for (int u = 0; u < kApplyCols; ++u) cur[u] = nxt[u];
+        for (int u = 0; u < COLS; ++u) cur[u] = nxt[u];
     }
     double pq = 0.0;
     if (i < n) {
@@ -358,10 +375,36 @@ __global__ __launch_bounds__(64) void cg_apply_kernel(int n, int k, const double
     if (threadIdx.x == 0) part[blockIdx.x] = pq;
 }
 
-// alpha = r.z / p.q (p.q summed from the waves' partials in a fixed order by
-// every workgroup); s += alpha p, r -= alpha q, z = r / Pc; part2[2b..] = (r.z, r.r).
+// The waves' partials of p.q in a fixed order, the same in every workgroup of
+// 256 threads.
+__device__ double sum_pq(int nblk, const double* __restrict__ part_pq) {
+    __shared__ double sh[4];
+    double v = 0.0;
+    for (int b = threadIdx.x; b < nblk; b += 256) {
+        const double* w = part_pq + 4 * (size_t)b;
+        v += (w[0] + w[1]) + (w[2] + w[3]);
+    }
+    v = wave_sum(v);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (lane == 0) sh[wave] = v;
+    __syncthreads();
+    return (sh[0] + sh[1]) + (sh[2] + sh[3]);
+}
+
+// *pq = p.q by one workgroup, for many of them to read.
+__global__ __launch_bounds__(256) void cg_pq_kernel(int nblk, const double* __restrict__ part_pq,
+                                                    double* __restrict__ pq,
+                                                    const CgState* __restrict__ st) {
+    if (cg_stopped(st)) return;
+    const double v = sum_pq(nblk, part_pq);
+    if (threadIdx.x == 0) *pq = v;
+}
+
+// alpha = r.z / p.q (from *pq, or summed from the waves' partials by every
+// workgroup); s += alpha p, r -= alpha q, z = r / Pc; part2[2b..] = (r.z, r.r).
 __global__ __launch_bounds__(256) void cg_update_kernel(int n, int nblk,
                                                         const double* __restrict__ part_pq,
+                                                        const double* __restrict__ pq_sum,
                                                         const double* __restrict__ p,
                                                         const double* __restrict__ q,
                                                         const double* __restrict__ Pc,
@@ -374,17 +417,7 @@ __global__ __launch_bounds__(256) void cg_update_kernel(int n, int nblk,
     __shared__ double sh[4];
     const int i = blockIdx.x * kRows + threadIdx.x, ic = min(i, n - 1);
     const double pi = p[ic], qi = q[ic], pc = Pc[ic], si = s[ic], r0 = r[ic];
-    double v = 0.0;
-    for (int b = threadIdx.x; b < nblk; b += 256) {
-        const double* w = part_pq + 4 * (size_t)b;
-        v += (w[0] + w[1]) + (w[2] + w[3]);
-    }
-    v = wave_sum(v);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane == 0) sh[wave] = v;
-    __syncthreads();
-    const double pq = (sh[0] + sh[1]) + (sh[2] + sh[3]);
-    __syncthreads();  // sh is reused below
+    const double pq = pq_sum ? *pq_sum : sum_pq(nblk, part_pq);
     const double alpha = st->rz / pq;
     double rz = 0.0, rr = 0.0;
     if (i < n) {
@@ -551,10 +584,69 @@ int grab(dh_handle_t h, int n, int k, Work& w) {
     return 0;
 }
 
+// Columns that a wave of Z^T x has in flight: two, which hide as much as eight and
+// leave more waves resident (us per CG iteration with eight, two and one: n = 20000,
+// k = 200 33.7, 31.9, 33.1; n = 1000000, k = 100 470, 426, 426); eight for whole column
+// groups on at most a workgroup per CU (n = 8000, k = 200: 27.2, 27.7); one where Z
+// fills the 256 MB cache and its columns are multiples of 32 KB apart, which fall
+// on the same channels (n = 524288, k = 256: 537, 513, 471).
+int columns_in_flight(dh_handle_t h, const Work& w, int ldz) {
+    if (w.k >= kColGrp && w.nchunks * w.ngrp <= h->num_cu) return 8;
+    return ldz % 4096 == 0 && sizeof(double) * (size_t)w.n * w.k >= (256u << 20) ? 1 : 2;
+}
+
+template <CgStart START>
+void launch_begin(dh_handle_t h, const Work& w, const double* Z, int ldz, const double* p,
+                  double* p_new, const CgState* in, CgState* out, double tol, int max_iter) {
+    const dim3 grid(w.nchunks, w.ngrp);
+#define DH_BEGIN(NC)                                                                          \
+    cg_begin_kernel<START, NC><<<grid, 256, 0, h->stream>>>(w.n, w.k, Z, ldz, w.nblk, w.part2, \
+                                                            w.z, p, p_new, w.ztpart, in, out, \
+                                                            tol, max_iter)
+    switch (columns_in_flight(h, w, ldz)) {
+        case 8:
+            DH_BEGIN(8);
+            break;
+        case 2:
+            DH_BEGIN(2);
+            break;
+        default:
+            DH_BEGIN(1);
+    }
+#undef DH_BEGIN
+}
+
+// Z v with as many columns in flight as pay: 64 where n gives less than two waves
+// per CU, and no more than k fills (n = 20000, k = 200: 33.7 us per iteration with 64,
+// 34.0 with 32, 34.6 with 16; n = 1000000, k = 16: 155, 129, 126; n = 300000, k = 256: 282,
+// 283, 288; n = 100000, k = 100: 56.0, 52.9, 52.2).
+void launch_apply(dh_handle_t h, const Work& w, const double* Z, int ldz, const double* p,
+                  const CgState* st) {
+    const int grid = 4 * w.nblk;
+    if (w.k <= 32)
+        cg_apply_kernel<16><<<grid, 64, 0, h->stream>>>(w.n, w.k, Z, ldz, w.v, w.D, p, w.q, w.part,
+                                                        st);
+    else if (grid < 2 * h->num_cu)
+        cg_apply_kernel<64><<<grid, 64, 0, h->stream>>>(w.n, w.k, Z, ldz, w.v, w.D, p, w.q, w.part,
+                                                        st);
+    else
+        cg_apply_kernel<32><<<grid, 64, 0, h->stream>>>(w.n, w.k, Z, ldz, w.v, w.D, p, w.q, w.part,
+                                                        st);
+}
+
 // out (k) = Z^T x.
 int zt(dh_handle_t h, const Work& w, const double* Z, int ldz, const double* x, double* out) {
-    ztx_partial_kernel<<<dim3(w.nchunks, w.ngrp), 256, 0, h->stream>>>(w.n, w.k, Z, ldz, x,
-                                                                       w.ztpart);
+    const dim3 grid(w.nchunks, w.ngrp);
+    switch (columns_in_flight(h, w, ldz)) {
+        case 8:
+            ztx_partial_kernel<8><<<grid, 256, 0, h->stream>>>(w.n, w.k, Z, ldz, x, w.ztpart);
+            break;
+        case 2:
+            ztx_partial_kernel<2><<<grid, 256, 0, h->stream>>>(w.n, w.k, Z, ldz, x, w.ztpart);
+            break;
+        default:
+            ztx_partial_kernel<1><<<grid, 256, 0, h->stream>>>(w.n, w.k, Z, ldz, x, w.ztpart);
+    }
     DH_CHECK_LAUNCH();
     reduce_cols_kernel<<<dh_cdiv(w.k, 4), 256, 0, h->stream>>>(w.nchunks, w.k, w.ztpart, out,
                                                                nullptr);
@@ -583,37 +675,55 @@ int cg_loop(dh_handle_t h, const Work& w, const double* Z, int ldz, double tol, 
     int it = 0;
     if (std::sqrt(rr) > tol && it < max_iter) {
         CgState *bank = w.st, *other = w.st + kCgBatch + 1;
-        double *p = w.p, *pn = w.p2;
+        double *p = w.p, *pn = w.p2, *pq = w.sc + 8;
         cg_start_kernel<<<1, 64, 0, h->stream>>>(bank, w.sc);
         DH_CHECK_LAUNCH();
-        const dim3 grid(w.nchunks, w.ngrp);
+        // Every workgroup sums all partials by itself, which costs their square in
+        // reads; from 1024 on one workgroup does it in a launch of its own (n =
+        // 1000000, k = 100: 470 -> 411 us per iteration, 300000, 256: 281 -> 274; the
+        // other way 200000, 64: 65 -> 66, 100000, 100: 56 -> 58).
+        const bool sums = w.nblk >= 1024;
         for (;;) {
             const int batch = std::min(kCgBatch, max_iter - it);
             for (int b = 0; b < batch; ++b) {
                 CgState* st = bank + b;
                 if (b == 0) {
-                    cg_begin_kernel<true><<<grid, 256, 0, h->stream>>>(
-                        w.n, w.k, Z, ldz, w.nblk, w.part2, w.z, p, nullptr, w.ztpart, st, nullptr,
-                        tol, max_iter);
+                    launch_begin<kFirst>(h, w, Z, ldz, p, nullptr, st, nullptr, tol, max_iter);
+                } else if (sums) {
+                    cg_state_kernel<<<1, 256, 0, h->stream>>>(w.nblk, w.part2, st - 1, st, tol,
+                                                              max_iter);
+                    DH_CHECK_LAUNCH();
+                    launch_begin<kEnded>(h, w, Z, ldz, p, pn, st - 1, st, tol, max_iter);
+                    std::swap(p, pn);
                 } else {
-                    cg_begin_kernel<false><<<grid, 256, 0, h->stream>>>(
-                        w.n, w.k, Z, ldz, w.nblk, w.part2, w.z, p, pn, w.ztpart, st - 1, st, tol,
-                        max_iter);
+                    launch_begin<kEnds>(h, w, Z, ldz, p, pn, st - 1, st, tol, max_iter);
                     std::swap(p, pn);
                 }
                 DH_CHECK_LAUNCH();
                 reduce_cols_kernel<<<dh_cdiv(w.k, 4), 256, 0, h->stream>>>(w.nchunks, w.k,
                                                                            w.ztpart, w.v, st);
                 DH_CHECK_LAUNCH();
-                cg_apply_kernel<<<4 * w.nblk, 64, 0, h->stream>>>(w.n, w.k, Z, ldz, w.v, w.D, p,
-                                                                  w.q, w.part, st);
+                launch_apply(h, w, Z, ldz, p, st);
                 DH_CHECK_LAUNCH();
-                cg_update_kernel<<<w.nblk, 256, 0, h->stream>>>(w.n, w.nblk, w.part, p, w.q, w.Pc,
+                if (sums) {
+                    cg_pq_kernel<<<1, 256, 0, h->stream>>>(w.nblk, w.part, pq, st);
+                    DH_CHECK_LAUNCH();
+                }
+                cg_update_kernel<<<w.nblk, 256, 0, h->stream>>>(w.n, w.nblk, w.part,
+                                                                sums ? pq : nullptr, p, w.q, w.Pc,
                                                                 w.s, w.r, w.z, w.part2, st);
                 DH_CHECK_LAUNCH();
             }
-            cg_end_kernel<<<w.nblk, 256, 0, h->stream>>>(w.n, w.nblk, w.part2, w.z, p, pn,
-                                                         bank + batch - 1, other, tol, max_iter);
+            if (sums) {
+                cg_state_kernel<<<1, 256, 0, h->stream>>>(w.nblk, w.part2, bank + batch - 1, other,
+                                                          tol, max_iter);
+                DH_CHECK_LAUNCH();
+                cg_end_kernel<kEnded><<<w.nblk, 256, 0, h->stream>>>(
+                    w.n, w.nblk, w.part2, w.z, p, pn, bank + batch - 1, other, tol, max_iter);
+            } else {
+                cg_end_kernel<kEnds><<<w.nblk, 256, 0, h->stream>>>(
+                    w.n, w.nblk, w.part2, w.z, p, pn, bank + batch - 1, other, tol, max_iter);
+            }
             DH_CHECK_LAUNCH();
             std::swap(p, pn);
             std::swap(bank, other);

@@ -129,3 +129,48 @@ def test_svm_on_range_finder_nystrom_factor(dev):
     print(f"svm n={n}: {stats} in {secs:.2f} s, f={f:.6e}, training accuracy {acc:.4f}", flush=True)
     assert np.all(ag > 0) and np.all(ag < Cb)
     assert acc >= 0.95
+
+
+@pytest.mark.parametrize("n,k", [(64, 1), (8000, 200), (8000, 33), (20000, 70), (40000, 17),
+                                 (262144, 20), (261889, 40), (524288, 64), (300000, 100)])
+def test_pcg_over_the_sizes_of_its_kernels(dev, n, k):
+    """Every choice of columns in flight, and the sums by one workgroup (n >= 261889):
+    the true residual of the returned solution meets the tolerance that the
+    recurrence reports, up to the rounding of b - (Z Z^T + D) x, whose terms are
+    at most a few |b| here: |Z Z^T| <= 4 in norm, 1 <= D <= 2, n + k operations."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    Z = torch.randn((k, n), dtype=torch.float64, device="cuda", generator=g) / n**0.5
+    D = 1.0 + torch.rand(n, dtype=torch.float64, device="cuda", generator=g)
+    b = torch.randn(n, dtype=torch.float64, device="cuda", generator=g)
+    x = torch.zeros(n, dtype=torch.float64, device="cuda")
+    nb = float(b.norm())
+    it, rnorm = dev.svm_pcg(Z, D, b, x, tol=1e-9 * nb, max_iter=200)
+    res = float((b - (Z.t() @ (Z @ x)) - D * x).norm())
+    assert 0 < it < 200 and rnorm <= 1e-9 * nb
+    assert res <= 1e-9 * nb + 8 * (n + k) * 2.0**-53 * nb
+
+
+def test_pcg_time_grows_with_n_and_not_its_square():
+    import time
+
+    import torch
+    h = dh.Handle(0)
+
+    def best(n):
+        Z = torch.rand((2, n), dtype=torch.float64, device="cuda")
+        D, b = torch.ones(n, dtype=torch.float64, device="cuda"), Z[0].clone()
+        x = torch.zeros_like(D)
+        ts = []
+        for _ in range(4):
+            x.zero_()
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            h.svm_pcg(Z, D, b, x, tol=0.0, max_iter=32)
+            ts.append(time.perf_counter() - t0)
+        return min(ts)
+
+    a, b = best(1000000), best(4000000)
+    print(f"pcg: {a * 1e6 / 32:.1f} and {b * 1e6 / 32:.1f} us per iteration", flush=True)
+    assert b < 4.5 * a
+    h.close()
