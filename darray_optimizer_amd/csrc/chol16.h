@@ -39,9 +39,11 @@ __device__ __forceinline__ void gather_rows(double v, double (&out)[4]) {
     out[3] = __hiloint2double((int)h13[1], (int)l13[1]);
 }
 
-// 1/sqrt(piv): hardware estimate and two Newton steps; 0 for infinity.
+// 1/sqrt(piv): hardware estimate and two Newton steps; INF: 0 for infinity (NaN
+// without it).
+template <bool INF>
 __device__ __forceinline__ double rsqrt_newton(double piv) {
-    const double hp = 0.5 * fmin(piv, 0x1.fffffffffffffp+1023);  // finite beside an estimate of 0
+    const double hp = 0.5 * (INF ? fmin(piv, 0x1.fffffffffffffp+1023) : piv);
     double y = __builtin_amdgcn_rsq(piv);
     y = fma(y, fma(-hp * y, y, 0.5), y);
     return fma(y, fma(-hp * y, y, 0.5), y);
@@ -54,11 +56,14 @@ __device__ __forceinline__ double rsqrt_newton(double piv) {
 // 4 x 4 diagonal block for itself (uniform values) and solves the four rows at
 // its own column, so the chain of square roots crosses no lanes; then d[b] =
 // the lane's row is the operand of one MFMA that updates all later rows (rows
-// and columns up to 4b+3 masked).  An FP64 MFMA is a chain of FMAs in ascending k, so each
+// up to 4b+3 masked).  An FP64 MFMA is a chain of FMAs in ascending k, so each
 // element gets fma(-u_k, u_k', a) once per step k, as column by column.
 // Returns 0, or the 1-based step of the first pivot p with !(p > tol) among
-// the first nreal.  About 450 cycles per four rows; a step per row with
-// broadcasts of the row took 300 per row.
+// the first nreal.  INF: an infinite pivot gives a row of zeros with inf / inf on
+// the diagonal, which stays there (finished columns are masked too); without it
+// the row and the pivots after it are NaN.  About 450 cycles per four rows; a
+// step per row with broadcasts of the row took 300 per row.
+template <bool INF = false>
 __device__ __forceinline__ int chol16(dh_d4& d, int g, int li, int nreal, double tol) {
     int bad = 0;  // no early exit: what follows a failed pivot is not used
 #pragma unroll
@@ -74,7 +79,7 @@ __device__ __forceinline__ int chol16(dh_d4& d, int g, int li, int nreal, double
         for (int r = 0; r < 4; ++r) {
             const int kk = 4 * b + r;
             bad = bad == 0 && kk < nreal && !(m[r][r] > tol) ? kk + 1 : bad;
-            const double y = rsqrt_newton(m[r][r]);
+            const double y = rsqrt_newton<INF>(m[r][r]);
             a[r] *= y;
 #pragma unroll
             for (int c = r + 1; c < 4; ++c) m[r][c] *= y;
@@ -90,10 +95,8 @@ __device__ __forceinline__ int chol16(dh_d4& d, int g, int li, int nreal, double
         u = g == 2 ? a[2] : u;
         u = g == 3 ? a[3] : u;
         d[b] = u;
-        // Columns up to 4b+3 of both operands masked: an infinite pivot's inf / inf
-        // stays where it is.
-        const double v = li > 4 * b + 3 ? u : 0.0;
-        if (b < 3) d = Mfma<double>::op(-v, v, d);
+        const bool later = li > 4 * b + 3;
+        if (b < 3) d = Mfma<double>::op(later ? -u : 0.0, INF && !later ? 0.0 : u, d);
     }
     return bad;
 }

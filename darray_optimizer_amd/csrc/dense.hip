@@ -488,7 +488,12 @@ __global__ __launch_bounds__(256) void potrf64_kernel(int nb, int depth, T* __re
     }
     // U_kk and its inverse from block (k, k) in accumulator layout, by wave 0.
     auto factor_diag = [&](int k, dh_d4 d) {
-        const int bad = chol16(d, g, li, nb - 16 * k, 0.0);
+        const dh_d4 d0 = d;
+        int bad = chol16(d, g, li, 16, 0.0);
+        if (bad) {  // a pivot that is not positive, or an infinite one before it
+            d = d0;
+            bad = chol16<true>(d, g, li, nb - 16 * k, 0.0);
+        }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             sU[g + 4 * r][li] = d[r];

@@ -877,7 +877,8 @@ def test_potrf_with_one_panel_is_as_fast_as_with_several(dev):
 
 
 @pytest.mark.parametrize("f32", [False, True])
-@pytest.mark.parametrize("n,at", [(50, 20), (200, 0), (700, 150), (700, 600)])
+@pytest.mark.parametrize("n,at", [(50, 20), (50, 48), (50, 49), (64, 15), (200, 0), (200, 63),
+                                  (700, 150), (700, 600), (700, 699)])
 def test_potrf_with_an_infinite_diagonal_entry(dev, n, at, f32):
     """An infinite pivot is positive: its row of U is zero beside the diagonal (inf /
     inf there) and the other rows are the Cholesky factor of the rest."""
