@@ -165,8 +165,9 @@ static int gemm_stop(dh_handle_t h, bool ta, bool tb, int m, int n, int k, T alp
         return 0;
     }
     // FP64 keeps 64 x 64 tiles (90 registers, five waves per SIMD): its 128 x 128
-    // tile (238 registers, two waves) measured slower in the blocked Cholesky
-    // (FP64 posv at n = 16384: 57.3 ms against 51.6 ms).
+    // tile (238 registers, two waves) measured slower as the trailing update of
+    // the blocked Cholesky, which has update_tn_kernel now (FP64 posv at n = 16384:
+    // 57.3 ms against 51.6 ms).
     if (sizeof(T) == 4 && (long)m * n >= 2048L * 2048L)
         return launch_gemm<T, 128, 128>(h, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc,
                                         uplo, stop);
