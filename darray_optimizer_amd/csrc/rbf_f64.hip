@@ -749,7 +749,9 @@ static int block_rows(int m, int n) {
 // (dkernel.cu:144-178).  With `keep` K is one block there: kmode 1 forms it,
 // from one triangle where both point sets are the same; kmode 2 takes it as an
 // earlier pass left it.  The j range is split until a row block has two
-// workgroups per CU, also where K is kept, so that both return the same bits.
+// workgroups per CU, into parts of at least four chunks of 32 points (2000 x 2000, d =
+// 300, l = 272: 145 us, with parts of 16 chunks 255, through the GEMM 155), also where
+// K is kept, so that both return the same bits.
 // (Column-major blocks through the 64 x 64 GEMM: n = 9000, d = 600, l = 74 took
 // 2.13 + 0.49 ms per pass; forming one triangle takes 1.07 and a pass 0.33.
 // One pass over row blocks, d = 300, l = 74, GEMM -> here, and with the split
@@ -771,7 +773,7 @@ static int project_f64_blocked(dh_handle_t h, int m, int n, int d, int l, const 
     kept_columns(l, &ncb, &groups);
     const int nch = dh_cdiv(n, 32);
     int splits = 1;
-    while ((long)dh_cdiv(rows, 64) * groups * splits < 2L * h->num_cu && nch >= 32 * splits)
+    while ((long)dh_cdiv(rows, 64) * groups * splits < 2L * h->num_cu && nch >= 8 * splits)
         splits *= 2;
     const int jps = splits == 1 ? n : dh_cdiv(nch, splits) * 32;
     splits = dh_cdiv(n, jps);

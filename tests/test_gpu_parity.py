@@ -913,3 +913,24 @@ def test_rbf_project_f64_wide_with_negative_gamma(dev):
     tol = 2 * (4 * (d + 4) * s + n + 4) * u * float(K.max() * O.abs().sum(1).max())
     assert float((Y.t() - K @ O.t().contiguous()).abs().max()) <= tol
     assert dev.lra(X, O, -1.0, 0, Q, W) == 0 and bool(torch.isfinite(W).all())
+
+
+def test_rbf_project_f64_wide_fills_the_gpu_with_few_points():
+    """2000 x 2000: 32 row tiles, so the j range goes in eight parts, whose partial
+    products (beside K and the packed panel) are held.  n products in any order and
+    distances off by (d + 4) u 4 s, s <= 1, on either side."""
+    import torch
+    h = dh.Handle(0)
+    n, d, l, gamma, u = 2000, 300, 272, 0.7, 2.0**-53
+    g = torch.Generator(device="cuda").manual_seed(4)
+    X = torch.rand((n, d), dtype=torch.float64, device="cuda", generator=g).div_(d**0.5)
+    O = torch.randn((l, n), dtype=torch.float64, device="cuda", generator=g)
+    Y = torch.empty_like(O)
+    h.rbf_project_f64(X, X, O, gamma, Y)
+    s = (X * X).sum(1)
+    K = torch.exp(-gamma * (s[:, None] + s[None, :] - 2.0 * (X @ X.t())).clamp(min=0.0))
+    Ot = O.t().contiguous()
+    tol = 2 * (gamma * 4 * (d + 4) + n + 4) * u * (K @ Ot.abs())
+    assert bool(((Y.t() - K @ Ot).abs() <= tol).all())
+    assert h.workspace_bytes() >= 8 * (n * n + n * l + 8 * n * l)
+    h.close()
