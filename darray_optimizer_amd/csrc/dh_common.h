@@ -58,7 +58,7 @@ struct dh_handle_s {
     // (queried on the handle's device on first use; handle.hip).
     void* occupancy = nullptr;
     size_t alloc_limit = 0;  // dh_debug_alloc_limit
-    bool no_scratch = false, scratch_used = false;  // ScratchHold
+    bool no_scratch = false, scratch_used = false, scratch_asked = false;  // ScratchHold
 };
 
 // Creates h->aux and its events if they do not exist yet.
@@ -125,12 +125,17 @@ void* dh_scratch_take(int device, size_t bytes);
 void dh_scratch_release(int device);
 
 // The device's scratch buffer for the length of a call (p = nullptr: not
-// available, not asked for, or the handle does without it).
+// available, not asked for, or the handle does without it).  fresh = false: a new
+// buffer is not worth its allocation and release for one call; the handle takes
+// one from its second such call on, as others will follow.
 struct ScratchHold {
     dh_handle_t h;
-    void* p;
-    ScratchHold(dh_handle_t h_, size_t bytes)
-        : h(h_), p(bytes && !h_->no_scratch ? dh_scratch_take(h_->device, bytes) : nullptr) {
+    void* p = nullptr;
+    ScratchHold(dh_handle_t h_, size_t bytes, bool fresh = true) : h(h_) {
+        if (bytes == 0 || h->no_scratch) return;
+        if (fresh || h->scratch_asked || dh_scratch_bytes(h) >= bytes)
+            p = dh_scratch_take(h->device, bytes);
+        h->scratch_asked = true;
         if (p) h->scratch_used = true;
     }
     ~ScratchHold() {

@@ -384,7 +384,13 @@ static int lra_f64(dh_handle_t h, int n, int d, int l, int q, const double* X, i
     double* nrm = (double*)dh_ws(h, DH_WS_NORMS, sizeof(double) * (size_t)n);
     if (!nrm) return DH_ERR_ALLOC;
     DH_CHECK_STATUS(dh_sqnorms_f64(h, n, d, X, ldx, nrm));
-    const ScratchHold kk(h, dh_kkeep_bytes(h, n, d, l, q));
+    // Allocating and freeing a buffer of more than 64 MB takes about 0.3 ms, which a
+    // single solve has to gain (with a handle per solve: n = 4096, d = 64, l = 100, q = 1
+    // 1.13 ms and 1.07 without; d = 256, l = 200, q = 2 3.1 and 3.7; n = 5000, d = 64, l =
+    // 100, q = 1 1.54 and 1.69; n = 3000, d = l = 16, q = 0 0.58 and 0.31).
+    const size_t bytes = dh_kkeep_bytes(h, n, d, l, q);
+    const double gain = (q + 1.0) * n * n * (d <= 32 ? 32 : d <= 64 ? 64 : d <= 128 ? 128 : 256);
+    const ScratchHold kk(h, bytes, bytes <= (64u << 20) || d > 256 || gain > 2.8e9);
     const int form = kk.p ? 1 : 0, use = kk.p ? 2 : 0;
     DH_CHECK_STATUS(dh_project_f64_split(h, n, n, d, l, X, ldx, X, ldx, nrm, nrm, y, y, gamma,
                                         Omega, ldo, Q, ldq, kk.p, form));

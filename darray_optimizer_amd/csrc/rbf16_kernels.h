@@ -679,6 +679,7 @@ int dh_project_fp8(dh_handle_t h, int dpad8, int ncb, int groups, int m, int nch
 // pass that reads it (rbf16_kept.hip).
 bool dh_kept16_pays(int n, int dpad, bool fp8, int ncb, int groups, int passes);
 size_t dh_kept16_bytes(int m, int nchunks);
+bool dh_kept16_fresh(int n, size_t bytes);
 int dh_form16(dh_handle_t h, bool f16, bool fp8, int dpad, int m, int nchunks, const bf16x8* Xi,
               const bf16x8* Xj, const float* ai, const float* bj, const float* si,
               const float* sj, float c2, void* keep);

@@ -575,7 +575,8 @@ int lra_16_passes(dh_handle_t h, int n, int d, int l, int q, const double* X, in
     const Bf16Cols cols = bf16_cols(l);
     const int nch = dh_cdiv(n, 32);
     const bool pays = dh_kept16_pays(n, dpad_of(d), false, cols.ncb, cols.groups, q + 2);
-    const ScratchHold kk(h, pays ? dh_kept16_bytes(n, nch) : 0);
+    const size_t bytes = pays ? dh_kept16_bytes(n, nch) : 0;
+    const ScratchHold kk(h, bytes, dh_kept16_fresh(n, bytes));
     if (kk.p)
         DH_CHECK_STATUS(dh_form16(h, F16, false, dpad_of(d), n, nch, (const bf16x8*)p.xb,
                                   (const bf16x8*)p.xb, p.a, p.a, nullptr, nullptr, c2, kk.p));
@@ -630,7 +631,8 @@ int dh_lra_fp8_passes(dh_handle_t h, int n, int d, int l, int q, const double* X
     const Bf16Cols cols = bf16_cols(l);
     const int nch = dh_cdiv(n, 32);
     const bool pays = dh_kept16_pays(n, dpad8_of(d), true, cols.ncb, cols.groups, q + 2);
-    const ScratchHold kk(h, pays ? dh_kept16_bytes(n, nch) : 0);
+    const size_t bytes = pays ? dh_kept16_bytes(n, nch) : 0;
+    const ScratchHold kk(h, bytes, dh_kept16_fresh(n, bytes));
     if (kk.p)
         DH_CHECK_STATUS(dh_form16(h, false, true, dpad8_of(d), n, nch, (const bf16x8*)p.xb,
                                   (const bf16x8*)p.xb, p.a, p.a, p.sinv, p.sinv, c2, kk.p));

@@ -15,6 +15,7 @@ def nothing_unwiped(dev):
 
     import torch
     wait = torch.cuda.get_device_properties(0).total_memory / 8 / 25e9
+    solve(dev, *problem(300, 8, 8)[:2])  # a handle's first solve may do without a buffer
     dev.scratch_trim()
     time.sleep(wait)
     yield
@@ -71,6 +72,7 @@ def test_allocations_take_the_idle_scratch_back(limit):
     import torch
     h = dh.Handle(0)
     X, Om, _ = problem(3000, 40, 24)
+    solve(h, X, Om)
     solve(h, X, Om)
     size = h.scratch_bytes()
     assert size >= 8 * 3000 * 3000
@@ -214,6 +216,24 @@ def test_f64_keeps_k_where_that_pays(dev, n, d, l, q, kept):
     dev.scratch_trim()
     solve(dev, X, Om, q)
     assert (dev.scratch_bytes() > 0) == kept
+
+
+@pytest.mark.parametrize("n,d,l,q,first", [(3000, 16, 16, 0, False), (4096, 64, 100, 1, False),
+                                           (4096, 256, 16, 2, True), (2048, 16, 16, 0, True),
+                                           (3000, 300, 16, 0, True), (8192, 64, 138, 1, True)])
+def test_a_handles_first_solve_takes_a_buffer_where_it_alone_pays(dev, n, d, l, q, first):
+    """Allocation and release of more than 64 MB take as long as a small solve gains,
+    so a program with a handle per solve does without; the second solve takes it."""
+    import torch
+    X, Om, _ = problem(n, d, l)
+    dev.scratch_trim()
+    h = dh.Handle(0)
+    a = solve(h, X, Om, q)
+    assert (h.scratch_bytes() > 0) == first
+    b = solve(h, X, Om, q)
+    assert h.scratch_bytes() > 0
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+    h.close()
 
 
 def test_handles_made_for_every_solve_do_not_wait_for_the_wipe(limit):
