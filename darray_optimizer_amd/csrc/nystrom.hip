@@ -578,8 +578,8 @@ int jacobi_sweeps(dh_handle_t h, int m, int n, double* A, int lda, double* V, in
                 DH_CHECK_HIP(hipEventRecord(h->ev_panel, s));
                 DH_CHECK_HIP(hipStreamWaitEvent(h->aux, h->ev_panel, 0));
             }
-            jacobi_apply_kernel<<<dh_cdiv(n, kJacRows),
-                                  std::min(1024, 64 * dh_cdiv(N / 2 * kJacRows, 64)), 0, beside ? h->aux : s>>>(
+            const int threads = std::min(1024, 64 * dh_cdiv(N / 2 * kJacRows, 64));
+            jacobi_apply_kernel<<<dh_cdiv(n, kJacRows), threads, 0, beside ? h->aux : s>>>(
                 n, N, log + (sweep & 1) * (size_t)(N - 1) * (N / 2), V, ldv,
                 words + 4 + sweep % 4);
             DH_CHECK_LAUNCH();

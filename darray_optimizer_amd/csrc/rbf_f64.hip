@@ -470,11 +470,12 @@ __global__ __launch_bounds__(256) void form_sym_f64_kernel(int n, int d,
     }
 }
 
-// K without labels in the kept layout, for points of any number of features: 64 x 64 distance tiles (tile_mma) with the points of the columns as
-// tile rows, so that the accumulators of lane (g, li) are already its pairs.
-// SYM (Xi = Xj): one triangle of tiles, of which the strict part is stored a
-// second time with every 16 x 16 block transposed through LDS; the products
-// and norms commute, so both halves have the bits of their own tile.
+// K without labels in the kept layout, for points of any number of features: 64
+// x 64 distance tiles (tile_mma) with the points of the columns as tile rows, so
+// that the accumulators of lane (g, li) are already its pairs.  SYM (Xi = Xj): one
+// triangle of tiles, of which the strict part is stored a second time with every
+// 16 x 16 block transposed through LDS; the products and norms commute, so both
+// halves have the bits of their own tile.
 template <bool SYM>
 __global__ __launch_bounds__(256) void form_f64_kernel(int m, int n, int d,
                                                        const double* __restrict__ Xi, int ldxi,
