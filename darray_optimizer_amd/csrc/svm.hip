@@ -105,7 +105,7 @@ __device__ __forceinline__ void ztx_columns(int n, int k, const double* __restri
     static_assert(kColGrp / 4 % NC == 0 && (NC & (NC - 1)) == 0, "columns of a wave");
     for (int u0 = 0; u0 < kColGrp / 4; u0 += NC) {
         const int c0 = blockIdx.y * kColGrp + wave + 4 * u0;  // columns c0 + 4 u
-        if (c0 >= k) break;
+        if (NC < kColGrp / 4 && c0 >= k) break;
         double s[NC], z[NC][4];
 #pragma unroll
         for (int u = 0; u < NC; ++u) {
@@ -400,11 +400,11 @@ __global__ __launch_bounds__(256) void cg_pq_kernel(int nblk, const double* __re
     if (threadIdx.x == 0) *pq = v;
 }
 
-// alpha = r.z / p.q (from *pq, or summed from the waves' partials by every
-// workgroup); s += alpha p, r -= alpha q, z = r / Pc; part2[2b..] = (r.z, r.r).
+// alpha = r.z / p.q (SUMMED: from *part_pq, else summed from the waves' partials by
+// every workgroup); s += alpha p, r -= alpha q, z = r / Pc; part2[2b..] = (r.z, r.r).
+template <bool SUMMED>
 __global__ __launch_bounds__(256) void cg_update_kernel(int n, int nblk,
                                                         const double* __restrict__ part_pq,
-                                                        const double* __restrict__ pq_sum,
                                                         const double* __restrict__ p,
                                                         const double* __restrict__ q,
                                                         const double* __restrict__ Pc,
@@ -417,7 +417,7 @@ __global__ __launch_bounds__(256) void cg_update_kernel(int n, int nblk,
     __shared__ double sh[4];
     const int i = blockIdx.x * kRows + threadIdx.x, ic = min(i, n - 1);
     const double pi = p[ic], qi = q[ic], pc = Pc[ic], si = s[ic], r0 = r[ic];
-    const double pq = pq_sum ? *pq_sum : sum_pq(nblk, part_pq);
+    const double pq = SUMMED ? *part_pq : sum_pq(nblk, part_pq);
     const double alpha = st->rz / pq;
     double rz = 0.0, rr = 0.0;
     if (i < n) {
@@ -708,10 +708,12 @@ int cg_loop(dh_handle_t h, const Work& w, const double* Z, int ldz, double tol, 
                 if (sums) {
                     cg_pq_kernel<<<1, 256, 0, h->stream>>>(w.nblk, w.part, pq, st);
                     DH_CHECK_LAUNCH();
+                    cg_update_kernel<true><<<w.nblk, 256, 0, h->stream>>>(
+                        w.n, w.nblk, pq, p, w.q, w.Pc, w.s, w.r, w.z, w.part2, st);
+                } else {
+                    cg_update_kernel<false><<<w.nblk, 256, 0, h->stream>>>(
+                        w.n, w.nblk, w.part, p, w.q, w.Pc, w.s, w.r, w.z, w.part2, st);
                 }
-                cg_update_kernel<<<w.nblk, 256, 0, h->stream>>>(w.n, w.nblk, w.part,
-                                                                sums ? pq : nullptr, p, w.q, w.Pc,
-                                                                w.s, w.r, w.z, w.part2, st);
                 DH_CHECK_LAUNCH();
             }
             if (sums) {
